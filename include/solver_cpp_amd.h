@@ -421,9 +421,8 @@ int sc_mp_update(int64_t n, double dt, const sc_material* m, const sc_phase_nume
  * a (3,3) field is 9 planes of n doubles (plane q = i+3j holds component
  * (i,j) of every point), a slip field 12 planes of n doubles, dPdF 81 planes
  * (plane i+3j+9k+27l), iterations 2 planes of n ints (Newton, state
- * iterations) and broken n ints.  The substep scratch, the pivoting pass's
- * point list and the terminally-ill flag live in one fixed device array of
- * the library sized for SC_MP_NOALLOC_MAX_POINTS points (about 16 MB, held
+ * iterations) and broken n ints.  The substep scratch lives in one fixed
+ * device array of the library sized for SC_MP_NOALLOC_MAX_POINTS points (about 16 MB, held
  * on each GPU the library runs on until the process ends); larger n is
  * refused with an error.  The call allocates nothing.  Calls that overlap on
  * one GPU share that array and race: serialise them. */

@@ -10,12 +10,11 @@
 //   phenopowerlaw LpAndItsTangent / dotState / kinetics_sl
 //                                        phase_mechanical_plastic_phenopowerlaw.f90:298-483
 // with Fi = I and Li = 0 (no eigen kinematics are active).  The 9x9 Newton
-// Jacobian I - dLp/dS : dS/dFe : dFe/dLp is assembled directly from its
-// rank-12 structure: with G = Fe^T A and K_s = P_s : C (cubic),
-//   J[(a,b),(p,l)] = delta + dt * sum_s c_s P_s(a,b) (G^T K_s)(p,l),
-// c_s = d(gamma_dot_s)/d(tau_s) * sign_s, instead of three 3x3x3x3 products;
-// the sum over s is taken from the slip groups' Hadamard sums
-// (assemble_jacobian8), on the 8 traceless coordinates.
+// Jacobian I - dLp/dS : dS/dFe : dFe/dLp is the identity plus a matrix of rank
+// five (the resolved shears see the five deviatoric numbers of the stress), so
+// its system is solved as a 5x5 one (newton_step).
+#include <cmath>
+
 #include "common.h"
 
 namespace sca {
@@ -45,7 +44,7 @@ __device__ constexpr int HTYPE[NSLIP][NSLIP] = {
 // - the systems 3p, 3p+1, 3p+2 lie on the same plane (normal), p = 0..3;
 // - the systems g, g+3, g+6, g+9 (g = 0, 1, 2) have direction component g
 //   zero.
-// The Jacobian (assemble_jacobian8) needs, for every row r = 3i+j < 8 and
+// The Newton step (newton_step) needs, for every entry r = 3i+j and
 // every symmetric pair (m,l), the sum over s of f_s P_s(i,j) k_s(m,l) with
 // k_s(m,l) = P_s(m,m) (m = l) or P_s(m,l) + P_s(l,m).  Restricted to one
 // direction group its coefficient vector is zero or plus/minus one of the
@@ -68,7 +67,7 @@ constexpr bool slip_structure_holds() {
   for (int s = 0; s < NSLIP; ++s)
     if (SLIP[s][s % 3] != 0) return false;
   const int had[4][4] = {{1, 1, 1, 1}, {1, 1, -1, -1}, {1, -1, 1, -1}, {1, -1, -1, 1}};
-  for (int r = 0; r < 8; ++r)
+  for (int r = 0; r < 9; ++r)
     for (int m = 0; m < 3; ++m)
       for (int l = m; l < 3; ++l) {
         int groups = 0;
@@ -84,7 +83,7 @@ constexpr bool slip_structure_holds() {
       }
   return true;
 }
-static_assert(slip_structure_holds(), "cF slip table: planes of three systems, Hadamard-structured Jacobian sums");
+static_assert(slip_structure_holds(), "cF slip table: planes of three systems, Hadamard-structured sums");
 
 // Material constants travel in the kernel arguments (not a __constant__
 // symbol) so that launches of different contexts on concurrent streams never
@@ -93,9 +92,8 @@ struct KernelArgs {
   MpState s;
   MatConst mc;
   double dt;
-  int* ill;
+  int* ill;     // may be null
   int* broken;  // per point, may be null
-  int* repivot; // [0] count, [1 + i] cells for the pivoting pass
   double* sub;  // substep scratch, SUB_PLANES planes of N doubles
   int64_t c_begin, c_end;  // cells [c_begin, c_end) of the N-cell planes
 };
@@ -302,37 +300,30 @@ __device__ __forceinline__ void slip_sum(const double* g, double v, double* L) {
     }
 }
 
-// kinetics_sl (phenopowerlaw.f90:444-483): tau_pos = t, tau_neg = -t, taking
-// the reciprocal slip resistances rxi = 1/xi (xi is fixed during the Newton
-// iteration, so the divisions are done once per state iteration).
-// dLp/dMp = sum_s c_s P_s (x) P_s with c_s = |gdot_s| n / |tau_s|; for a
-// compile-time exponent this is gdot0 n x^(n-1) / xi, x = |tau_s| / xi, taken
-// from the same powering chain without a division.
-template <int NE4>
-__device__ __forceinline__ void kinetics(const double* S, const double* rxi, double* dg, double* c,
-                                         const MatConst& mc) {
+// kinetics_sl (phenopowerlaw.f90:444-483) with tau_pos = t, tau_neg = -t:
+// gamma_dot_s = sign(tau_s) gdot0 x_s^n, x_s = |tau_s| / xi_s, and its
+// derivative c_s = gdot0 n x_s^(n-1) / xi_s.  Gives pw_s = x_s^n and (DERIV)
+// pm_s = x_s^(n-1) / xi_s; sign, gdot0 and n are left to the caller, which
+// multiplies a sum by them instead of every term.  Takes the reciprocal slip
+// resistances rxi = 1/xi (xi is fixed during the Newton iteration, so the
+// divisions are done once per state iteration).  A compile-time exponent
+// takes both powers from one chain; there is no zero test on it: c_s of a
+// rate below 1e-306 is below 1e-290 and changes no Newton system.
+template <int NE4, bool DERIV>
+__device__ __forceinline__ void slip_powers(const double* tau, const double* rxi, double* pw, double* pm,
+                                            const MatConst& mc) {
   constexpr double TINY10 = 2.2250738585072014e-308 * 10.0;
-  double tau[NSLIP];
-  resolved_shears(S, mc.v, tau);
 #pragma unroll
   for (int s = 0; s < NSLIP; ++s) {
-    const double tp = tau[s];
-    const double tn = -tp;
-    const double sgn = (tp > tn) ? 1.0 : -1.0;
-    const double tmax = fmax(tp, tn);
-    const double x = tmax * rxi[s];
-    if constexpr (NE4 >= 4) {
+    const double t = fabs(tau[s]);
+    const double x = t * rxi[s];
+    if constexpr (NE4 >= 8) {
       const double xm1 = powc<NE4 - 4>(x);
-      const double g = sgn * mc.gdot0 * (xm1 * x);
-      dg[s] = g;
-      if (c) c[s] = (fabs(g) <= TINY10) ? 0.0 : mc.gdot0 * mc.n * xm1 * rxi[s];
+      pw[s] = xm1 * x;
+      if constexpr (DERIV) pm[s] = xm1 * rxi[s];
     } else {
-      const double g = sgn * mc.gdot0 * powe<NE4>(x, mc.n_e4, mc.n);
-      dg[s] = g;
-      if (c) {
-        const double dd = (fabs(g) <= TINY10) ? 0.0 : g * mc.n / tmax;
-        c[s] = dd * ((g > 0.0) ? 1.0 : -1.0);
-      }
+      pw[s] = powe<NE4>(x, mc.n_e4, mc.n);
+      if constexpr (DERIV) pm[s] = (mc.gdot0 * pw[s] <= TINY10) ? 0.0 : pw[s] / t;
     }
   }
 }
@@ -342,11 +333,12 @@ __device__ __forceinline__ void kinetics(const double* S, const double* rxi, dou
 template <int NE4, int AE4>
 __device__ __forceinline__ void dot_state(const double* S, const double* st, const double* rxi, double* dot,
                                           const MatConst& mc) {
-  double dg[NSLIP];
-  kinetics<NE4>(S, rxi, dg, nullptr, mc);
+  double tau[NSLIP], dg[NSLIP];
+  resolved_shears(S, mc.v, tau);
+  slip_powers<NE4, false>(tau, rxi, dg, nullptr, mc);
   const double rxinf = 1.0 / mc.xi_inf;
 #pragma unroll
-  for (int s = 0; s < NSLIP; ++s) dg[s] = fabs(dg[s]);
+  for (int s = 0; s < NSLIP; ++s) dg[s] = mc.gdot0 * dg[s];
 #pragma unroll
   for (int s = 0; s < NSLIP; ++s) {
     const double x = 1.0 - st[s] * rxinf;
@@ -360,28 +352,63 @@ __device__ __forceinline__ void dot_state(const double* S, const double* st, con
   for (int s = 0; s < NSLIP; ++s) dot[NSLIP + s] = dg[s];
 }
 
-// The Newton system J x = b of the Lp iteration lives in the traceless
-// subspace: every P_s is traceless, so J maps traceless matrices to traceless
-// ones, and b = Lp - Lp_constitutive is traceless.  Its solution is therefore
-// traceless and solves the 8x8 system on the coordinates
-//   y_k = x_k (k = 1,2,3,5,6,7, the off-diagonal row-major positions),
-//   y_0 = x_00, y_4 = x_11 (x_22 = -y_0 - y_4),
-// taking the rows 0..7 of J (row 8 = -(row 0 + row 4) on this subspace) and,
-// for the columns 0 and 4, J[:,k] - J[:,8].  The 9x9 solution is recovered
-// exactly; this is the same linear solve with an 8x8 factorisation.
-constexpr int NR = 8;
+// The Newton system of the Lp iteration, J x = b, as a 5x5 system.
+//
+// A change x of Lp (traceless, as b and every P_s are) changes the stress by
+// dS = -dt C : sym(X), X = G x, G = Fe^T A, and the constitutive Lp by
+// sum_s c_s P_s (P_s : dS), so
+//   J x = x + dt sum_s c_s P_s (P_s : C : sym(X)).
+// P_s is traceless and C cubic: P_s : C : sym(X) is a combination of the five
+// numbers w(x) = (X00 - X22, X11 - X22, X01 + X10, X02 + X20, X12 + X21) with
+// the coefficients kD sgn_s(0,0), kD sgn_s(1,1), kA k_s(0,1), kA k_s(0,2),
+// kA k_s(1,2) (kD = v (C11 - C12), kA = v C44, P_s = v sgn_s).  With
+// f_s = dt v c_s and the five matrices U_j = sum_s f_s sgn_s k_s(j) that is
+//   J x = x + sum_j kappa_j U_j w_j(x),
+// and applying w to J x = b leaves the 5x5 system
+//   (1/kappa_i delta_ij + w_i(U_j)) y_j = w_i(b),   x = b - sum_j U_j y_j,
+// y_i = kappa_i w_i(x).
+// The same solution as that of the 9x9 system (up to rounding), from 25
+// instead of 81 (traceless: 64) matrix entries.  G is near the identity, which
+// makes the 5x5 matrix near a symmetric positive definite one times a 2x2
+// block: its LU rarely needs row exchanges.  Every entry of every U_j is plus
+// or minus one of 23 sums of one or two of the Hadamard sums of the direction
+// groups' f_s (qhad), formed once.
+//
+// GENERAL: rows scaled by kappa_i instead of divided by it (any C44 and
+// C11 - C12, zero included); otherwise f_s carries kA and the first two
+// diagonal entries are kA / kD (30 multiplications fewer).
+constexpr int NW = 5;
+__device__ __forceinline__ constexpr int um(int j) { return j == 0 ? 0 : j == 1 ? 1 : j == 2 ? 0 : j == 3 ? 0 : 1; }
+__device__ __forceinline__ constexpr int ul(int j) { return j == 0 ? 0 : j == 1 ? 1 : j == 2 ? 1 : j == 3 ? 2 : 2; }
+// sign of the first term of U_j(r), so that entries equal up to their sign
+// are the same expression
+__device__ __forceinline__ constexpr int usign(int j, int r) {
+  for (int g = 0; g < 3; ++g) {
+    const int code = qhad(g, r, um(j), ul(j));
+    if (code != 0) return code > 0 ? 1 : -1;
+  }
+  return 1;
+}
+// the five numbers w of X = G x (x row-major 3x3)
+__device__ __forceinline__ void newton_w(const double* G, const double* x, double* w) {
+  const double x22 = G[6] * x[2] + G[7] * x[5] + G[8] * x[8];
+  w[0] = G[0] * x[0] + G[1] * x[3] + G[2] * x[6] - x22;
+  w[1] = G[3] * x[1] + G[4] * x[4] + G[5] * x[7] - x22;
+  w[2] = G[0] * x[1] + G[1] * x[4] + G[2] * x[7] + G[3] * x[0] + G[4] * x[3] + G[5] * x[6];
+  w[3] = G[0] * x[2] + G[1] * x[5] + G[2] * x[8] + G[6] * x[0] + G[7] * x[3] + G[8] * x[6];
+  w[4] = G[3] * x[2] + G[4] * x[5] + G[5] * x[8] + G[6] * x[1] + G[7] * x[4] + G[8] * x[7];
+}
 
-// Solve J y = b (8x8, row-major) by LU with partial pivoting (first largest
-// entry of the column, as LAPACK's idamax).  Used only by the pivoting pass
-// (its own kernel), with J in registers.
-__device__ __forceinline__ bool solve8_pivot(double* J, double* b) {
+// Solves M y = b (NW x NW, row-major) by LU with partial pivoting (first
+// largest entry of the column, as LAPACK's idamax); false: singular.
+__device__ __forceinline__ bool solve_pivot(double* M, double* b) {
 #pragma unroll
-  for (int k = 0; k < NR; ++k) {
+  for (int k = 0; k < NW; ++k) {
     int p = k;
-    double mx = fabs(J[NR * k + k]);
+    double mx = fabs(M[NW * k + k]);
 #pragma unroll
-    for (int i = k + 1; i < NR; ++i) {
-      const double v = fabs(J[NR * i + k]);
+    for (int i = k + 1; i < NW; ++i) {
+      const double v = fabs(M[NW * i + k]);
       if (v > mx) {
         mx = v;
         p = i;
@@ -391,35 +418,171 @@ __device__ __forceinline__ bool solve8_pivot(double* J, double* b) {
     // exchange rows k and p by selects over the candidate rows (static
     // register indices; the columns left of k are not read again)
 #pragma unroll
-    for (int i = k + 1; i < NR; ++i) {
+    for (int i = k + 1; i < NW; ++i) {
       const bool sw = p == i;
 #pragma unroll
-      for (int c = k; c < NR; ++c) {
-        const double u = J[NR * k + c], w = J[NR * i + c];
-        J[NR * k + c] = sw ? w : u;
-        J[NR * i + c] = sw ? u : w;
+      for (int c = k; c < NW; ++c) {
+        const double u = M[NW * k + c], w = M[NW * i + c];
+        M[NW * k + c] = sw ? w : u;
+        M[NW * i + c] = sw ? u : w;
       }
       const double u = b[k], w = b[i];
       b[k] = sw ? w : u;
       b[i] = sw ? u : w;
     }
-    const double inv = 1.0 / J[NR * k + k];
+    const double inv = 1.0 / M[NW * k + k];
 #pragma unroll
-    for (int i = k + 1; i < NR; ++i) {
-      const double l = J[NR * i + k] * inv;
+    for (int i = k + 1; i < NW; ++i) {
+      const double l = M[NW * i + k] * inv;
 #pragma unroll
-      for (int c = k + 1; c < NR; ++c) J[NR * i + c] -= l * J[NR * k + c];
+      for (int c = k + 1; c < NW; ++c) M[NW * i + c] -= l * M[NW * k + c];
       b[i] -= l * b[k];
     }
   }
 #pragma unroll
-  for (int i = NR - 1; i >= 0; --i) {
+  for (int i = NW - 1; i >= 0; --i) {
     double s = b[i];
 #pragma unroll
-    for (int c = i + 1; c < NR; ++c) s -= J[NR * i + c] * b[c];
-    b[i] = s / J[NR * i + i];
+    for (int c = i + 1; c < NW; ++c) s -= M[NW * i + c] * b[c];
+    b[i] = s / M[NW * i + i];
   }
   return true;
+}
+
+// Solves M y = b by LU without row exchanges.  Refuses (returns false; b then
+// holds no meaning) when a multiplier exceeds 1e6 in magnitude or a pivot's
+// magnitude is below 2^-1000 (zero and NaN included: the pivot's reciprocal is
+// the refined hardware one, so a pivot near the bottom of the range goes to
+// the pivoted solve and its exact division).  Multipliers up to 1e6 cost at
+// most a few of the 16 digits of a Newton step that needs 6, and the residual
+// test of the next iteration uses the exact residual.  Refusals are collected
+// and tested once at the end (what is computed after one is discarded): no
+// branches inside the unrolled elimination, and the multipliers' magnitudes
+// enter one running maximum (a NaN multiplier is ignored by the maximum).
+__device__ __forceinline__ bool solve_nopivot(double* M, double* b) {
+  bool refused = false;
+  double lmax = 0.0;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+#pragma unroll
+    for (int k = 0; k < i; ++k) {
+      const double l = M[NW * i + k] * M[NW * k + k];
+      lmax = fmax(lmax, fabs(l));
+#pragma unroll
+      for (int c = k + 1; c < NW; ++c) M[NW * i + c] -= l * M[NW * k + c];
+      b[i] -= l * b[k];
+    }
+    const double piv = M[NW * i + i];
+    refused = refused || !(fabs(piv) >= 0x1p-1000);
+    M[NW * i + i] = rcp_refined(piv);
+  }
+#pragma unroll
+  for (int i = NW - 1; i >= 0; --i) {
+    double s = b[i];
+#pragma unroll
+    for (int c = i + 1; c < NW; ++c) s -= M[NW * i + c] * b[c];
+    b[i] = s * M[NW * i + i];
+  }
+  return !(refused || lmax > 1e6);
+}
+
+// The Newton step x of J x = b, in place of b (row-major 3x3, traceless);
+// pm: slip_powers' derivatives.  false: refused (without PIVOT) or singular.
+template <bool GENERAL, bool PIVOT>
+__device__ __forceinline__ bool newton_step(const double* Fe, const double* A, const double* pm, double dt,
+                                            double* b, const MatConst& mc) {
+  double G[9];
+#pragma unroll
+  for (int m = 0; m < 3; ++m)
+#pragma unroll
+    for (int p = 0; p < 3; ++p) G[3 * m + p] = Fe[m] * A[p] + Fe[3 + m] * A[3 + p] + Fe[6 + m] * A[6 + p];
+  // Hadamard sums of f_s over each direction group
+  const double f = dt * (GENERAL ? mc.newton_f : mc.newton_fA);
+  double H[3][4];
+#pragma unroll
+  for (int g = 0; g < 3; ++g) {
+    const double a = pm[g] * f, bb = pm[g + 3] * f, x = pm[g + 6] * f, y = pm[g + 9] * f;
+    const double ab = a + bb, amb = a - bb, xy = x + y, xmy = x - y;
+    H[g][0] = ab + xy;
+    H[g][1] = ab - xy;
+    H[g][2] = amb + xmy;
+    H[g][3] = amb - xmy;
+  }
+  double U[NW][9];
+#pragma unroll
+  for (int j = 0; j < NW; ++j)
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+      double t = 0.0;
+      bool first = true;
+#pragma unroll
+      for (int g = 0; g < 3; ++g) {
+        const int code = qhad(g, r, um(j), ul(j)) * usign(j, r);
+        if (code != 0) {
+          const double h = H[g][(code > 0 ? code : -code) - 1];
+          t = first ? h : (code > 0 ? t + h : t - h);
+          first = false;
+        }
+      }
+      U[j][r] = usign(j, r) > 0 ? t : -t;
+    }
+  b[8] = -(b[0] + b[4]);
+  double M[NW * NW], y[NW];
+  newton_w(G, b, y);
+#pragma unroll
+  for (int j = 0; j < NW; ++j) {
+    double w[NW];
+    newton_w(G, U[j], w);
+#pragma unroll
+    for (int i = 0; i < NW; ++i) M[NW * i + j] = w[i];
+  }
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    if constexpr (GENERAL) {
+      const double k = mc.v * (i < 2 ? mc.C11 - mc.C12 : mc.C44);
+      y[i] *= k;
+#pragma unroll
+      for (int j = 0; j < NW; ++j) M[NW * i + j] *= k;
+      M[NW * i + i] += 1.0;
+    } else {
+      M[NW * i + i] += i < 2 ? mc.newton_d : 1.0;
+    }
+  }
+  const bool ok = PIVOT ? solve_pivot(M, y) : solve_nopivot(M, y);
+#pragma unroll
+  for (int r = 0; r < 8; ++r)
+#pragma unroll
+    for (int j = 0; j < NW; ++j) b[r] -= U[j][r] * y[j];
+  b[8] = -(b[0] + b[4]);
+  // Where the rates are stiff (an overshot iterate), b and sum U y agree in
+  // many digits and x keeps a rounding error of the size of b's, which J
+  // multiplies.  J acts on the five numbers w(x) only, and those are known
+  // without cancellation: y_i / kappa_i.  The symmetric traceless matrix that
+  // has the difference for its five numbers (G taken as the identity) removes
+  // it to within |G - I|.  Without it 871 instead of 162 of the 4096 points of
+  // 2 % strain steps take other iteration counts than with a pivoted 9x9 LU.
+  double e[NW];
+  newton_w(G, b, e);
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    if constexpr (GENERAL) {
+      const double k = mc.v * (i < 2 ? mc.C11 - mc.C12 : mc.C44);
+      e[i] = k != 0.0 ? y[i] / k - e[i] : 0.0;
+    } else {
+      e[i] = i < 2 ? mc.newton_d * y[i] - e[i] : y[i] - e[i];
+    }
+  }
+  const double tr = (e[0] + e[1]) * (-1.0 / 3.0);
+  b[0] += e[0] + tr;
+  b[4] += e[1] + tr;
+  b[1] += 0.5 * e[2];
+  b[3] += 0.5 * e[2];
+  b[2] += 0.5 * e[3];
+  b[6] += 0.5 * e[3];
+  b[5] += 0.5 * e[4];
+  b[7] += 0.5 * e[4];
+  b[8] = -(b[0] + b[4]);
+  return ok;
 }
 
 // Column-major plane q = i+3j of a (3,3) field <-> row-major register 3*i+j
@@ -456,13 +619,24 @@ __device__ __forceinline__ double ld(const double* plane, Lane l) {
 __device__ __forceinline__ void st(double* plane, Lane l, double v) {
   *reinterpret_cast<gdouble*>(uniform_u64(reinterpret_cast<uint64_t>(plane)) + l.off) = v;
 }
+// The plane stride as a value of this place only: pointers formed from it are
+// formed here (two scalar adds a plane).  From the plain N the compiler forms
+// the pointers of every access once at the kernel's entry, keeps them in
+// vector lanes (it has no scalar registers for 150 of them) and reads each
+// back at its use: 630 instructions of the 12000 that a wave executes.
+__device__ __forceinline__ int64_t stride_here(int64_t N) {
+  asm volatile("" : "+s"(N));
+  return N;
+}
 __device__ __forceinline__ void load33(const double* base, int64_t N, Lane l, double* m) {
+  const int64_t n = stride_here(N);
 #pragma unroll
-  for (int q = 0; q < 9; ++q) m[rm(q)] = ld(base + q * N, l);
+  for (int q = 0; q < 9; ++q) m[rm(q)] = ld(base + q * n, l);
 }
 __device__ __forceinline__ void store33(double* base, int64_t N, Lane l, const double* m) {
+  const int64_t n = stride_here(N);
 #pragma unroll
-  for (int q = 0; q < 9; ++q) st(base + q * N, l, m[rm(q)]);
+  for (int q = 0; q < 9; ++q) st(base + q * n, l, m[rm(q)]);
 }
 // load from a plane chosen per lane (the base may differ between lanes): a
 // 64-bit lane address and one unconditional load, so that the loads of all
@@ -474,167 +648,9 @@ __device__ __forceinline__ double ldv(const double* plane, Lane l) {
 __device__ __forceinline__ void load33_sel(bool sel, const double* a, const double* b, int64_t N, Lane l,
                                            double* m) {
   const double* base = sel ? a : b;
+  const int64_t n = stride_here(N);
 #pragma unroll
-  for (int q = 0; q < 9; ++q) m[rm(q)] = ldv(base + q * N, l);
-}
-
-// J = I + dt sum_s c_s vec(P_s) vec(G^T K_s)^T with G = Fe^T A, restricted to
-// the traceless coordinates (rows 0..7; columns 0 and 4 minus column 8), as
-// an 8x8 row-major matrix.
-//
-// K_s = P_s : C for the cubic stiffness (tr P_s = 0) is K_s(m,l) =
-// kappa(m,l) k_s(m,l) with kappa = 2 kA + kB on the diagonal and kA off it,
-// kA = v C44, kB = v (C11 - C12 - 2 C44).  With f_s = dt v c_s, row r = 3i+j is
-//   J(r,(p,l)) = delta + sum_m kappa(m,l) G(m,p) Q_r(m,l),
-//   Q_r(m,l) = sum_s f_s P_s(i,j) k_s(m,l)   (symmetric in m,l),
-// and every Q_r(m,l) is a signed sum of one or two of the twelve Hadamard sums
-// of the direction groups' f_s (qhad): 24 additions for all the Q_r instead of
-// a rank-one update of the 8x8 matrix per slip system.
-
-// Row-independent part of the Jacobian: kappa G (or, LEAN, G alone, kappa
-// then scaling Q in every row: 18 registers fewer for 48 more products) and
-// the Hadamard sums
-template <bool LEAN>
-struct JacobianParts {
-  double Gd[9], Go[LEAN ? 1 : 9];  // kappa G for the diagonal / off-diagonal (m,l); LEAN: G in Gd
-  double H[3][4];                  // Hadamard sums of f_s over each direction group
-};
-template <bool LEAN>
-__device__ __forceinline__ void jacobian_parts(const double* Fe, const double* A, const double* c, double dt,
-                                               JacobianParts<LEAN>& jp, const MatConst& mc) {
-  const double kA = mc.v * mc.C44, kB = mc.v * (mc.C11 - mc.C12 - 2.0 * mc.C44);
-  const double kD = 2.0 * kA + kB;
-#pragma unroll
-  for (int m = 0; m < 3; ++m)
-#pragma unroll
-    for (int p = 0; p < 3; ++p) {
-      const double g = Fe[m] * A[p] + Fe[3 + m] * A[3 + p] + Fe[6 + m] * A[6 + p];
-      if constexpr (LEAN) {
-        jp.Gd[3 * m + p] = g;
-      } else {
-        jp.Gd[3 * m + p] = g * kD;
-        jp.Go[3 * m + p] = g * kA;
-      }
-    }
-  const double fv = dt * mc.v;
-#pragma unroll
-  for (int g = 0; g < 3; ++g) {
-    const double a = c[g] * fv, b = c[g + 3] * fv, x = c[g + 6] * fv, y = c[g + 9] * fv;
-    const double ab = a + b, amb = a - b, xy = x + y, xmy = x - y;
-    jp.H[g][0] = ab + xy;
-    jp.H[g][1] = ab - xy;
-    jp.H[g][2] = amb + xmy;
-    jp.H[g][3] = amb - xmy;
-  }
-}
-// row r of the 8x8 Jacobian
-template <bool LEAN>
-__device__ __forceinline__ void jacobian_row(const JacobianParts<LEAN>& jp, int r, double* row, const MatConst& mc) {
-  double Q[3][3];
-#pragma unroll
-  for (int m = 0; m < 3; ++m)
-#pragma unroll
-    for (int l = m; l < 3; ++l) {
-      double t = 0.0;
-      bool first = true;
-#pragma unroll
-      for (int g = 0; g < 3; ++g) {
-        const int code = qhad(g, r, m, l);
-        if (code != 0) {
-          const double h = jp.H[g][(code > 0 ? code : -code) - 1];
-          t = first ? (code > 0 ? h : -h) : (code > 0 ? t + h : t - h);
-          first = false;
-        }
-      }
-      if constexpr (LEAN) {
-        const double kA = mc.v * mc.C44, kB = mc.v * (mc.C11 - mc.C12 - 2.0 * mc.C44);
-        t = t * (m == l ? 2.0 * kA + kB : kA);
-      }
-      Q[m][l] = t;
-      Q[l][m] = t;
-    }
-  double Y[9];
-#pragma unroll
-  for (int p = 0; p < 3; ++p)
-#pragma unroll
-    for (int l = 0; l < 3; ++l) {
-      if constexpr (LEAN) {
-        double y = jp.Gd[p] * Q[0][l];
-        y += jp.Gd[3 + p] * Q[1][l];
-        y += jp.Gd[6 + p] * Q[2][l];
-        Y[3 * p + l] = y;
-      } else {
-        double y = (l == 0 ? jp.Gd : jp.Go)[p] * Q[0][l];
-        y += (l == 1 ? jp.Gd : jp.Go)[3 + p] * Q[1][l];
-        y += (l == 2 ? jp.Gd : jp.Go)[6 + p] * Q[2][l];
-        Y[3 * p + l] = y;
-      }
-    }
-#pragma unroll
-  for (int q = 0; q < NR; ++q) {
-    const double y = (q == 0 || q == 4) ? Y[q] - Y[8] : Y[q];
-    row[q] = (q == r) ? 1.0 + y : y;
-  }
-}
-__device__ __forceinline__ void assemble_jacobian8(const double* Fe, const double* A, const double* c, double dt,
-                                                   double* J, const MatConst& mc) {
-  JacobianParts<true> jp;
-  jacobian_parts(Fe, A, c, dt, jp, mc);
-#pragma unroll
-  for (int r = 0; r < NR; ++r) jacobian_row(jp, r, J + NR * r, mc);
-}
-
-// The Newton system assembled and solved by LU without row exchanges, one row
-// at a time: row i is eliminated by the factor rows 0..i-1 as soon as it is
-// formed (the same operations on every entry, in the same order, as the
-// column-by-column elimination), so only the factor rows are held.  Refuses
-// (returns false; b then holds no meaning) when a multiplier exceeds 1e6 in
-// magnitude or a pivot's magnitude is below 2^-1000 (zero and NaN included:
-// the pivot's reciprocal is the refined hardware one, so a pivot near the
-// bottom of the range goes to the pivoted pass and its exact division; the
-// pivots of this system, 1 plus rate terms, are never near the top of the
-// range): multipliers up to 1e6 cost at most a few of
-// the 16 digits of the Newton step, far below the Newton tolerance, and the
-// residual test of the next iteration uses the exact residual; only steeper
-// cases (about 1 % of points had pivots below 1/100 of their column in the
-// 128^3 tension case) need the pivoted pass.
-__device__ __forceinline__ bool assemble_solve8_nopivot(const double* Fe, const double* A, const double* c,
-                                                        double dt, double* b, const MatConst& mc) {
-  JacobianParts<false> jp;
-  jacobian_parts(Fe, A, c, dt, jp, mc);
-  double U[NR * NR];  // factor rows (upper part), reciprocal pivots on the diagonal
-  // refusals are collected and tested once at the end (what is computed
-  // after one is discarded): no branches inside the unrolled elimination, and
-  // the multipliers' magnitudes enter one running maximum (a NaN multiplier
-  // is ignored by the maximum, as by the comparison it replaces)
-  bool refused = false;
-  double lmax = 0.0;
-#pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    double row[NR];
-    jacobian_row(jp, i, row, mc);
-#pragma unroll
-    for (int k = 0; k < i; ++k) {
-      const double l = row[k] * U[NR * k + k];
-      lmax = fmax(lmax, fabs(l));
-#pragma unroll
-      for (int c2 = k + 1; c2 < NR; ++c2) row[c2] -= l * U[NR * k + c2];
-      b[i] -= l * b[k];
-    }
-    const double piv = row[i];
-    refused = refused || !(fabs(piv) >= 0x1p-1000);
-    U[NR * i + i] = rcp_refined(piv);
-#pragma unroll
-    for (int c2 = i + 1; c2 < NR; ++c2) U[NR * i + c2] = row[c2];
-  }
-#pragma unroll
-  for (int i = NR - 1; i >= 0; --i) {
-    double s = b[i];
-#pragma unroll
-    for (int c2 = i + 1; c2 < NR; ++c2) s -= U[NR * i + c2] * b[c2];
-    b[i] = s * U[NR * i + i];
-  }
-  return !(refused || lmax > 1e6);
+  for (int q = 0; q < 9; ++q) m[rm(q)] = ldv(base + q * n, l);
 }
 
 // Per-point output / scratch addressing
@@ -644,21 +660,42 @@ struct PointIO {
   Lane l;
 };
 
-// integrateStress (phase_mechanical.f90:380-604); returns 0 (integrated),
-// 1 (broken) or, without PIVOT, 2 when the LU without row exchanges refused a
-// pivot (the point is then redone by the PIVOT instantiation, which solves
-// every Newton system with partial pivoting).  Takes the reciprocal slip
-// resistances of the state and updates S and Lp in registers; Fe, P and Fp
-// of the integration the state loop keeps are formed and stored by
-// store_integrated.
+// Elastic deformation and constitutive velocity gradient at Lp: Fe = A (I -
+// dt Lp), pm (slip_powers) and Lpc = v gdot0 sum_s sign_s x_s^n d_s n_s^T
+template <int NE4>
+__device__ __forceinline__ void lp_constitutive(const double* A, double dt, const double* Lp, const double* rxi,
+                                                double* Fe, double* pm, double* Lpc, const MatConst& mc) {
+  double B[9], Sl[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) B[k] = (k % 4 == 0 ? 1.0 : 0.0) - dt * Lp[k];
+  mm33(A, B, Fe);  // Fe = A B invFi_new, invFi_new = I
+  hooke_S(Fe, Sl, mc);
+  double tau[NSLIP], g[NSLIP];
+  resolved_shears(Sl, mc.v, tau);
+  slip_powers<NE4, true>(tau, rxi, g, pm, mc);
+#pragma unroll
+  for (int s = 0; s < NSLIP; ++s) g[s] = copysign(g[s], tau[s]);
+  slip_sum(g, mc.newton_vg, Lpc);
+}
+
+// integrateStress (phase_mechanical.f90:380-604); returns 0 (integrated) or
+// 1 (broken).  Takes the reciprocal slip resistances of the state and updates
+// S and Lp in registers; Fe, P and Fp of the integration the state loop keeps
+// are formed and stored by store_integrated.
 //
 // A = F invFp0 of the (sub)step and invFp0 (both in LDS, lane t) are formed
 // once per substep by the caller: they do not change during the state fixed
 // point.
-template <int NE4, bool PIVOT>
+//
+// A Newton system whose LU without row exchanges is refused (a steep or
+// singular one) is formed again and solved with partial pivoting, as LAPACK's
+// dgesv in the reference: a branch that a wave takes only when one of its
+// lanes does.
+template <int NE4>
 __device__ __forceinline__ int integrate_stress(const double (*hA)[64], const double (*invFp0)[64], int t, double dt,
                                                 const double* rxi, double* Lp, double* S, int& newton,
                                                 const MatConst& mc) {
+  constexpr bool GENERAL = NE4 < 0;
   // A is read from LDS where it is used, not hoisted into the registers the
   // Newton system needs: the lane index passes through an empty asm, so every
   // call's nine ds_reads are new loads (issued together, one wait), not the
@@ -684,19 +721,9 @@ __device__ __forceinline__ int integrate_stress(const double (*hA)[64], const do
   for (;;) {
     it++;
     if (it > mc.N_iter_Lp_max) return 1;
-    double Fe[9], Sl[9];
-    {
-      double B[9], A[9];
-#pragma unroll
-      for (int k = 0; k < 9; ++k) B[k] = (k % 4 == 0 ? 1.0 : 0.0) - dt * Lp[k];
-      loadA(A);
-      mm33(A, B, Fe);  // Fe = A B invFi_new, invFi_new = I
-    }
-    hooke_S(Fe, Sl, mc);
-    double dg[NSLIP], c[NSLIP];
-    kinetics<NE4>(Sl, rxi, dg, c, mc);
-    double res[9];
-    slip_sum(dg, mc.v, res);
+    double A[9], Fe[9], pm[NSLIP], res[9];
+    loadA(A);
+    lp_constitutive<NE4>(A, dt, Lp, rxi, Fe, pm, res, mc);
     // res holds Lp_constitutive here
     double n2Lpc = 0.0, n2Lp = 0.0, n2res = 0.0;
 #pragma unroll
@@ -725,18 +752,15 @@ __device__ __forceinline__ int integrate_stress(const double (*hA)[64], const do
         continue;
       }
     }
-    {
-      double J[NR * NR], A[9];
+    if (!newton_step<GENERAL, false>(Fe, A, pm, dt, res, mc)) {
+      // formed again from Lp (the same values: the same operations), so that
+      // nothing is held for this rare branch
       loadA(A);
-      if constexpr (PIVOT) {
-        assemble_jacobian8(Fe, A, c, dt, J, mc);
-        if (!solve8_pivot(J, res)) return 1;  // singular
-      } else {
-        // the point is redone by the pivoting pass
-        if (!assemble_solve8_nopivot(Fe, A, c, dt, res, mc)) return 2;
-      }
+      lp_constitutive<NE4>(A, dt, Lp, rxi, Fe, pm, res, mc);
+#pragma unroll
+      for (int k = 0; k < 9; ++k) res[k] = Lp[k] - res[k];
+      if (!newton_step<GENERAL, true>(Fe, A, pm, dt, res, mc)) return 1;  // singular
     }
-    res[8] = -(res[0] + res[4]);  // x_22 of the traceless solution
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
       dLp[k] = -res[k];
@@ -810,19 +834,6 @@ __device__ __forceinline__ void store_integrated(const double (*hA)[64], const d
 // being integrated (9).  Touched only when the first full step was cut back.
 constexpr int SUB_F0 = 0, SUB_LP0 = 9, SUB_FP0 = 18, SUB_ST0 = 27, SUB_FLOC = 51, SUB_PLANES = 60;
 
-// One residual evaluation's material-point loop, in two passes.  The first
-// (mp_response_kernel) carries no pivoted factorisation, so that its
-// registers serve the common path only; a point whose Newton system the LU
-// without row exchanges refuses leaves its loops, stores no output and is
-// appended to the repivot list (its inputs are unchanged: Lp, the only plane
-// that is both read and written, is stored last).  The second
-// (mp_repivot_kernel) redoes exactly the listed points from the same inputs,
-// every Newton system of them solved with partial pivoting (as LAPACK's
-// dgesv in the reference), in a grid-stride loop over the list.  Points are
-// independent, so the list order does not change any result.
-//
-// repivot: [0] = number of listed points, [1 + i] = cell index.
-
 // per-lane LDS columns of one 64-lane block: FPI history
 // (dotState_last(:,1), its difference to dotState_last(:,2)) and the
 // accumulated-shear half of the state stay in LDS while the Lp Newton
@@ -835,7 +846,7 @@ struct MpLds {
   double A[9][64];     // F_(sub)step invFp0
 };
 
-template <int NE4, int AE4, bool PIVOT>
+template <int NE4, int AE4>
 __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, MpLds& sh) {
   const MatConst& mc = a.mc;
   const MpState& s = a.s;
@@ -857,9 +868,9 @@ __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, M
   // substep scratch planes
   bool in_sub = false;
   int newton = 0, fpi = 0;
-  auto st0 = [&](int k) -> double {
-    if (k < NSLIP) return ldv((in_sub ? sub + SUB_ST0 * N : s.xi0) + k * N, l);
-    return ldv((in_sub ? sub + (SUB_ST0 + NSLIP) * N : s.gamma0) + (k - NSLIP) * N, l);
+  auto st0 = [&](int k, int64_t n) -> double {
+    if (k < NSLIP) return ldv((in_sub ? sub + SUB_ST0 * n : s.xi0) + k * n, l);
+    return ldv((in_sub ? sub + (SUB_ST0 + NSLIP) * n : s.gamma0) + (k - NSLIP) * n, l);
   };
 
   // F and F0 of the increment (not written here), loaded once with Lp
@@ -885,7 +896,6 @@ __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, M
   };
   double stepFrac = 0.0, step = 1.0 / mc.r_cutback;
   bool converged = false, todo = true;
-  bool refused = false;  // first pass only: the Newton system needs row exchanges
   double fp0v[9];        // Fp0 of the (sub)step about to be integrated (planes in order)
   // step control: the next substep after a converged one, else a cut-back
   // step from the restored start values; sets todo
@@ -898,23 +908,24 @@ __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, M
         // all loads before the stores: the compiler cannot tell the planes
         // apart, and a load after a store would wait for the one before it
         double fl[9], fp[9];
+        const int64_t n = stride_here(N);
 #pragma unroll
         for (int k = 0; k < 9; ++k) {
-          fl[k] = ld(sub + (SUB_FLOC + k) * N, l);
-          fp[k] = ld(s.Fp + (k) * N, l);
+          fl[k] = ld(sub + (SUB_FLOC + k) * n, l);
+          fp[k] = ld(s.Fp + (k) * n, l);
         }
         __builtin_amdgcn_sched_barrier(0);  // all issued before the first store (one round trip)
 #pragma unroll
         for (int k = 0; k < 9; ++k) {
-          st(sub + (SUB_F0 + k) * N, l, fl[k]);
-          st(sub + (SUB_LP0 + k) * N, l, Lp[rm(k)]);
-          st(sub + (SUB_FP0 + k) * N, l, fp[k]);
+          st(sub + (SUB_F0 + k) * n, l, fl[k]);
+          st(sub + (SUB_LP0 + k) * n, l, Lp[rm(k)]);
+          st(sub + (SUB_FP0 + k) * n, l, fp[k]);
           fp0v[k] = fp[k];
         }
 #pragma unroll
         for (int k = 0; k < NSLIP; ++k) {
-          st(sub + (SUB_ST0 + k) * N, l, xi[k]);
-          st(sub + (SUB_ST0 + NSLIP + k) * N, l, h_gam[k][t]);
+          st(sub + (SUB_ST0 + k) * n, l, xi[k]);
+          st(sub + (SUB_ST0 + NSLIP + k) * n, l, h_gam[k][t]);
         }
         in_sub = true;
       }
@@ -925,12 +936,13 @@ __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, M
       // itself, the scheduler interleaves them with the LDS stores of the
       // shear column through a few staging registers, a round trip per pair.
       double stl[NSTATE];
-      load33(s.S0, N, l, S);
+      const int64_t n = stride_here(N);
+      load33(s.S0, n, l, S);
 #pragma unroll
-      for (int k = 0; k < 9; ++k) fp0v[k] = ldv((in_sub ? sub + SUB_FP0 * N : s.Fp0) + k * N, l);
-      if (step < 1.0) load33_sel(in_sub, sub + SUB_LP0 * N, s.Lp0, N, l, Lp);
+      for (int k = 0; k < 9; ++k) fp0v[k] = ldv((in_sub ? sub + SUB_FP0 * n : s.Fp0) + k * n, l);
+      if (step < 1.0) load33_sel(in_sub, sub + SUB_LP0 * n, s.Lp0, n, l, Lp);
 #pragma unroll
-      for (int k = 0; k < NSTATE; ++k) stl[k] = st0(k);
+      for (int k = 0; k < NSTATE; ++k) stl[k] = st0(k, n);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int k = 0; k < NSLIP; ++k) {
@@ -938,18 +950,14 @@ __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, M
         h_gam[k][t] = stl[NSLIP + k];
       }
 #pragma unroll
-      for (int k = 0; k < 9; ++k) st(s.Fp + (k) * N, l, fp0v[k]);  // after the loads, as above
+      for (int k = 0; k < 9; ++k) st(s.Fp + (k) * n, l, fp0v[k]);  // after the loads, as above
       todo = step > mc.r_cutback_min;
     }
   };
-  // first pass: the first call restores the increment's start values; it
-  // follows the entry loads directly, so that its loads and theirs share one
-  // round trip.  The pivoting pass (a few points per launch, registers
-  // tighter) keeps the control at the top of the loop.
-  if constexpr (!PIVOT) control();
-  for (;;) {
-    if constexpr (PIVOT) control();
-    if (!todo) break;
+  // the first call restores the increment's start values; it follows the
+  // entry loads directly, so that its loads and theirs share one round trip
+  control();
+  while (todo) {
     {
       // A = F_(sub)step invFp0 and invFp0 are fixed during the state fixed
       // point (integrateStress, phase_mechanical.f90:425-432)
@@ -1012,10 +1020,7 @@ __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, M
           }
 #pragma unroll
           for (int k = 0; k < NSLIP; ++k) rxi[k] = rcp_refined(xi[k]);
-          const int rc =
-              fp0_singular ? 1 : integrate_stress<NE4, PIVOT>(sh.A, sh.iFp0, t, sdt, rxi, Lp, S, newton, mc);
-          refused = rc == 2;
-          broken = rc != 0;
+          broken = fp0_singular || integrate_stress<NE4>(sh.A, sh.iFp0, t, sdt, rxi, Lp, S, newton, mc) != 0;
           if (broken) break;
           {
             double stt[NSTATE];
@@ -1081,33 +1086,26 @@ __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, M
         }
       }
       converged = !broken;
-      if (refused) break;  // the pivoting pass redoes this point from its inputs
     }
-    if constexpr (!PIVOT) control();
-  }
-  if constexpr (!PIVOT) {
-    if (refused) {
-      const int slot = atomicAdd(a.repivot, 1);
-      a.repivot[1 + slot] = (int)c;
-      return;
-    }
+    control();
   }
   store33(s.Lp, N, l, Lp);
   store33(s.S, N, l, S);
   double gv[NSLIP];  // the shear column, read from LDS in one batch
 #pragma unroll
   for (int k = 0; k < NSLIP; ++k) gv[k] = h_gam[k][t];
+  const int64_t n = stride_here(N);
 #pragma unroll
   for (int k = 0; k < NSLIP; ++k) {
-    st(s.xi + (k) * N, l, xi[k]);
-    st(s.gamma + (k) * N, l, gv[k]);
+    st(s.xi + (k) * n, l, xi[k]);
+    st(s.gamma + (k) * n, l, gv[k]);
   }
   if (s.iters) {
     s.iters[c] = newton;
     s.iters[N + c] = fpi;
   }
   if (a.broken) a.broken[c] = converged ? 0 : 1;
-  if (!converged) atomicOr(a.ill, 1);
+  if (!converged && a.ill) atomicOr(a.ill, 1);
 }
 
 template <int NE4, int AE4>
@@ -1115,22 +1113,11 @@ __global__ void __launch_bounds__(64) mp_response_kernel(KernelArgs a) {
   __shared__ MpLds sh;
   const int64_t c = a.c_begin + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= a.c_end) return;
-  mp_point<NE4, AE4, false>(a, c, sh);
+  mp_point<NE4, AE4>(a, c, sh);
 }
 
-template <int NE4, int AE4>
-__global__ void __launch_bounds__(64) mp_repivot_kernel(KernelArgs a) {
-  __shared__ MpLds sh;
-  const int64_t cnt = a.repivot[0];  // complete: the first pass ran before this launch
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += (int64_t)gridDim.x * blockDim.x)
-    mp_point<NE4, AE4, true>(a, a.repivot[1 + i], sh);
-}
-
-// clears the repivot list and the terminally-ill flag of one response
-__global__ void repivot_reset_kernel(int* repivot, int* ill) {
-  repivot[0] = 0;
-  *ill = 0;
-}
+// clears the terminally-ill flag of one response
+__global__ void ill_reset_kernel(int* ill) { *ill = 0; }
 
 // ---- many RVEs in one launch ---------------------------------------------------
 // The material-point updates of a batch of RVEs (each with its own planes,
@@ -1170,25 +1157,12 @@ __global__ void __launch_bounds__(64) mp_response_batch_kernel(const KernelArgs*
   const KernelArgs a = load_args(tab + r);
   const int64_t c = a.c_begin + (int64_t)(blockIdx.x - (unsigned)blk_off[r]) * 64 + threadIdx.x;
   if (c >= a.c_end) return;
-  mp_point<NE4, AE4, false>(a, c, sh);
+  mp_point<NE4, AE4>(a, c, sh);
 }
 
-// pivoting pass of a batch: blockIdx.y is the RVE, blockIdx.x strides over
-// its list as mp_repivot_kernel does
-template <int NE4, int AE4>
-__global__ void __launch_bounds__(64) mp_repivot_batch_kernel(const KernelArgs* __restrict__ tab) {
-  __shared__ MpLds sh;
-  const KernelArgs a = load_args(tab + blockIdx.y);
-  const int64_t cnt = a.repivot[0];
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += (int64_t)gridDim.x * blockDim.x)
-    mp_point<NE4, AE4, true>(a, a.repivot[1 + i], sh);
-}
-
-__global__ void repivot_reset_batch_kernel(const KernelArgs* __restrict__ tab, int n) {
+__global__ void ill_reset_batch_kernel(const KernelArgs* __restrict__ tab, int n) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  tab[r].repivot[0] = 0;
-  *tab[r].ill = 0;
+  if (r < n) *tab[r].ill = 0;
 }
 
 
@@ -1345,10 +1319,13 @@ __global__ void __launch_bounds__(64) mp_tangent_kernel(TangentArgs a) {
 #pragma unroll
     for (int k = 0; k < 9; ++k) invFp0[k] = 0.0;
   }
-  double dg[NSLIP], cs[NSLIP], rxi[NSLIP];
+  double tau[NSLIP], dg[NSLIP], cs[NSLIP], rxi[NSLIP];
 #pragma unroll
   for (int k = 0; k < NSLIP; ++k) rxi[k] = 1.0 / xi[k];
-  kinetics<NE4>(S, rxi, dg, cs, mc);
+  resolved_shears(S, mc.v, tau);
+  slip_powers<NE4, true>(tau, rxi, dg, cs, mc);
+#pragma unroll
+  for (int k = 0; k < NSLIP; ++k) cs[k] = mc.gdot0 * mc.n * cs[k];
 
   // L = I + dt sum_s c_s vec(U_s) vec(P_s)^T, U_s = C : (H P_s), H = Fe^T F invFp0
   double T2[9], H[9];
@@ -1621,6 +1598,13 @@ __global__ void mp_init_kernel(MpState s, const double* Fp_init, double xi_0) {
 int mp_partial_blocks(int64_t N) { return (int)((N + PAV_CELLS - 1) / PAV_CELLS); }
 int mp_sub_planes() { return SUB_PLANES; }
 
+// The exponents of the example material (n_sl = 20, a_sl = 2.25) are compiled
+// in, with the Newton system divided by its stiffness scales, which must not
+// vanish; any other material runs the runtime-exponent instantiation.
+static bool example_class(const MatConst& mc) {
+  return mc.n_e4 == 80 && mc.a_e4 == 9 && std::isfinite(mc.newton_d) && mc.newton_d != 0.0;
+}
+
 void launch_mp_response(const MpState& s, const MatConst& mc, double dt, int* d_ill, double* d_sub, hipStream_t st,
                         int* d_broken, int64_t c_begin, int64_t c_end) {
   if (c_end < 0) c_end = s.N;
@@ -1628,22 +1612,11 @@ void launch_mp_response(const MpState& s, const MatConst& mc, double dt, int* d_
   if (c_begin == c_end) return;
   // lanes address planes by a 32-bit byte offset (cell index * 8)
   if (s.N > ((int64_t)1 << 29)) throw std::runtime_error("material-point planes longer than 2^29 cells");
-  if (!s.repivot) throw std::runtime_error("material-point state without the repivot plane");
-  KernelArgs a{s, mc, dt, d_ill, d_broken, s.repivot, d_sub, c_begin, c_end};
+  KernelArgs a{s, mc, dt, d_ill, d_broken, d_sub, c_begin, c_end};
   const int blocks = (int)((c_end - c_begin + 63) / 64);
-  // exponents of the example material (n_sl = 20, a_sl = 2.25) are compiled
-  // in; any other material runs the runtime-exponent instantiation
-  // second pass: a fixed grid striding over the list (it holds at most the
-  // range's points)
-  const int blocks2 = std::min(blocks, 1024);
-  hipLaunchKernelGGL(repivot_reset_kernel, dim3(1), dim3(1), 0, st, s.repivot, d_ill);
-  if (mc.n_e4 == 80 && mc.a_e4 == 9) {
-    hipLaunchKernelGGL((mp_response_kernel<80, 9>), dim3(blocks), dim3(64), 0, st, a);
-    hipLaunchKernelGGL((mp_repivot_kernel<80, 9>), dim3(blocks2), dim3(64), 0, st, a);
-  } else {
-    hipLaunchKernelGGL((mp_response_kernel<-1, -1>), dim3(blocks), dim3(64), 0, st, a);
-    hipLaunchKernelGGL((mp_repivot_kernel<-1, -1>), dim3(blocks2), dim3(64), 0, st, a);
-  }
+  if (d_ill) hipLaunchKernelGGL(ill_reset_kernel, dim3(1), dim3(1), 0, st, d_ill);
+  if (example_class(mc)) hipLaunchKernelGGL((mp_response_kernel<80, 9>), dim3(blocks), dim3(64), 0, st, a);
+  else hipLaunchKernelGGL((mp_response_kernel<-1, -1>), dim3(blocks), dim3(64), 0, st, a);
   SCA_HIP(hipGetLastError());
 }
 
@@ -1659,21 +1632,19 @@ void launch_mp_response_batch(const MpBatchItem* items, int n, TableArena& ta, h
   int* off = ta.add<int>(n + 2, &doff);
   MpBatchPav* pv = ta.add<MpBatchPav>(n, &dpv);
   int* pvoff = ta.add<int>(n + 1, &dpvoff);
-  auto cls = [](const MatConst& mc) { return (mc.n_e4 == 80 && mc.a_e4 == 9) ? 0 : 1; };
+  auto cls = [](const MatConst& mc) { return example_class(mc) ? 0 : 1; };
   int n0 = 0;
   for (int i = 0; i < n; ++i) n0 += cls(items[i].mc) == 0 ? 1 : 0;
   int k0 = 0, k1 = n0;
-  int64_t maxN = 0;
   for (int i = 0; i < n; ++i) {
     const MpBatchItem& it = items[i];
     const MpState& s = it.s;
     if (s.N > ((int64_t)1 << 29)) throw std::runtime_error("material-point planes longer than 2^29 cells");
-    if (!s.repivot || !it.ill || !it.sub) throw std::runtime_error("incomplete batch item");
+    if (!it.ill || !it.sub) throw std::runtime_error("incomplete batch item");
     const int e = cls(it.mc) == 0 ? k0++ : k1++;
-    ka[e] = KernelArgs{s, it.mc, it.dt, it.ill, nullptr, s.repivot, it.sub, 0, s.N};
+    ka[e] = KernelArgs{s, it.mc, it.dt, it.ill, nullptr, it.sub, 0, s.N};
     // no pav_partial: the P sums come from elsewhere (no blocks)
     pv[e] = MpBatchPav{s.P, s.N, it.pav_partial, it.pav_partial ? mp_partial_blocks(s.N) : 0};
-    maxN = std::max(maxN, s.N);
   }
   // block offsets: class 0 in off[0..n0], class 1 in off[n0+1..n+1]
   int64_t tot = 0;
@@ -1702,18 +1673,12 @@ void launch_mp_response_batch(const MpBatchItem* items, int n, TableArena& ta, h
   ta.upload(off, n + 2, st);
   ta.upload(pv, n, st);
   ta.upload(pvoff, n + 1, st);
-  hipLaunchKernelGGL(repivot_reset_batch_kernel, dim3((n + 63) / 64), dim3(64), 0, st, dka, n);
-  // pivoting pass: enough lanes per RVE for its list (about 1 % of its points)
-  const int x2 = (int)std::min<int64_t>(1024, std::max<int64_t>(16, (maxN + 1023) / 1024));
-  if (n0 > 0) {
+  hipLaunchKernelGGL(ill_reset_batch_kernel, dim3((n + 63) / 64), dim3(64), 0, st, dka, n);
+  if (n0 > 0)
     hipLaunchKernelGGL((mp_response_batch_kernel<80, 9>), dim3((unsigned)blocks0), dim3(64), 0, st, dka, doff, n0);
-    hipLaunchKernelGGL((mp_repivot_batch_kernel<80, 9>), dim3(x2, n0), dim3(64), 0, st, dka);
-  }
-  if (n > n0) {
+  if (n > n0)
     hipLaunchKernelGGL((mp_response_batch_kernel<-1, -1>), dim3((unsigned)blocks1), dim3(64), 0, st, dka + n0,
                        doff + n0 + 1, n - n0);
-    hipLaunchKernelGGL((mp_repivot_batch_kernel<-1, -1>), dim3(x2, n - n0), dim3(64), 0, st, dka + n0);
-  }
   if (pav_blocks > 0)
     hipLaunchKernelGGL(pav_partial_batch_kernel, dim3((unsigned)pav_blocks), dim3(256), 0, st, dpv, dpvoff, n);
   SCA_HIP(hipGetLastError());

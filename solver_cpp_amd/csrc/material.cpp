@@ -43,6 +43,10 @@ void build_matconst(const sc_material& m, const sc_phase_numerics& p, MatConst& 
   o.eps_abs_Lp = p.eps_abs_Lp;
   o.n_e4 = quarter(m.n_sl);
   o.a_e4 = quarter(m.a_sl);
+  o.newton_vg = o.v * o.gdot0;
+  o.newton_f = o.newton_vg * o.n;
+  o.newton_fA = o.newton_f * (o.v * o.C44);
+  o.newton_d = o.C44 / (o.C11 - o.C12);
 }
 
 // qu2om with P = -1 (rotations.f90:423-447), (3,3) column-major out

@@ -3,17 +3,13 @@
 //
 // The kernels are those of sc_mp_update (launch_mp_response, launch_mp_tangent).
 // The device memory they need beyond the caller's inputs and outputs -- the
-// substep scratch planes, the list of points the pivoting pass redoes and the
-// terminally-ill flag -- lives in `scratch`, one fixed array per GPU that the
+// substep scratch planes -- lives in `scratch`, one fixed array per GPU that the
 // code object carries.  In host code `scratch` names a host-side stand-in, not
 // the device array: its device address is taken once per device with
 // hipGetSymbolAddress and only that address is ever handed to kernels.
 //
 // Every call on a GPU shares that GPU's array and leaves its contents behind.
-// The pivoting list's count and the flag are cleared by a kernel at the start
-// of each update (a kernel, not hipMemsetAsync, so that the update can be
-// captured into a HIP graph); the substep planes of a point are written before
-// they are read.  Two calls that overlap on one GPU race on the array: callers
+// The substep planes of a point are written before they are read.  Two calls that overlap on one GPU race on the array: callers
 // serialise them (one stream, or one call at a time).
 #include <mutex>
 
@@ -28,13 +24,7 @@ namespace {
 constexpr int64_t MAX_POINTS = SC_MP_NOALLOC_MAX_POINTS;
 constexpr int NOALLOC_SUB_PLANES = 60;  // planes of substep scratch per point
 constexpr int64_t SUB_DOUBLES = NOALLOC_SUB_PLANES * MAX_POINTS;
-// ints after the substep planes: the flag at 0, the pivoting list from 64 on
-// (a count and up to MAX_POINTS cells)
-constexpr int64_t INT_LIST = 64;
-constexpr int64_t INTS = INT_LIST + 1 + MAX_POINTS;
-constexpr int64_t SCRATCH_DOUBLES = SUB_DOUBLES + (INTS + 1) / 2;
-
-static __device__ __align__(256) double scratch[SCRATCH_DOUBLES];
+static __device__ __align__(256) double scratch[SUB_DOUBLES];
 
 constexpr int MAX_DEVICES = 64;
 std::mutex g_mu;
@@ -97,10 +87,8 @@ extern "C" int sc_mp_update_noalloc(int64_t n, double dt, const sc_material* m, 
     s.xi = pl->xi;
     s.gamma = pl->gamma;
     s.iters = pl->iterations;
-    int* ints = reinterpret_cast<int*>(base + SUB_DOUBLES);
-    s.repivot = ints + INT_LIST;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    launch_mp_response(s, mc, dt, ints, base, st, pl->broken);
+    launch_mp_response(s, mc, dt, nullptr, base, st, pl->broken);
     if (pl->dPdF) launch_mp_tangent(s, mc, dt, pl->dPdF, st);
     return 0;
   } catch (std::exception& e) {
