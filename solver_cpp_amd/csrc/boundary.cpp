@@ -179,7 +179,7 @@ void f_materialpoint_initDamask(void) {
     b.dPdF_dev = b.dalloc(81 * (size_t)N);
     b.sub = b.dalloc((size_t)mp_sub_planes() * N);
     SCA_HIP(hipMalloc(&mp.iters, 2 * N * sizeof(int)));
-    SCA_HIP(hipMalloc(&b.d_ill, sizeof(int)));
+    SCA_HIP(hipMalloc(&b.d_ill, 2 * sizeof(int)));
     // Fp0 = orientation matrix of each cell's material (material.f90:155)
     std::vector<double> om(9 * (size_t)nm), fp(9 * (size_t)N);
     for (int m = 0; m < nm; ++m) qu2om_host(&b.mat.orientations[4 * m], &om[9 * m]);
@@ -252,7 +252,7 @@ void f_homogenization_mechanical_response(double* dt, int* cell_start, int* cell
         SCA_HIP(hipStreamSynchronize(b.st));
       }
     }
-    launch_mp_response(b.mp, b.mc, *dt, b.d_ill, b.sub, b.st, nullptr, c0, c1);
+    launch_mp_points(b.mp, b.mc, *dt, b.d_ill, b.sub, b.st, nullptr, c0, c1);
     int ill = 0;
     SCA_HIP(hipMemcpyAsync(&ill, b.d_ill, sizeof(int), hipMemcpyDeviceToHost, b.st));
     SCA_HIP(hipStreamSynchronize(b.st));

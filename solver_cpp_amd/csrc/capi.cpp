@@ -850,7 +850,7 @@ int sc_mp_update(int64_t n, double dt, const sc_material* m, const sc_phase_nume
     double** t12[4] = {&st.xi0, &st.gamma0, &st.xi, &st.gamma};
     for (int k = 0; k < 4; ++k) *t12[k] = b + (int64_t)90 * n + (int64_t)12 * n * k;
     int *d_ill = nullptr, *d_br = nullptr, *d_it = nullptr;
-    SCA_HIP(hipMalloc(&d_ill, sizeof(int)));
+    SCA_HIP(hipMalloc(&d_ill, 2 * sizeof(int)));
     std::unique_ptr<int, void (*)(int*)> g1(d_ill, [](int* p) { (void)hipFree(p); });
     SCA_HIP(hipMalloc(&d_br, n * sizeof(int)));
     std::unique_ptr<int, void (*)(int*)> g2(d_br, [](int* p) { (void)hipFree(p); });
@@ -874,7 +874,7 @@ int sc_mp_update(int64_t n, double dt, const sc_material* m, const sc_phase_nume
     up(Lp, st.Lp, 9);
     up(xi0, st.xi0, 12);
     up(gamma0, st.gamma0, 12);
-    sca::launch_mp_response(st, mc, dt, d_ill, sub.p, s.s, d_br);
+    sca::launch_mp_points(st, mc, dt, d_ill, sub.p, s.s, d_br);
     down(st.Lp, Lp, 9);
     down(st.P, P, 9);
     down(st.Fp, Fp, 9);

@@ -54,9 +54,9 @@ struct MatConst {
   // are, so that x^e = x^(e4/4 integer part) * x^(quarter part) needs only
   // squarings and square roots; -1 means "use pow()"
   int n_e4, a_e4;
-  // scalars of the Newton system (newton_step, constitutive.hip):
-  // v gdot0, v n gdot0, that times v C44, and C44 / (C11 - C12)
-  double newton_vg, newton_f, newton_fA, newton_d;
+  // scalars of the point updates (points.hip): 1 / xi_inf, v gdot0,
+  // v^2 n gdot0, that times C44, and C44 / (C11 - C12)
+  double rxi_inf, newton_vg, newton_f, newton_fA, newton_d;
 };
 
 // Host-side setup (material.cpp)
@@ -83,6 +83,7 @@ struct MpState {
   double* xi = nullptr;
   double* gamma = nullptr;
   int* iters = nullptr;      // (2,N): Newton iterations, state iterations of the last update
+  int* repivot = nullptr;    // (1 + N): list of the points the solver's pivoting pass redoes (count first)
 };
 
 // Argument tables of batched launches: pinned host staging and a device
@@ -137,12 +138,16 @@ struct MpBatchPav {
 };
 
 // Kernel launchers (constitutive.hip)
-// cells [c_begin, c_end) of the planes (c_end < 0: all N); *d_ill (may be
-// null) is cleared by the launch and set when a point is terminally ill
-void launch_mp_response(const MpState& s, const MatConst& mc, double dt, int* d_ill, double* d_sub, hipStream_t st,
-                        int* d_broken = nullptr, int64_t c_begin = 0, int64_t c_end = -1);
+// callers' point updates: cells [c_begin, c_end) of the planes (c_end < 0: all
+// N); *d_ill (may be null) is cleared by the launch and set when a point is
+// terminally ill
+void launch_mp_points(const MpState& s, const MatConst& mc, double dt, int* d_ill, double* d_sub, hipStream_t st,
+                      int* d_broken = nullptr, int64_t c_begin = 0, int64_t c_end = -1);
+// the grid solver's update of all cells (needs s.repivot); *d_ill as above
+void launch_mp_response(const MpState& s, const MatConst& mc, double dt, int* d_ill, double* d_sub, hipStream_t st);
 int mp_partial_blocks(int64_t N);
-// Material-point updates of n RVEs in one launch (and their P block sums), each RVE's results bitwise those of launch_mp_response
+// Material-point updates of n RVEs in one launch (and their pivoting passes
+// and P block sums), each RVE's results bitwise those of launch_mp_response
 // + launch_pav_partial; the argument tables go into ta.
 void launch_mp_response_batch(const MpBatchItem* items, int n, TableArena& ta, hipStream_t st);
 int mp_sub_planes();

@@ -10,80 +10,17 @@
 //   phenopowerlaw LpAndItsTangent / dotState / kinetics_sl
 //                                        phase_mechanical_plastic_phenopowerlaw.f90:298-483
 // with Fi = I and Li = 0 (no eigen kinematics are active).  The 9x9 Newton
-// Jacobian I - dLp/dS : dS/dFe : dFe/dLp is the identity plus a matrix of rank
-// five (the resolved shears see the five deviatoric numbers of the stress), so
-// its system is solved as a 5x5 one (newton_step).
-#include <cmath>
-
-#include "common.h"
+// Jacobian I - dLp/dS : dS/dFe : dFe/dLp is assembled directly from its
+// rank-12 structure: with G = Fe^T A and K_s = P_s : C (cubic),
+//   J[(a,b),(p,l)] = delta + dt * sum_s c_s P_s(a,b) (G^T K_s)(p,l),
+// c_s = d(gamma_dot_s)/d(tau_s) * sign_s, instead of three 3x3x3x3 products;
+// the sum over s is taken from the slip groups' Hadamard sums
+// (assemble_jacobian8), on the 8 traceless coordinates.
+#include "mp_device.h"
 
 namespace sca {
 
 namespace {
-
-// cF <110>{111} slip systems (crystal.f90:41-63): direction, normal.
-__device__ constexpr int SLIP[NSLIP][6] = {
-    {0, 1, -1, 1, 1, 1},   {-1, 0, 1, 1, 1, 1},   {1, -1, 0, 1, 1, 1},
-    {0, -1, -1, -1, -1, 1}, {1, 0, 1, -1, -1, 1},  {-1, 1, 0, -1, -1, 1},
-    {0, -1, 1, 1, -1, -1}, {-1, 0, -1, 1, -1, -1}, {1, 1, 0, 1, -1, -1},
-    {0, 1, 1, -1, 1, -1},  {1, 0, -1, -1, 1, -1},  {-1, -1, 0, -1, 1, -1}};
-
-// sign pattern of P_s(i,j) = d_i n_j
-__device__ __forceinline__ constexpr int psg(int s, int i, int j) { return SLIP[s][i] * SLIP[s][3 + j]; }
-
-// cF slip-slip interaction types (reacting, acting), crystal.f90:623-640
-__device__ constexpr int HTYPE[NSLIP][NSLIP] = {
-    {1, 2, 2, 4, 7, 5, 3, 5, 5, 4, 6, 7}, {2, 1, 2, 7, 4, 5, 6, 4, 7, 5, 3, 5},
-    {2, 2, 1, 5, 5, 3, 6, 7, 4, 7, 6, 4}, {4, 7, 6, 1, 2, 2, 4, 6, 7, 3, 5, 5},
-    {7, 4, 6, 2, 1, 2, 5, 3, 5, 6, 4, 7}, {5, 5, 3, 2, 2, 1, 7, 6, 4, 6, 7, 4},
-    {3, 5, 5, 4, 6, 7, 1, 2, 2, 4, 7, 6}, {6, 4, 7, 5, 3, 5, 2, 1, 2, 7, 4, 6},
-    {6, 7, 4, 7, 6, 4, 2, 2, 1, 5, 5, 3}, {4, 6, 7, 3, 5, 5, 4, 7, 6, 1, 2, 2},
-    {5, 3, 5, 6, 4, 7, 7, 4, 6, 2, 1, 2}, {7, 6, 4, 6, 7, 4, 5, 5, 3, 2, 2, 1}};
-
-// Structure of the table used to share work between slip systems:
-// - the systems 3p, 3p+1, 3p+2 lie on the same plane (normal), p = 0..3;
-// - the systems g, g+3, g+6, g+9 (g = 0, 1, 2) have direction component g
-//   zero.
-// The Newton step (newton_step) needs, for every entry r = 3i+j and
-// every symmetric pair (m,l), the sum over s of f_s P_s(i,j) k_s(m,l) with
-// k_s(m,l) = P_s(m,m) (m = l) or P_s(m,l) + P_s(l,m).  Restricted to one
-// direction group its coefficient vector is zero or plus/minus one of the
-// four Hadamard rows (1,1,1,1), (1,1,-1,-1), (1,-1,1,-1), (1,-1,-1,1), so
-// the sums come from the four Hadamard sums of each group's f_s.
-__device__ __forceinline__ constexpr int qcoef(int s, int r, int m, int l) {
-  return psg(s, r / 3, r % 3) * (m == l ? psg(s, m, m) : psg(s, m, l) + psg(s, l, m));
-}
-// 0 when group g does not enter Q_r(m,l), else sign * (1 + Hadamard row)
-__device__ __forceinline__ constexpr int qhad(int g, int r, int m, int l) {
-  const int a = qcoef(g, r, m, l), b = qcoef(g + 3, r, m, l), c = qcoef(g + 6, r, m, l);
-  if (a == 0) return 0;
-  return a * (1 + (b * a > 0 ? (c * a > 0 ? 0 : 1) : (c * a > 0 ? 2 : 3)));
-}
-constexpr bool slip_structure_holds() {
-  for (int p = 0; p < 4; ++p)
-    for (int k = 1; k < 3; ++k)
-      for (int j = 0; j < 3; ++j)
-        if (SLIP[3 * p + k][3 + j] != SLIP[3 * p][3 + j]) return false;
-  for (int s = 0; s < NSLIP; ++s)
-    if (SLIP[s][s % 3] != 0) return false;
-  const int had[4][4] = {{1, 1, 1, 1}, {1, 1, -1, -1}, {1, -1, 1, -1}, {1, -1, -1, 1}};
-  for (int r = 0; r < 9; ++r)
-    for (int m = 0; m < 3; ++m)
-      for (int l = m; l < 3; ++l) {
-        int groups = 0;
-        for (int g = 0; g < 3; ++g) {
-          const int code = qhad(g, r, m, l);
-          for (int k = 0; k < 4; ++k) {
-            const int want = code == 0 ? 0 : (code > 0 ? 1 : -1) * had[(code > 0 ? code : -code) - 1][k];
-            if (qcoef(g + 3 * k, r, m, l) != want) return false;
-          }
-          groups += code != 0;
-        }
-        if (groups == 0) return false;
-      }
-  return true;
-}
-static_assert(slip_structure_holds(), "cF slip table: planes of three systems, Hadamard-structured sums");
 
 // Material constants travel in the kernel arguments (not a __constant__
 // symbol) so that launches of different contexts on concurrent streams never
@@ -92,238 +29,41 @@ struct KernelArgs {
   MpState s;
   MatConst mc;
   double dt;
-  int* ill;     // may be null
-  int* broken;  // per point, may be null
+  int* ill;
   double* sub;  // substep scratch, SUB_PLANES planes of N doubles
-  int64_t c_begin, c_end;  // cells [c_begin, c_end) of the N-cell planes
 };
 
-
-// ---- small dense helpers (row-major 3x3 in registers: m[3*i+j]) ----------
-__device__ __forceinline__ void mm33(const double* A, const double* B, double* C) {
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) C[3 * i + j] = A[3 * i] * B[j] + A[3 * i + 1] * B[3 + j] + A[3 * i + 2] * B[6 + j];
-}
-
-// Divisions without the compiler's range fix-ups, for operands far from the
-// range limits (slip resistances, the 3x3 determinants of deformation
-// gradients, the pivots of the Newton system, none of them near 2^+-1000):
-// 1/x as the hardware reciprocal refined by two Newton steps (as the
-// compiler's own division does before its fix-ups), and a / b as the rounded
-// product a (1/b) corrected once by its exact remainder a - b q (Markstein):
-// the correctly rounded quotient when 1/b is the correctly rounded
-// reciprocal, within one rounding of it otherwise
-__device__ __forceinline__ double rcp_refined(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-#pragma unroll
-  for (int k = 0; k < 2; ++k) r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
-  return r;
-}
-__device__ __forceinline__ double div_rcp(double a, double b, double rb) {
-  const double q = a * rb;
-  return __builtin_fma(__builtin_fma(-q, b, a), rb, q);
-}
-
-// math_invert33 (math.f90:511-545); returns false if |det| <= 10*tiny
-__device__ __forceinline__ bool inv33(const double* A, double* R, double* detOut) {
-  R[0] = A[4] * A[8] - A[5] * A[7];
-  R[3] = -A[3] * A[8] + A[5] * A[6];
-  R[6] = A[3] * A[7] - A[4] * A[6];
-  double det = A[0] * R[0] + A[1] * R[3] + A[2] * R[6];
-  if (fabs(det) <= 2.2250738585072014e-308 * 10.0) return false;
-  R[1] = -A[1] * A[8] + A[2] * A[7];
-  R[4] = A[0] * A[8] - A[2] * A[6];
-  R[7] = -A[0] * A[7] + A[1] * A[6];
-  R[2] = A[1] * A[5] - A[2] * A[4];
-  R[5] = -A[0] * A[5] + A[2] * A[3];
-  R[8] = A[0] * A[4] - A[1] * A[3];
-  const double rd = rcp_refined(det);
-#pragma unroll
-  for (int k = 0; k < 9; ++k) R[k] = div_rcp(R[k], det, rd);
-  if (detOut) *detOut = det;
-  return true;
-}
-
-__device__ __forceinline__ double det33(const double* m) {
-  return m[0] * (m[4] * m[8] - m[5] * m[7]) - m[1] * (m[3] * m[8] - m[5] * m[6]) + m[2] * (m[3] * m[7] - m[4] * m[6]);
-}
-
-
-// x^e for x >= 0 with e = e4/4: binary powering of the integer part times
-// sqrt / sqrt-sqrt for the quarter part; libm pow() when e4 < 0
-__device__ __noinline__ double pow_general(double x, double e) { return pow(x, e); }
-__device__ __forceinline__ double powq(double x, int e4, double e) {
-  if (e4 < 0) return pow_general(x, e);
-  double r = 1.0, b = x;
-  int m = e4 >> 2;
-  while (m) {
-    if (m & 1) r *= b;
-    b *= b;
-    m >>= 1;
-  }
-  const int q = e4 & 3;
-  if (q) {
-    const double h = sqrt(x);
-    const double f = sqrt(h);
-    r *= (q == 1) ? f : (q == 2) ? h : h * f;
-  }
-  return r;
-}
-// compile-time quarter exponent E4/4 (E4 >= 0): fully unrolled
-// x^(-1/4) for x in [2^-1000, 2^1000]: a start value from the hardware
-// square root and reciprocal square root, then three Newton steps
-// y <- y (5 - x y^4) / 4 (quadratic: full precision from any start within
-// 2^-8 of the root); two correctly rounded square roots cost about three
-// times as many instructions
-__device__ __forceinline__ double rqrt_refined(double x) {
-  double y = __builtin_amdgcn_rsq(__builtin_amdgcn_sqrt(x));
-  const double mq = -0.25 * x;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const double y2 = y * y;
-    y = y * __builtin_fma(mq, y2 * y2, 1.25);
-  }
-  return y;
-}
-
-template <int E4>
-__device__ __forceinline__ double powc(double x) {
-  double r = 1.0, b = x;
-#pragma unroll
-  for (int m = E4 >> 2; m; m >>= 1) {
-    if (m & 1) r *= b;
-    b *= b;
-  }
-  constexpr int q = E4 & 3;
-  if constexpr (q == 2) {
-    r *= sqrt(x);
-  } else if constexpr (q != 0) {
-    // x^(1/4) = x y^3 and x^(3/4) = x y with y = x^(-1/4) (within 10 ulp),
-    // y taken at x clamped to [2^-1000, 2^1000] and multiplied by the true x:
-    // for x = 0 this gives 0, NaN propagates, and outside the range the
-    // power x^(E4 >> 2) >= x^1 (E4 >= 4) underflows to 0 or overflows to inf
-    // as the exact result does (E4 < 4 exponents run the runtime path)
-    static_assert(E4 >= 4, "quarter exponents below 1 are not compiled in");
-    const double y = rqrt_refined(fmin(fmax(x, 0x1p-1000), 0x1p1000));
-    r *= (q == 1) ? x * (y * (y * y)) : x * y;
-  }
-  return r;
-}
-// exponent dispatch: E4 >= 0 compile-time, E4 == -1 runtime (mc)
-template <int E4>
-__device__ __forceinline__ double powe(double x, int e4rt, double e) {
-  if constexpr (E4 >= 0) return powc<E4>(x);
-  else return powq(x, e4rt, e);
-}
-
-// Hooke (elastic.f90:157-195) with Fi = I, cubic C66:
-// E = (Fe^T Fe - I)/2, S = C66 : E (Voigt strain with engineering shear)
-__device__ __forceinline__ void hooke_S(const double* Fe, double* S, const MatConst& mc) {
-  double E[9];
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-      E[3 * i + j] = 0.5 * ((Fe[i] * Fe[j] + Fe[3 + i] * Fe[3 + j] + Fe[6 + i] * Fe[6 + j]) - (i == j ? 1.0 : 0.0));
-  const double e11 = E[0], e22 = E[4], e33 = E[8];
-  const double s11 = mc.C11 * e11 + mc.C12 * e22 + mc.C12 * e33;
-  const double s22 = mc.C12 * e11 + mc.C11 * e22 + mc.C12 * e33;
-  const double s33 = mc.C12 * e11 + mc.C12 * e22 + mc.C11 * e33;
-  const double s23 = mc.C44 * (2.0 * E[7]);
-  const double s13 = mc.C44 * (2.0 * E[6]);
-  const double s12 = mc.C44 * (2.0 * E[1]);
-  S[0] = s11; S[1] = s12; S[2] = s13;
-  S[3] = s12; S[4] = s22; S[5] = s23;
-  S[6] = s13; S[7] = s23; S[8] = s33;
-}
-
-// tau_s = Mp : P_s with Mp = S (Fi = I), for all systems: tau_s = v d_s . (S n_s),
-// the three systems of a plane sharing S n (signed sums: every entry of d_s and
-// n_s is 0 or +-1)
-__device__ __forceinline__ void resolved_shears(const double* S, double v, double* tau) {
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    double u[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      double t = SLIP[3 * p][3] > 0 ? S[3 * i] : -S[3 * i];
-#pragma unroll
-      for (int j = 1; j < 3; ++j) t = SLIP[3 * p][3 + j] > 0 ? t + S[3 * i + j] : t - S[3 * i + j];
-      u[i] = t;
-    }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const int s = 3 * p + k;
-      double t = 0.0;
-      bool first = true;
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-        if (SLIP[s][i] != 0) {
-          t = first ? (SLIP[s][i] > 0 ? u[i] : -u[i]) : (SLIP[s][i] > 0 ? t + u[i] : t - u[i]);
-          first = false;
-        }
-      tau[s] = v * t;
-    }
-  }
-}
-
-// Lp = v sum_s g_s d_s n_s^T, the systems of a plane summed first:
-// Lp = v sum_p (sum_{s on p} g_s d_s) n_p^T (row-major 3x3 out)
-__device__ __forceinline__ void slip_sum(const double* g, double v, double* L) {
-  double w[4][3];
-#pragma unroll
-  for (int p = 0; p < 4; ++p)
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      double t = 0.0;
-      bool first = true;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const int s = 3 * p + k;
-        if (SLIP[s][i] != 0) {
-          t = first ? (SLIP[s][i] > 0 ? g[s] : -g[s]) : (SLIP[s][i] > 0 ? t + g[s] : t - g[s]);
-          first = false;
-        }
-      }
-      w[p][i] = t;
-    }
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      double t = SLIP[0][3 + j] > 0 ? w[0][i] : -w[0][i];
-#pragma unroll
-      for (int p = 1; p < 4; ++p) t = SLIP[3 * p][3 + j] > 0 ? t + w[p][i] : t - w[p][i];
-      L[3 * i + j] = v * t;
-    }
-}
-
-// kinetics_sl (phenopowerlaw.f90:444-483) with tau_pos = t, tau_neg = -t:
-// gamma_dot_s = sign(tau_s) gdot0 x_s^n, x_s = |tau_s| / xi_s, and its
-// derivative c_s = gdot0 n x_s^(n-1) / xi_s.  Gives pw_s = x_s^n and (DERIV)
-// pm_s = x_s^(n-1) / xi_s; sign, gdot0 and n are left to the caller, which
-// multiplies a sum by them instead of every term.  Takes the reciprocal slip
-// resistances rxi = 1/xi (xi is fixed during the Newton iteration, so the
-// divisions are done once per state iteration).  A compile-time exponent
-// takes both powers from one chain; there is no zero test on it: c_s of a
-// rate below 1e-306 is below 1e-290 and changes no Newton system.
-template <int NE4, bool DERIV>
-__device__ __forceinline__ void slip_powers(const double* tau, const double* rxi, double* pw, double* pm,
-                                            const MatConst& mc) {
+// kinetics_sl (phenopowerlaw.f90:444-483): tau_pos = t, tau_neg = -t, taking
+// the reciprocal slip resistances rxi = 1/xi (xi is fixed during the Newton
+// iteration, so the divisions are done once per state iteration).
+// dLp/dMp = sum_s c_s P_s (x) P_s with c_s = |gdot_s| n / |tau_s|; for a
+// compile-time exponent this is gdot0 n x^(n-1) / xi, x = |tau_s| / xi, taken
+// from the same powering chain without a division.
+template <int NE4>
+__device__ __forceinline__ void kinetics(const double* S, const double* rxi, double* dg, double* c,
+                                         const MatConst& mc) {
   constexpr double TINY10 = 2.2250738585072014e-308 * 10.0;
+  double tau[NSLIP];
+  resolved_shears(S, mc.v, tau);
 #pragma unroll
   for (int s = 0; s < NSLIP; ++s) {
-    const double t = fabs(tau[s]);
-    const double x = t * rxi[s];
-    if constexpr (NE4 >= 8) {
+    const double tp = tau[s];
+    const double tn = -tp;
+    const double sgn = (tp > tn) ? 1.0 : -1.0;
+    const double tmax = fmax(tp, tn);
+    const double x = tmax * rxi[s];
+    if constexpr (NE4 >= 4) {
       const double xm1 = powc<NE4 - 4>(x);
-      pw[s] = xm1 * x;
-      if constexpr (DERIV) pm[s] = xm1 * rxi[s];
+      const double g = sgn * mc.gdot0 * (xm1 * x);
+      dg[s] = g;
+      if (c) c[s] = (fabs(g) <= TINY10) ? 0.0 : mc.gdot0 * mc.n * xm1 * rxi[s];
     } else {
-      pw[s] = powe<NE4>(x, mc.n_e4, mc.n);
-      if constexpr (DERIV) pm[s] = (mc.gdot0 * pw[s] <= TINY10) ? 0.0 : pw[s] / t;
+      const double g = sgn * mc.gdot0 * powe<NE4>(x, mc.n_e4, mc.n);
+      dg[s] = g;
+      if (c) {
+        const double dd = (fabs(g) <= TINY10) ? 0.0 : g * mc.n / tmax;
+        c[s] = dd * ((g > 0.0) ? 1.0 : -1.0);
+      }
     }
   }
 }
@@ -333,12 +73,11 @@ __device__ __forceinline__ void slip_powers(const double* tau, const double* rxi
 template <int NE4, int AE4>
 __device__ __forceinline__ void dot_state(const double* S, const double* st, const double* rxi, double* dot,
                                           const MatConst& mc) {
-  double tau[NSLIP], dg[NSLIP];
-  resolved_shears(S, mc.v, tau);
-  slip_powers<NE4, false>(tau, rxi, dg, nullptr, mc);
+  double dg[NSLIP];
+  kinetics<NE4>(S, rxi, dg, nullptr, mc);
   const double rxinf = 1.0 / mc.xi_inf;
 #pragma unroll
-  for (int s = 0; s < NSLIP; ++s) dg[s] = mc.gdot0 * dg[s];
+  for (int s = 0; s < NSLIP; ++s) dg[s] = fabs(dg[s]);
 #pragma unroll
   for (int s = 0; s < NSLIP; ++s) {
     const double x = 1.0 - st[s] * rxinf;
@@ -352,63 +91,28 @@ __device__ __forceinline__ void dot_state(const double* S, const double* st, con
   for (int s = 0; s < NSLIP; ++s) dot[NSLIP + s] = dg[s];
 }
 
-// The Newton system of the Lp iteration, J x = b, as a 5x5 system.
-//
-// A change x of Lp (traceless, as b and every P_s are) changes the stress by
-// dS = -dt C : sym(X), X = G x, G = Fe^T A, and the constitutive Lp by
-// sum_s c_s P_s (P_s : dS), so
-//   J x = x + dt sum_s c_s P_s (P_s : C : sym(X)).
-// P_s is traceless and C cubic: P_s : C : sym(X) is a combination of the five
-// numbers w(x) = (X00 - X22, X11 - X22, X01 + X10, X02 + X20, X12 + X21) with
-// the coefficients kD sgn_s(0,0), kD sgn_s(1,1), kA k_s(0,1), kA k_s(0,2),
-// kA k_s(1,2) (kD = v (C11 - C12), kA = v C44, P_s = v sgn_s).  With
-// f_s = dt v c_s and the five matrices U_j = sum_s f_s sgn_s k_s(j) that is
-//   J x = x + sum_j kappa_j U_j w_j(x),
-// and applying w to J x = b leaves the 5x5 system
-//   (1/kappa_i delta_ij + w_i(U_j)) y_j = w_i(b),   x = b - sum_j U_j y_j,
-// y_i = kappa_i w_i(x).
-// The same solution as that of the 9x9 system (up to rounding), from 25
-// instead of 81 (traceless: 64) matrix entries.  G is near the identity, which
-// makes the 5x5 matrix near a symmetric positive definite one times a 2x2
-// block: its LU rarely needs row exchanges.  Every entry of every U_j is plus
-// or minus one of 23 sums of one or two of the Hadamard sums of the direction
-// groups' f_s (qhad), formed once.
-//
-// GENERAL: rows scaled by kappa_i instead of divided by it (any C44 and
-// C11 - C12, zero included); otherwise f_s carries kA and the first two
-// diagonal entries are kA / kD (30 multiplications fewer).
-constexpr int NW = 5;
-__device__ __forceinline__ constexpr int um(int j) { return j == 0 ? 0 : j == 1 ? 1 : j == 2 ? 0 : j == 3 ? 0 : 1; }
-__device__ __forceinline__ constexpr int ul(int j) { return j == 0 ? 0 : j == 1 ? 1 : j == 2 ? 1 : j == 3 ? 2 : 2; }
-// sign of the first term of U_j(r), so that entries equal up to their sign
-// are the same expression
-__device__ __forceinline__ constexpr int usign(int j, int r) {
-  for (int g = 0; g < 3; ++g) {
-    const int code = qhad(g, r, um(j), ul(j));
-    if (code != 0) return code > 0 ? 1 : -1;
-  }
-  return 1;
-}
-// the five numbers w of X = G x (x row-major 3x3)
-__device__ __forceinline__ void newton_w(const double* G, const double* x, double* w) {
-  const double x22 = G[6] * x[2] + G[7] * x[5] + G[8] * x[8];
-  w[0] = G[0] * x[0] + G[1] * x[3] + G[2] * x[6] - x22;
-  w[1] = G[3] * x[1] + G[4] * x[4] + G[5] * x[7] - x22;
-  w[2] = G[0] * x[1] + G[1] * x[4] + G[2] * x[7] + G[3] * x[0] + G[4] * x[3] + G[5] * x[6];
-  w[3] = G[0] * x[2] + G[1] * x[5] + G[2] * x[8] + G[6] * x[0] + G[7] * x[3] + G[8] * x[6];
-  w[4] = G[3] * x[2] + G[4] * x[5] + G[5] * x[8] + G[6] * x[1] + G[7] * x[4] + G[8] * x[7];
-}
+// The Newton system J x = b of the Lp iteration lives in the traceless
+// subspace: every P_s is traceless, so J maps traceless matrices to traceless
+// ones, and b = Lp - Lp_constitutive is traceless.  Its solution is therefore
+// traceless and solves the 8x8 system on the coordinates
+//   y_k = x_k (k = 1,2,3,5,6,7, the off-diagonal row-major positions),
+//   y_0 = x_00, y_4 = x_11 (x_22 = -y_0 - y_4),
+// taking the rows 0..7 of J (row 8 = -(row 0 + row 4) on this subspace) and,
+// for the columns 0 and 4, J[:,k] - J[:,8].  The 9x9 solution is recovered
+// exactly; this is the same linear solve with an 8x8 factorisation.
+constexpr int NR = 8;
 
-// Solves M y = b (NW x NW, row-major) by LU with partial pivoting (first
-// largest entry of the column, as LAPACK's idamax); false: singular.
-__device__ __forceinline__ bool solve_pivot(double* M, double* b) {
+// Solve J y = b (8x8, row-major) by LU with partial pivoting (first largest
+// entry of the column, as LAPACK's idamax).  Used only by the pivoting pass
+// (its own kernel), with J in registers.
+__device__ __forceinline__ bool solve8_pivot(double* J, double* b) {
 #pragma unroll
-  for (int k = 0; k < NW; ++k) {
+  for (int k = 0; k < NR; ++k) {
     int p = k;
-    double mx = fabs(M[NW * k + k]);
+    double mx = fabs(J[NR * k + k]);
 #pragma unroll
-    for (int i = k + 1; i < NW; ++i) {
-      const double v = fabs(M[NW * i + k]);
+    for (int i = k + 1; i < NR; ++i) {
+      const double v = fabs(J[NR * i + k]);
       if (v > mx) {
         mx = v;
         p = i;
@@ -418,239 +122,194 @@ __device__ __forceinline__ bool solve_pivot(double* M, double* b) {
     // exchange rows k and p by selects over the candidate rows (static
     // register indices; the columns left of k are not read again)
 #pragma unroll
-    for (int i = k + 1; i < NW; ++i) {
+    for (int i = k + 1; i < NR; ++i) {
       const bool sw = p == i;
 #pragma unroll
-      for (int c = k; c < NW; ++c) {
-        const double u = M[NW * k + c], w = M[NW * i + c];
-        M[NW * k + c] = sw ? w : u;
-        M[NW * i + c] = sw ? u : w;
+      for (int c = k; c < NR; ++c) {
+        const double u = J[NR * k + c], w = J[NR * i + c];
+        J[NR * k + c] = sw ? w : u;
+        J[NR * i + c] = sw ? u : w;
       }
       const double u = b[k], w = b[i];
       b[k] = sw ? w : u;
       b[i] = sw ? u : w;
     }
-    const double inv = 1.0 / M[NW * k + k];
+    const double inv = 1.0 / J[NR * k + k];
 #pragma unroll
-    for (int i = k + 1; i < NW; ++i) {
-      const double l = M[NW * i + k] * inv;
+    for (int i = k + 1; i < NR; ++i) {
+      const double l = J[NR * i + k] * inv;
 #pragma unroll
-      for (int c = k + 1; c < NW; ++c) M[NW * i + c] -= l * M[NW * k + c];
+      for (int c = k + 1; c < NR; ++c) J[NR * i + c] -= l * J[NR * k + c];
       b[i] -= l * b[k];
     }
   }
 #pragma unroll
-  for (int i = NW - 1; i >= 0; --i) {
+  for (int i = NR - 1; i >= 0; --i) {
     double s = b[i];
 #pragma unroll
-    for (int c = i + 1; c < NW; ++c) s -= M[NW * i + c] * b[c];
-    b[i] = s / M[NW * i + i];
+    for (int c = i + 1; c < NR; ++c) s -= J[NR * i + c] * b[c];
+    b[i] = s / J[NR * i + i];
   }
   return true;
 }
 
-// Solves M y = b by LU without row exchanges.  Refuses (returns false; b then
-// holds no meaning) when a multiplier exceeds 1e6 in magnitude or a pivot's
-// magnitude is below 2^-1000 (zero and NaN included: the pivot's reciprocal is
-// the refined hardware one, so a pivot near the bottom of the range goes to
-// the pivoted solve and its exact division).  Multipliers up to 1e6 cost at
-// most a few of the 16 digits of a Newton step that needs 6, and the residual
-// test of the next iteration uses the exact residual.  Refusals are collected
-// and tested once at the end (what is computed after one is discarded): no
-// branches inside the unrolled elimination, and the multipliers' magnitudes
-// enter one running maximum (a NaN multiplier is ignored by the maximum).
-__device__ __forceinline__ bool solve_nopivot(double* M, double* b) {
-  bool refused = false;
-  double lmax = 0.0;
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-#pragma unroll
-    for (int k = 0; k < i; ++k) {
-      const double l = M[NW * i + k] * M[NW * k + k];
-      lmax = fmax(lmax, fabs(l));
-#pragma unroll
-      for (int c = k + 1; c < NW; ++c) M[NW * i + c] -= l * M[NW * k + c];
-      b[i] -= l * b[k];
-    }
-    const double piv = M[NW * i + i];
-    refused = refused || !(fabs(piv) >= 0x1p-1000);
-    M[NW * i + i] = rcp_refined(piv);
-  }
-#pragma unroll
-  for (int i = NW - 1; i >= 0; --i) {
-    double s = b[i];
-#pragma unroll
-    for (int c = i + 1; c < NW; ++c) s -= M[NW * i + c] * b[c];
-    b[i] = s * M[NW * i + i];
-  }
-  return !(refused || lmax > 1e6);
-}
+// J = I + dt sum_s c_s vec(P_s) vec(G^T K_s)^T with G = Fe^T A, restricted to
+// the traceless coordinates (rows 0..7; columns 0 and 4 minus column 8), as
+// an 8x8 row-major matrix.
+//
+// K_s = P_s : C for the cubic stiffness (tr P_s = 0) is K_s(m,l) =
+// kappa(m,l) k_s(m,l) with kappa = 2 kA + kB on the diagonal and kA off it,
+// kA = v C44, kB = v (C11 - C12 - 2 C44).  With f_s = dt v c_s, row r = 3i+j is
+//   J(r,(p,l)) = delta + sum_m kappa(m,l) G(m,p) Q_r(m,l),
+//   Q_r(m,l) = sum_s f_s P_s(i,j) k_s(m,l)   (symmetric in m,l),
+// and every Q_r(m,l) is a signed sum of one or two of the twelve Hadamard sums
+// of the direction groups' f_s (qhad): 24 additions for all the Q_r instead of
+// a rank-one update of the 8x8 matrix per slip system.
 
-// The Newton step x of J x = b, in place of b (row-major 3x3, traceless);
-// pm: slip_powers' derivatives.  false: refused (without PIVOT) or singular.
-template <bool GENERAL, bool PIVOT>
-__device__ __forceinline__ bool newton_step(const double* Fe, const double* A, const double* pm, double dt,
-                                            double* b, const MatConst& mc) {
-  double G[9];
+// Row-independent part of the Jacobian: kappa G (or, LEAN, G alone, kappa
+// then scaling Q in every row: 18 registers fewer for 48 more products) and
+// the Hadamard sums
+template <bool LEAN>
+struct JacobianParts {
+  double Gd[9], Go[LEAN ? 1 : 9];  // kappa G for the diagonal / off-diagonal (m,l); LEAN: G in Gd
+  double H[3][4];                  // Hadamard sums of f_s over each direction group
+};
+template <bool LEAN>
+__device__ __forceinline__ void jacobian_parts(const double* Fe, const double* A, const double* c, double dt,
+                                               JacobianParts<LEAN>& jp, const MatConst& mc) {
+  const double kA = mc.v * mc.C44, kB = mc.v * (mc.C11 - mc.C12 - 2.0 * mc.C44);
+  const double kD = 2.0 * kA + kB;
 #pragma unroll
   for (int m = 0; m < 3; ++m)
 #pragma unroll
-    for (int p = 0; p < 3; ++p) G[3 * m + p] = Fe[m] * A[p] + Fe[3 + m] * A[3 + p] + Fe[6 + m] * A[6 + p];
-  // Hadamard sums of f_s over each direction group
-  const double f = dt * (GENERAL ? mc.newton_f : mc.newton_fA);
-  double H[3][4];
+    for (int p = 0; p < 3; ++p) {
+      const double g = Fe[m] * A[p] + Fe[3 + m] * A[3 + p] + Fe[6 + m] * A[6 + p];
+      if constexpr (LEAN) {
+        jp.Gd[3 * m + p] = g;
+      } else {
+        jp.Gd[3 * m + p] = g * kD;
+        jp.Go[3 * m + p] = g * kA;
+      }
+    }
+  const double fv = dt * mc.v;
 #pragma unroll
   for (int g = 0; g < 3; ++g) {
-    const double a = pm[g] * f, bb = pm[g + 3] * f, x = pm[g + 6] * f, y = pm[g + 9] * f;
-    const double ab = a + bb, amb = a - bb, xy = x + y, xmy = x - y;
-    H[g][0] = ab + xy;
-    H[g][1] = ab - xy;
-    H[g][2] = amb + xmy;
-    H[g][3] = amb - xmy;
+    const double a = c[g] * fv, b = c[g + 3] * fv, x = c[g + 6] * fv, y = c[g + 9] * fv;
+    const double ab = a + b, amb = a - b, xy = x + y, xmy = x - y;
+    jp.H[g][0] = ab + xy;
+    jp.H[g][1] = ab - xy;
+    jp.H[g][2] = amb + xmy;
+    jp.H[g][3] = amb - xmy;
   }
-  double U[NW][9];
+}
+// row r of the 8x8 Jacobian
+template <bool LEAN>
+__device__ __forceinline__ void jacobian_row(const JacobianParts<LEAN>& jp, int r, double* row, const MatConst& mc) {
+  double Q[3][3];
 #pragma unroll
-  for (int j = 0; j < NW; ++j)
+  for (int m = 0; m < 3; ++m)
 #pragma unroll
-    for (int r = 0; r < 9; ++r) {
+    for (int l = m; l < 3; ++l) {
       double t = 0.0;
       bool first = true;
 #pragma unroll
       for (int g = 0; g < 3; ++g) {
-        const int code = qhad(g, r, um(j), ul(j)) * usign(j, r);
+        const int code = qhad(g, r, m, l);
         if (code != 0) {
-          const double h = H[g][(code > 0 ? code : -code) - 1];
-          t = first ? h : (code > 0 ? t + h : t - h);
+          const double h = jp.H[g][(code > 0 ? code : -code) - 1];
+          t = first ? (code > 0 ? h : -h) : (code > 0 ? t + h : t - h);
           first = false;
         }
       }
-      U[j][r] = usign(j, r) > 0 ? t : -t;
+      if constexpr (LEAN) {
+        const double kA = mc.v * mc.C44, kB = mc.v * (mc.C11 - mc.C12 - 2.0 * mc.C44);
+        t = t * (m == l ? 2.0 * kA + kB : kA);
+      }
+      Q[m][l] = t;
+      Q[l][m] = t;
     }
-  b[8] = -(b[0] + b[4]);
-  double M[NW * NW], y[NW];
-  newton_w(G, b, y);
+  double Y[9];
 #pragma unroll
-  for (int j = 0; j < NW; ++j) {
-    double w[NW];
-    newton_w(G, U[j], w);
+  for (int p = 0; p < 3; ++p)
 #pragma unroll
-    for (int i = 0; i < NW; ++i) M[NW * i + j] = w[i];
-  }
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    if constexpr (GENERAL) {
-      const double k = mc.v * (i < 2 ? mc.C11 - mc.C12 : mc.C44);
-      y[i] *= k;
-#pragma unroll
-      for (int j = 0; j < NW; ++j) M[NW * i + j] *= k;
-      M[NW * i + i] += 1.0;
-    } else {
-      M[NW * i + i] += i < 2 ? mc.newton_d : 1.0;
+    for (int l = 0; l < 3; ++l) {
+      if constexpr (LEAN) {
+        double y = jp.Gd[p] * Q[0][l];
+        y += jp.Gd[3 + p] * Q[1][l];
+        y += jp.Gd[6 + p] * Q[2][l];
+        Y[3 * p + l] = y;
+      } else {
+        double y = (l == 0 ? jp.Gd : jp.Go)[p] * Q[0][l];
+        y += (l == 1 ? jp.Gd : jp.Go)[3 + p] * Q[1][l];
+        y += (l == 2 ? jp.Gd : jp.Go)[6 + p] * Q[2][l];
+        Y[3 * p + l] = y;
+      }
     }
+#pragma unroll
+  for (int q = 0; q < NR; ++q) {
+    const double y = (q == 0 || q == 4) ? Y[q] - Y[8] : Y[q];
+    row[q] = (q == r) ? 1.0 + y : y;
   }
-  const bool ok = PIVOT ? solve_pivot(M, y) : solve_nopivot(M, y);
+}
+__device__ __forceinline__ void assemble_jacobian8(const double* Fe, const double* A, const double* c, double dt,
+                                                   double* J, const MatConst& mc) {
+  JacobianParts<true> jp;
+  jacobian_parts(Fe, A, c, dt, jp, mc);
 #pragma unroll
-  for (int r = 0; r < 8; ++r)
-#pragma unroll
-    for (int j = 0; j < NW; ++j) b[r] -= U[j][r] * y[j];
-  b[8] = -(b[0] + b[4]);
-  // Where the rates are stiff (an overshot iterate), b and sum U y agree in
-  // many digits and x keeps a rounding error of the size of b's, which J
-  // multiplies.  J acts on the five numbers w(x) only, and those are known
-  // without cancellation: y_i / kappa_i.  The symmetric traceless matrix that
-  // has the difference for its five numbers (G taken as the identity) removes
-  // it to within |G - I|.  Without it 871 instead of 162 of the 4096 points of
-  // 2 % strain steps take other iteration counts than with a pivoted 9x9 LU.
-  double e[NW];
-  newton_w(G, b, e);
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    if constexpr (GENERAL) {
-      const double k = mc.v * (i < 2 ? mc.C11 - mc.C12 : mc.C44);
-      e[i] = k != 0.0 ? y[i] / k - e[i] : 0.0;
-    } else {
-      e[i] = i < 2 ? mc.newton_d * y[i] - e[i] : y[i] - e[i];
-    }
-  }
-  const double tr = (e[0] + e[1]) * (-1.0 / 3.0);
-  b[0] += e[0] + tr;
-  b[4] += e[1] + tr;
-  b[1] += 0.5 * e[2];
-  b[3] += 0.5 * e[2];
-  b[2] += 0.5 * e[3];
-  b[6] += 0.5 * e[3];
-  b[5] += 0.5 * e[4];
-  b[7] += 0.5 * e[4];
-  b[8] = -(b[0] + b[4]);
-  return ok;
+  for (int r = 0; r < NR; ++r) jacobian_row(jp, r, J + NR * r, mc);
 }
 
-// Column-major plane q = i+3j of a (3,3) field <-> row-major register 3*i+j
-__device__ __forceinline__ int rm(int q) { return 3 * (q % 3) + q / 3; }
-
-__device__ __forceinline__ void load33(const double* base, int64_t N, int64_t c, double* m) {
+// The Newton system assembled and solved by LU without row exchanges, one row
+// at a time: row i is eliminated by the factor rows 0..i-1 as soon as it is
+// formed (the same operations on every entry, in the same order, as the
+// column-by-column elimination), so only the factor rows are held.  Refuses
+// (returns false; b then holds no meaning) when a multiplier exceeds 1e6 in
+// magnitude or a pivot's magnitude is below 2^-1000 (zero and NaN included:
+// the pivot's reciprocal is the refined hardware one, so a pivot near the
+// bottom of the range goes to the pivoted pass and its exact division; the
+// pivots of this system, 1 plus rate terms, are never near the top of the
+// range): multipliers up to 1e6 cost at most a few of
+// the 16 digits of the Newton step, far below the Newton tolerance, and the
+// residual test of the next iteration uses the exact residual; only steeper
+// cases (about 1 % of points had pivots below 1/100 of their column in the
+// 128^3 tension case) need the pivoted pass.
+__device__ __forceinline__ bool assemble_solve8_nopivot(const double* Fe, const double* A, const double* c,
+                                                        double dt, double* b, const MatConst& mc) {
+  JacobianParts<false> jp;
+  jacobian_parts(Fe, A, c, dt, jp, mc);
+  double U[NR * NR];  // factor rows (upper part), reciprocal pivots on the diagonal
+  // refusals are collected and tested once at the end (what is computed
+  // after one is discarded): no branches inside the unrolled elimination, and
+  // the multipliers' magnitudes enter one running maximum (a NaN multiplier
+  // is ignored by the maximum, as by the comparison it replaces)
+  bool refused = false;
+  double lmax = 0.0;
 #pragma unroll
-  for (int q = 0; q < 9; ++q) m[rm(q)] = base[q * N + c];
-}
-
-// Plane addressing by a uniform plane pointer plus the lane's 32-bit byte
-// offset (scalar base + vector offset): one offset register serves every
-// plane, instead of a 64-bit lane address per plane.  Needs (c_end) * 8 < 2^32,
-// which the launcher checks.
-//
-// Every plane pointer given to ld/st/load33/store33 with a Lane must be the
-// same in all lanes (formed from kernel arguments and uniform indices only):
-// it is read from the first active lane, which keeps the compiler from
-// folding the lane offset into a 64-bit per-lane address for every plane.
-// A per-lane choice between two planes is made on the loaded values
-// (load33_sel), never on the pointer.
-struct Lane {
-  uint32_t off;  // cell index * 8
-};
-__device__ __forceinline__ uint64_t uniform_u64(uint64_t v) {
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return ((uint64_t)hi << 32) | lo;
-}
-typedef __attribute__((address_space(1))) double gdouble;  // global memory
-__device__ __forceinline__ double ld(const double* plane, Lane l) {
-  return *reinterpret_cast<const gdouble*>(uniform_u64(reinterpret_cast<uint64_t>(plane)) + l.off);
-}
-__device__ __forceinline__ void st(double* plane, Lane l, double v) {
-  *reinterpret_cast<gdouble*>(uniform_u64(reinterpret_cast<uint64_t>(plane)) + l.off) = v;
-}
-// The plane stride as a value of this place only: pointers formed from it are
-// formed here (two scalar adds a plane).  From the plain N the compiler forms
-// the pointers of every access once at the kernel's entry, keeps them in
-// vector lanes (it has no scalar registers for 150 of them) and reads each
-// back at its use: 630 instructions of the 12000 that a wave executes.
-__device__ __forceinline__ int64_t stride_here(int64_t N) {
-  asm volatile("" : "+s"(N));
-  return N;
-}
-__device__ __forceinline__ void load33(const double* base, int64_t N, Lane l, double* m) {
-  const int64_t n = stride_here(N);
+  for (int i = 0; i < NR; ++i) {
+    double row[NR];
+    jacobian_row(jp, i, row, mc);
 #pragma unroll
-  for (int q = 0; q < 9; ++q) m[rm(q)] = ld(base + q * n, l);
-}
-__device__ __forceinline__ void store33(double* base, int64_t N, Lane l, const double* m) {
-  const int64_t n = stride_here(N);
+    for (int k = 0; k < i; ++k) {
+      const double l = row[k] * U[NR * k + k];
+      lmax = fmax(lmax, fabs(l));
 #pragma unroll
-  for (int q = 0; q < 9; ++q) st(base + q * n, l, m[rm(q)]);
-}
-// load from a plane chosen per lane (the base may differ between lanes): a
-// 64-bit lane address and one unconditional load, so that the loads of all
-// lanes and planes issue together instead of in divergent branches
-__device__ __forceinline__ double ldv(const double* plane, Lane l) {
-  return *reinterpret_cast<const gdouble*>(reinterpret_cast<uint64_t>(plane) + l.off);
-}
-// per-lane choice of the plane set: sel ? a : b
-__device__ __forceinline__ void load33_sel(bool sel, const double* a, const double* b, int64_t N, Lane l,
-                                           double* m) {
-  const double* base = sel ? a : b;
-  const int64_t n = stride_here(N);
+      for (int c2 = k + 1; c2 < NR; ++c2) row[c2] -= l * U[NR * k + c2];
+      b[i] -= l * b[k];
+    }
+    const double piv = row[i];
+    refused = refused || !(fabs(piv) >= 0x1p-1000);
+    U[NR * i + i] = rcp_refined(piv);
 #pragma unroll
-  for (int q = 0; q < 9; ++q) m[rm(q)] = ldv(base + q * n, l);
+    for (int c2 = i + 1; c2 < NR; ++c2) U[NR * i + c2] = row[c2];
+  }
+#pragma unroll
+  for (int i = NR - 1; i >= 0; --i) {
+    double s = b[i];
+#pragma unroll
+    for (int c2 = i + 1; c2 < NR; ++c2) s -= U[NR * i + c2] * b[c2];
+    b[i] = s * U[NR * i + i];
+  }
+  return !(refused || lmax > 1e6);
 }
 
 // Per-point output / scratch addressing
@@ -660,42 +319,21 @@ struct PointIO {
   Lane l;
 };
 
-// Elastic deformation and constitutive velocity gradient at Lp: Fe = A (I -
-// dt Lp), pm (slip_powers) and Lpc = v gdot0 sum_s sign_s x_s^n d_s n_s^T
-template <int NE4>
-__device__ __forceinline__ void lp_constitutive(const double* A, double dt, const double* Lp, const double* rxi,
-                                                double* Fe, double* pm, double* Lpc, const MatConst& mc) {
-  double B[9], Sl[9];
-#pragma unroll
-  for (int k = 0; k < 9; ++k) B[k] = (k % 4 == 0 ? 1.0 : 0.0) - dt * Lp[k];
-  mm33(A, B, Fe);  // Fe = A B invFi_new, invFi_new = I
-  hooke_S(Fe, Sl, mc);
-  double tau[NSLIP], g[NSLIP];
-  resolved_shears(Sl, mc.v, tau);
-  slip_powers<NE4, true>(tau, rxi, g, pm, mc);
-#pragma unroll
-  for (int s = 0; s < NSLIP; ++s) g[s] = copysign(g[s], tau[s]);
-  slip_sum(g, mc.newton_vg, Lpc);
-}
-
-// integrateStress (phase_mechanical.f90:380-604); returns 0 (integrated) or
-// 1 (broken).  Takes the reciprocal slip resistances of the state and updates
-// S and Lp in registers; Fe, P and Fp of the integration the state loop keeps
-// are formed and stored by store_integrated.
+// integrateStress (phase_mechanical.f90:380-604); returns 0 (integrated),
+// 1 (broken) or, without PIVOT, 2 when the LU without row exchanges refused a
+// pivot (the point is then redone by the PIVOT instantiation, which solves
+// every Newton system with partial pivoting).  Takes the reciprocal slip
+// resistances of the state and updates S and Lp in registers; Fe, P and Fp
+// of the integration the state loop keeps are formed and stored by
+// store_integrated.
 //
 // A = F invFp0 of the (sub)step and invFp0 (both in LDS, lane t) are formed
 // once per substep by the caller: they do not change during the state fixed
 // point.
-//
-// A Newton system whose LU without row exchanges is refused (a steep or
-// singular one) is formed again and solved with partial pivoting, as LAPACK's
-// dgesv in the reference: a branch that a wave takes only when one of its
-// lanes does.
-template <int NE4>
+template <int NE4, bool PIVOT>
 __device__ __forceinline__ int integrate_stress(const double (*hA)[64], const double (*invFp0)[64], int t, double dt,
                                                 const double* rxi, double* Lp, double* S, int& newton,
                                                 const MatConst& mc) {
-  constexpr bool GENERAL = NE4 < 0;
   // A is read from LDS where it is used, not hoisted into the registers the
   // Newton system needs: the lane index passes through an empty asm, so every
   // call's nine ds_reads are new loads (issued together, one wait), not the
@@ -721,9 +359,19 @@ __device__ __forceinline__ int integrate_stress(const double (*hA)[64], const do
   for (;;) {
     it++;
     if (it > mc.N_iter_Lp_max) return 1;
-    double A[9], Fe[9], pm[NSLIP], res[9];
-    loadA(A);
-    lp_constitutive<NE4>(A, dt, Lp, rxi, Fe, pm, res, mc);
+    double Fe[9], Sl[9];
+    {
+      double B[9], A[9];
+#pragma unroll
+      for (int k = 0; k < 9; ++k) B[k] = (k % 4 == 0 ? 1.0 : 0.0) - dt * Lp[k];
+      loadA(A);
+      mm33(A, B, Fe);  // Fe = A B invFi_new, invFi_new = I
+    }
+    hooke_S(Fe, Sl, mc);
+    double dg[NSLIP], c[NSLIP];
+    kinetics<NE4>(Sl, rxi, dg, c, mc);
+    double res[9];
+    slip_sum(dg, mc.v, res);
     // res holds Lp_constitutive here
     double n2Lpc = 0.0, n2Lp = 0.0, n2res = 0.0;
 #pragma unroll
@@ -752,15 +400,18 @@ __device__ __forceinline__ int integrate_stress(const double (*hA)[64], const do
         continue;
       }
     }
-    if (!newton_step<GENERAL, false>(Fe, A, pm, dt, res, mc)) {
-      // formed again from Lp (the same values: the same operations), so that
-      // nothing is held for this rare branch
+    {
+      double J[NR * NR], A[9];
       loadA(A);
-      lp_constitutive<NE4>(A, dt, Lp, rxi, Fe, pm, res, mc);
-#pragma unroll
-      for (int k = 0; k < 9; ++k) res[k] = Lp[k] - res[k];
-      if (!newton_step<GENERAL, true>(Fe, A, pm, dt, res, mc)) return 1;  // singular
+      if constexpr (PIVOT) {
+        assemble_jacobian8(Fe, A, c, dt, J, mc);
+        if (!solve8_pivot(J, res)) return 1;  // singular
+      } else {
+        // the point is redone by the pivoting pass
+        if (!assemble_solve8_nopivot(Fe, A, c, dt, res, mc)) return 2;
+      }
     }
+    res[8] = -(res[0] + res[4]);  // x_22 of the traceless solution
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
       dLp[k] = -res[k];
@@ -829,10 +480,18 @@ __device__ __forceinline__ void store_integrated(const double (*hA)[64], const d
 
 }  // namespace
 
-// Substep scratch layout (per point, planes of N doubles): F0 (9), Lp0 (9),
-// Fp0 (9), state0 (24) of the current substep start, and F of the substep
-// being integrated (9).  Touched only when the first full step was cut back.
-constexpr int SUB_F0 = 0, SUB_LP0 = 9, SUB_FP0 = 18, SUB_ST0 = 27, SUB_FLOC = 51, SUB_PLANES = 60;
+// One residual evaluation's material-point loop, in two passes.  The first
+// (mp_response_kernel) carries no pivoted factorisation, so that its
+// registers serve the common path only; a point whose Newton system the LU
+// without row exchanges refuses leaves its loops, stores no output and is
+// appended to the repivot list (its inputs are unchanged: Lp, the only plane
+// that is both read and written, is stored last).  The second
+// (mp_repivot_kernel) redoes exactly the listed points from the same inputs,
+// every Newton system of them solved with partial pivoting (as LAPACK's
+// dgesv in the reference), in a grid-stride loop over the list.  Points are
+// independent, so the list order does not change any result.
+//
+// repivot: [0] = number of listed points, [1 + i] = cell index.
 
 // per-lane LDS columns of one 64-lane block: FPI history
 // (dotState_last(:,1), its difference to dotState_last(:,2)) and the
@@ -846,7 +505,7 @@ struct MpLds {
   double A[9][64];     // F_(sub)step invFp0
 };
 
-template <int NE4, int AE4>
+template <int NE4, int AE4, bool PIVOT>
 __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, MpLds& sh) {
   const MatConst& mc = a.mc;
   const MpState& s = a.s;
@@ -896,6 +555,7 @@ __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, M
   };
   double stepFrac = 0.0, step = 1.0 / mc.r_cutback;
   bool converged = false, todo = true;
+  bool refused = false;  // first pass only: the Newton system needs row exchanges
   double fp0v[9];        // Fp0 of the (sub)step about to be integrated (planes in order)
   // step control: the next substep after a converged one, else a cut-back
   // step from the restored start values; sets todo
@@ -949,15 +609,23 @@ __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, M
         xi[k] = stl[k];
         h_gam[k][t] = stl[NSLIP + k];
       }
-#pragma unroll
-      for (int k = 0; k < 9; ++k) st(s.Fp + (k) * n, l, fp0v[k]);  // after the loads, as above
       todo = step > mc.r_cutback_min;
+      // the restored Fp is stored only by a point that leaves with it: an
+      // integrated one stores its own
+      if (!todo) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) st(s.Fp + (k) * n, l, fp0v[k]);
+      }
     }
   };
-  // the first call restores the increment's start values; it follows the
-  // entry loads directly, so that its loads and theirs share one round trip
-  control();
-  while (todo) {
+  // first pass: the first call restores the increment's start values; it
+  // follows the entry loads directly, so that its loads and theirs share one
+  // round trip.  The pivoting pass (a few points per launch, registers
+  // tighter) keeps the control at the top of the loop.
+  if constexpr (!PIVOT) control();
+  for (;;) {
+    if constexpr (PIVOT) control();
+    if (!todo) break;
     {
       // A = F_(sub)step invFp0 and invFp0 are fixed during the state fixed
       // point (integrateStress, phase_mechanical.f90:425-432)
@@ -1020,7 +688,10 @@ __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, M
           }
 #pragma unroll
           for (int k = 0; k < NSLIP; ++k) rxi[k] = rcp_refined(xi[k]);
-          broken = fp0_singular || integrate_stress<NE4>(sh.A, sh.iFp0, t, sdt, rxi, Lp, S, newton, mc) != 0;
+          const int rc =
+              fp0_singular ? 1 : integrate_stress<NE4, PIVOT>(sh.A, sh.iFp0, t, sdt, rxi, Lp, S, newton, mc);
+          refused = rc == 2;
+          broken = rc != 0;
           if (broken) break;
           {
             double stt[NSTATE];
@@ -1086,8 +757,16 @@ __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, M
         }
       }
       converged = !broken;
+      if (refused) break;  // the pivoting pass redoes this point from its inputs
     }
-    control();
+    if constexpr (!PIVOT) control();
+  }
+  if constexpr (!PIVOT) {
+    if (refused) {
+      const int slot = atomicAdd(s.repivot, 1);
+      s.repivot[1 + slot] = (int)c;
+      return;
+    }
   }
   store33(s.Lp, N, l, Lp);
   store33(s.S, N, l, S);
@@ -1104,20 +783,30 @@ __device__ __forceinline__ void mp_point(const KernelArgs& a, const int64_t c, M
     s.iters[c] = newton;
     s.iters[N + c] = fpi;
   }
-  if (a.broken) a.broken[c] = converged ? 0 : 1;
-  if (!converged && a.ill) atomicOr(a.ill, 1);
+  if (!converged) atomicOr(a.ill, 1);
 }
 
 template <int NE4, int AE4>
 __global__ void __launch_bounds__(64) mp_response_kernel(KernelArgs a) {
   __shared__ MpLds sh;
-  const int64_t c = a.c_begin + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= a.c_end) return;
-  mp_point<NE4, AE4>(a, c, sh);
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= a.s.N) return;
+  mp_point<NE4, AE4, false>(a, c, sh);
 }
 
-// clears the terminally-ill flag of one response
-__global__ void ill_reset_kernel(int* ill) { *ill = 0; }
+template <int NE4, int AE4>
+__global__ void __launch_bounds__(64) mp_repivot_kernel(KernelArgs a) {
+  __shared__ MpLds sh;
+  const int64_t cnt = a.s.repivot[0];  // complete: the first pass ran before this launch
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += (int64_t)gridDim.x * blockDim.x)
+    mp_point<NE4, AE4, true>(a, a.s.repivot[1 + i], sh);
+}
+
+// clears the repivot list and the terminally-ill flag of one response
+__global__ void repivot_reset_kernel(int* repivot, int* ill) {
+  repivot[0] = 0;
+  *ill = 0;
+}
 
 // ---- many RVEs in one launch ---------------------------------------------------
 // The material-point updates of a batch of RVEs (each with its own planes,
@@ -1155,14 +844,27 @@ __global__ void __launch_bounds__(64) mp_response_batch_kernel(const KernelArgs*
   __shared__ MpLds sh;
   const int r = batch_entry(blk_off, n, blockIdx.x);
   const KernelArgs a = load_args(tab + r);
-  const int64_t c = a.c_begin + (int64_t)(blockIdx.x - (unsigned)blk_off[r]) * 64 + threadIdx.x;
-  if (c >= a.c_end) return;
-  mp_point<NE4, AE4>(a, c, sh);
+  const int64_t c = (int64_t)(blockIdx.x - (unsigned)blk_off[r]) * 64 + threadIdx.x;
+  if (c >= a.s.N) return;
+  mp_point<NE4, AE4, false>(a, c, sh);
 }
 
-__global__ void ill_reset_batch_kernel(const KernelArgs* __restrict__ tab, int n) {
+// pivoting pass of a batch: blockIdx.y is the RVE, blockIdx.x strides over
+// its list as mp_repivot_kernel does
+template <int NE4, int AE4>
+__global__ void __launch_bounds__(64) mp_repivot_batch_kernel(const KernelArgs* __restrict__ tab) {
+  __shared__ MpLds sh;
+  const KernelArgs a = load_args(tab + blockIdx.y);
+  const int64_t cnt = a.s.repivot[0];
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += (int64_t)gridDim.x * blockDim.x)
+    mp_point<NE4, AE4, true>(a, a.s.repivot[1 + i], sh);
+}
+
+__global__ void repivot_reset_batch_kernel(const KernelArgs* __restrict__ tab, int n) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < n) *tab[r].ill = 0;
+  if (r >= n) return;
+  tab[r].s.repivot[0] = 0;
+  *tab[r].ill = 0;
 }
 
 
@@ -1235,7 +937,7 @@ struct TangentArgs {
   MpState s;
   MatConst mc;
   double dt;
-  double* dPdF;  // MODE 0: 81 planes of N (plane k+3l+9p+27o); MODE 2: 81 values per listed cell
+  double* dPdF;  // MODE 2: 81 values per listed cell (k+3l+9p+27o)
   double* n2;    // MODE 1: per cell |dPdF|^2 (the 81 squares summed in the order they are formed)
   double* bpart; // MODE 1: per 16 cells the sums of the 81 planes, at plane * nblk + 4 * block + row
   int64_t nblk;  // MODE 1: 4 x the blocks of 64 cells
@@ -1243,18 +945,6 @@ struct TangentArgs {
   int64_t c_begin, c_end;  // cells [c_begin, c_end); MODE 2: c_end - c_begin listed cells (at most 64)
 };
 
-// (C : X)(i,j) = sum_kl C(i,j,k,l) X(k,l) for the cubic stiffness
-// (math_Voigt66to3333_stiffness of C11, C12, C44): C11 X_ii + C12 sum_{k!=i}
-// X_kk on the diagonal, C44 (X_ij + X_ji) off it (row-major 3x3)
-__device__ __forceinline__ void cubic_contract(const double* X, double* Y, const MatConst& mc) {
-  const double t = X[0] + X[4] + X[8];
-  const double d = mc.C11 - mc.C12;
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-      Y[3 * i + j] = (i == j) ? mc.C12 * t + d * X[4 * i] : mc.C44 * (X[3 * i + j] + X[3 * j + i]);
-}
 }  // namespace
 
 // x[j] += x[j] of the lane DPP control CTRL selects, for nine doubles (the
@@ -1272,8 +962,7 @@ __device__ __forceinline__ void dpp_step(double* x) {
 }
 
 // NE4: the slip-rate exponent n_sl as a compile-time quarter (-1: runtime).
-// MODE 0: dPdF of every cell into 81 planes.  MODE 1 (the solver's
-// C_volAvg and C_minMaxAvg): no dPdF field, only each cell's |dPdF|^2 and
+// MODE 1 (the solver's C_volAvg and C_minMaxAvg): no dPdF field, only each cell's |dPdF|^2 and
 // per 16-cell row of a block the sums of the 81 planes, in a fixed order.
 // MODE 2:
 // dPdF of up to 64 listed cells (one block), e.g. the two extreme cells
@@ -1292,13 +981,9 @@ __global__ void __launch_bounds__(64) mp_tangent_kernel(TangentArgs a) {
   } else {
     c = a.c_begin + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     live = c < a.c_end;
-    if constexpr (MODE == 0) {
-      if (!live) return;
-    } else {
-      // the whole wave takes part in the block sums: a lane past the end
-      // computes the last cell again and contributes nothing
-      if (!live) c = a.c_end - 1;
-    }
+    // the whole wave takes part in the block sums: a lane past the end
+    // computes the last cell again and contributes nothing
+    if (!live) c = a.c_end - 1;
   }
   [[maybe_unused]] double n2acc = 0.0;
   const double dt = a.dt;
@@ -1319,13 +1004,10 @@ __global__ void __launch_bounds__(64) mp_tangent_kernel(TangentArgs a) {
 #pragma unroll
     for (int k = 0; k < 9; ++k) invFp0[k] = 0.0;
   }
-  double tau[NSLIP], dg[NSLIP], cs[NSLIP], rxi[NSLIP];
+  double dg[NSLIP], cs[NSLIP], rxi[NSLIP];
 #pragma unroll
   for (int k = 0; k < NSLIP; ++k) rxi[k] = 1.0 / xi[k];
-  resolved_shears(S, mc.v, tau);
-  slip_powers<NE4, true>(tau, rxi, dg, cs, mc);
-#pragma unroll
-  for (int k = 0; k < NSLIP; ++k) cs[k] = mc.gdot0 * mc.n * cs[k];
+  kinetics<NE4>(S, rxi, dg, cs, mc);
 
   // L = I + dt sum_s c_s vec(U_s) vec(P_s)^T, U_s = C : (H P_s), H = Fe^T F invFp0
   double T2[9], H[9];
@@ -1482,9 +1164,7 @@ __global__ void __launch_bounds__(64) mp_tangent_kernel(TangentArgs a) {
           v = v + a1[3 * k + l] + a2[3 * k + l] + a3[3 * k + l];
           // plane index of dPdF(k,l,p,o): k + 3l + 9p + 27o
           const int q = k + 3 * l + 9 * p + 27 * o;
-          if constexpr (MODE == 0) {
-            a.dPdF[(int64_t)q * N + c] = v;
-          } else if constexpr (MODE == 2) {
+          if constexpr (MODE == 2) {
             a.dPdF[81 * threadIdx.x + q] = v;
           } else {
             n2acc += v * v;
@@ -1598,25 +1278,26 @@ __global__ void mp_init_kernel(MpState s, const double* Fp_init, double xi_0) {
 int mp_partial_blocks(int64_t N) { return (int)((N + PAV_CELLS - 1) / PAV_CELLS); }
 int mp_sub_planes() { return SUB_PLANES; }
 
-// The exponents of the example material (n_sl = 20, a_sl = 2.25) are compiled
-// in, with the Newton system divided by its stiffness scales, which must not
-// vanish; any other material runs the runtime-exponent instantiation.
-static bool example_class(const MatConst& mc) {
-  return mc.n_e4 == 80 && mc.a_e4 == 9 && std::isfinite(mc.newton_d) && mc.newton_d != 0.0;
-}
-
-void launch_mp_response(const MpState& s, const MatConst& mc, double dt, int* d_ill, double* d_sub, hipStream_t st,
-                        int* d_broken, int64_t c_begin, int64_t c_end) {
-  if (c_end < 0) c_end = s.N;
-  if (c_begin < 0 || c_end > s.N || c_begin > c_end) throw std::runtime_error("material-point range out of bounds");
-  if (c_begin == c_end) return;
+void launch_mp_response(const MpState& s, const MatConst& mc, double dt, int* d_ill, double* d_sub, hipStream_t st) {
+  if (s.N < 1) return;
   // lanes address planes by a 32-bit byte offset (cell index * 8)
   if (s.N > ((int64_t)1 << 29)) throw std::runtime_error("material-point planes longer than 2^29 cells");
-  KernelArgs a{s, mc, dt, d_ill, d_broken, d_sub, c_begin, c_end};
-  const int blocks = (int)((c_end - c_begin + 63) / 64);
-  if (d_ill) hipLaunchKernelGGL(ill_reset_kernel, dim3(1), dim3(1), 0, st, d_ill);
-  if (example_class(mc)) hipLaunchKernelGGL((mp_response_kernel<80, 9>), dim3(blocks), dim3(64), 0, st, a);
-  else hipLaunchKernelGGL((mp_response_kernel<-1, -1>), dim3(blocks), dim3(64), 0, st, a);
+  if (!s.repivot) throw std::runtime_error("material-point state without the repivot plane");
+  const KernelArgs a{s, mc, dt, d_ill, d_sub};
+  const int blocks = (int)((s.N + 63) / 64);
+  // exponents of the example material (n_sl = 20, a_sl = 2.25) are compiled
+  // in; any other material runs the runtime-exponent instantiation
+  // second pass: a fixed grid striding over the list (it holds at most the
+  // range's points)
+  const int blocks2 = std::min(blocks, 1024);
+  hipLaunchKernelGGL(repivot_reset_kernel, dim3(1), dim3(1), 0, st, s.repivot, d_ill);
+  if (mc.n_e4 == 80 && mc.a_e4 == 9) {
+    hipLaunchKernelGGL((mp_response_kernel<80, 9>), dim3(blocks), dim3(64), 0, st, a);
+    hipLaunchKernelGGL((mp_repivot_kernel<80, 9>), dim3(blocks2), dim3(64), 0, st, a);
+  } else {
+    hipLaunchKernelGGL((mp_response_kernel<-1, -1>), dim3(blocks), dim3(64), 0, st, a);
+    hipLaunchKernelGGL((mp_repivot_kernel<-1, -1>), dim3(blocks2), dim3(64), 0, st, a);
+  }
   SCA_HIP(hipGetLastError());
 }
 
@@ -1632,32 +1313,34 @@ void launch_mp_response_batch(const MpBatchItem* items, int n, TableArena& ta, h
   int* off = ta.add<int>(n + 2, &doff);
   MpBatchPav* pv = ta.add<MpBatchPav>(n, &dpv);
   int* pvoff = ta.add<int>(n + 1, &dpvoff);
-  auto cls = [](const MatConst& mc) { return example_class(mc) ? 0 : 1; };
+  auto cls = [](const MatConst& mc) { return (mc.n_e4 == 80 && mc.a_e4 == 9) ? 0 : 1; };
   int n0 = 0;
   for (int i = 0; i < n; ++i) n0 += cls(items[i].mc) == 0 ? 1 : 0;
   int k0 = 0, k1 = n0;
+  int64_t maxN = 0;
   for (int i = 0; i < n; ++i) {
     const MpBatchItem& it = items[i];
     const MpState& s = it.s;
     if (s.N > ((int64_t)1 << 29)) throw std::runtime_error("material-point planes longer than 2^29 cells");
-    if (!it.ill || !it.sub) throw std::runtime_error("incomplete batch item");
+    if (!s.repivot || !it.ill || !it.sub) throw std::runtime_error("incomplete batch item");
     const int e = cls(it.mc) == 0 ? k0++ : k1++;
-    ka[e] = KernelArgs{s, it.mc, it.dt, it.ill, nullptr, it.sub, 0, s.N};
+    ka[e] = KernelArgs{s, it.mc, it.dt, it.ill, it.sub};
     // no pav_partial: the P sums come from elsewhere (no blocks)
     pv[e] = MpBatchPav{s.P, s.N, it.pav_partial, it.pav_partial ? mp_partial_blocks(s.N) : 0};
+    maxN = std::max(maxN, s.N);
   }
   // block offsets: class 0 in off[0..n0], class 1 in off[n0+1..n+1]
   int64_t tot = 0;
   off[0] = 0;
   for (int i = 0; i < n0; ++i) {
-    tot += (ka[i].c_end + 63) / 64;
+    tot += (ka[i].s.N + 63) / 64;
     off[i + 1] = (int)tot;
   }
   const int64_t blocks0 = tot;
   tot = 0;
   off[n0 + 1] = 0;
   for (int i = n0; i < n; ++i) {
-    tot += (ka[i].c_end + 63) / 64;
+    tot += (ka[i].s.N + 63) / 64;
     off[i + 2] = (int)tot;
   }
   const int64_t blocks1 = tot;
@@ -1673,12 +1356,18 @@ void launch_mp_response_batch(const MpBatchItem* items, int n, TableArena& ta, h
   ta.upload(off, n + 2, st);
   ta.upload(pv, n, st);
   ta.upload(pvoff, n + 1, st);
-  hipLaunchKernelGGL(ill_reset_batch_kernel, dim3((n + 63) / 64), dim3(64), 0, st, dka, n);
-  if (n0 > 0)
+  hipLaunchKernelGGL(repivot_reset_batch_kernel, dim3((n + 63) / 64), dim3(64), 0, st, dka, n);
+  // pivoting pass: enough lanes per RVE for its list (about 1 % of its points)
+  const int x2 = (int)std::min<int64_t>(1024, std::max<int64_t>(16, (maxN + 1023) / 1024));
+  if (n0 > 0) {
     hipLaunchKernelGGL((mp_response_batch_kernel<80, 9>), dim3((unsigned)blocks0), dim3(64), 0, st, dka, doff, n0);
-  if (n > n0)
+    hipLaunchKernelGGL((mp_repivot_batch_kernel<80, 9>), dim3(x2, n0), dim3(64), 0, st, dka);
+  }
+  if (n > n0) {
     hipLaunchKernelGGL((mp_response_batch_kernel<-1, -1>), dim3((unsigned)blocks1), dim3(64), 0, st, dka + n0,
                        doff + n0 + 1, n - n0);
+    hipLaunchKernelGGL((mp_repivot_batch_kernel<-1, -1>), dim3(x2, n - n0), dim3(64), 0, st, dka + n0);
+  }
   if (pav_blocks > 0)
     hipLaunchKernelGGL(pav_partial_batch_kernel, dim3((unsigned)pav_blocks), dim3(256), 0, st, dpv, dpvoff, n);
   SCA_HIP(hipGetLastError());
@@ -1698,24 +1387,6 @@ static void launch_tangent_mode(const TangentArgs& a, int64_t blocks, hipStream_
   if (a.mc.n_e4 == 80) hipLaunchKernelGGL((mp_tangent_kernel<80, MODE>), dim3((unsigned)blocks), dim3(64), 0, st, a);
   else hipLaunchKernelGGL((mp_tangent_kernel<-1, MODE>), dim3((unsigned)blocks), dim3(64), 0, st, a);
   SCA_HIP(hipGetLastError());
-}
-
-void launch_mp_tangent(const MpState& s, const MatConst& mc, double dt, double* dPdF, hipStream_t st,
-                       int64_t c_begin, int64_t c_end) {
-  if (c_end < 0) c_end = s.N;
-  if (c_begin < 0 || c_end > s.N || c_begin > c_end) throw std::runtime_error("material-point range out of bounds");
-  if (c_begin == c_end) return;
-  TangentArgs a;
-  a.s = s;
-  a.mc = mc;
-  a.dt = dt;
-  a.dPdF = dPdF;
-  a.c_begin = c_begin;
-  a.c_end = c_end;
-  a.n2 = a.bpart = nullptr;
-  a.nblk = 0;
-  a.cells = nullptr;
-  launch_tangent_mode<0>(a, (c_end - c_begin + 63) / 64, st);
 }
 
 int64_t tangent_blocks(int64_t N) { return (N + 63) / 64; }

@@ -26,6 +26,7 @@ void build_matconst(const sc_material& m, const sc_phase_numerics& p, MatConst& 
   o.v = (1.0 / std::sqrt(2.0)) * (1.0 / std::sqrt(3.0));
   for (int i = 0; i < 7; ++i) o.hv[i] = m.h_sl_sl[i];
   o.xi_inf = m.xi_inf_sl;
+  o.rxi_inf = 1.0 / m.xi_inf_sl;
   o.h0 = m.h_0_sl_sl;
   o.n = m.n_sl;
   o.a = m.a_sl;
@@ -44,8 +45,8 @@ void build_matconst(const sc_material& m, const sc_phase_numerics& p, MatConst& 
   o.n_e4 = quarter(m.n_sl);
   o.a_e4 = quarter(m.a_sl);
   o.newton_vg = o.v * o.gdot0;
-  o.newton_f = o.newton_vg * o.n;
-  o.newton_fA = o.newton_f * (o.v * o.C44);
+  o.newton_f = o.v * o.newton_vg * o.n;
+  o.newton_fA = o.newton_f * o.C44;
   o.newton_d = o.C44 / (o.C11 - o.C12);
 }
 

@@ -1,7 +1,7 @@
 // Material-point update on caller-owned device planes without any device
 // allocation (sc_mp_update_noalloc).
 //
-// The kernels are those of sc_mp_update (launch_mp_response, launch_mp_tangent).
+// The kernels are those of sc_mp_update (launch_mp_points, launch_mp_tangent).
 // The device memory they need beyond the caller's inputs and outputs -- the
 // substep scratch planes -- lives in `scratch`, one fixed array per GPU that the
 // code object carries.  In host code `scratch` names a host-side stand-in, not
@@ -88,7 +88,7 @@ extern "C" int sc_mp_update_noalloc(int64_t n, double dt, const sc_material* m, 
     s.gamma = pl->gamma;
     s.iters = pl->iterations;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    launch_mp_response(s, mc, dt, nullptr, base, st, pl->broken);
+    launch_mp_points(s, mc, dt, nullptr, base, st, pl->broken);
     if (pl->dPdF) launch_mp_tangent(s, mc, dt, pl->dPdF, st);
     return 0;
   } catch (std::exception& e) {

@@ -1,0 +1,1009 @@
+// Point updates of callers that bring their own solver (sc_mp_update,
+// sc_mp_update_noalloc, the drop-in boundary): the physics and the stopping
+// rules of the grid solver's kernels (constitutive.hip, where the references to
+// the reference's code are), with the Newton system solved as a 5x5 instead of
+// an 8x8 one, the consistent tangent likewise, and fewer operations in the
+// rates.  Results equal the solver's kernels' to rounding.  They are not used
+// by the grid solver: its N-GMRES iteration amplifies a rounding difference of
+// the stress (1e-16 to 1e-11 of P in double precision, to 2e-7 where the
+// spectral stages are in single), and a load case, its checkpoints and its
+// restarts keep their bits.
+//
+// Bound: one lane per point and one wave per SIMD (456 of 512 registers), so a
+// call of up to 65536 points is one wave's chain of dependent operations, and
+// part of that is fetching its instructions: the code is kept short (one copy
+// of the rate evaluation, no second pass).  60 points: 45 -> 32 us a call;
+// 32768 points 56 -> 41 us; with the tangent, 4097 points 74 -> 50 us.
+#include <cmath>
+
+#include "mp_device.h"
+
+namespace sca {
+namespace {
+
+// Material constants travel in the kernel arguments (not a __constant__
+// symbol) so that launches of different contexts on concurrent streams never
+// share them.
+struct KernelArgs {
+  MpState s;
+  MatConst mc;
+  double dt;
+  int* ill;     // may be null
+  int* broken;  // per point, may be null
+  double* sub;  // substep scratch, SUB_PLANES planes of N doubles
+  int64_t c_begin, c_end;  // cells [c_begin, c_end) of the N-cell planes
+};
+// The arguments are read through the constant address space (invariant, into
+// scalar registers).  here() makes the pointer a value of its place: the plane
+// pointers read through it are loaded there, not kept from the kernel's entry
+// on (they and the material constants are more than the scalar registers).
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(4))) const KernelArgs ConstArgs;
+#else
+typedef const KernelArgs ConstArgs;
+#endif
+__device__ __forceinline__ ConstArgs* here(ConstArgs* p) {
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
+// 1/x as the hardware reciprocal r (within 2^-24) corrected once by
+// r (e + e^2), e = 1 - x r (to e^3)
+__device__ __forceinline__ double rcp_cubic(double x) {
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = __builtin_fma(-x, r, 1.0);
+  return __builtin_fma(r, __builtin_fma(e, e, e), r);
+}
+// x^(9/4) for x >= 0, from x^(-1/4): a start value from the hardware square
+// root and reciprocal square root (within 2^-23), corrected once by
+// y (e/4 + 5 e^2/32), e = 1 - x y^4 (to e^3).  y is taken at x clamped to
+// [2^-1000, 2^1000] and multiplied by the true x: 0 gives 0, NaN propagates,
+// and outside the range the power underflows or overflows as the exact one.
+__device__ __forceinline__ double pow_9_4(double x) {
+  const double xc = fmin(fmax(x, 0x1p-1000), 0x1p1000);
+  const double y0 = __builtin_amdgcn_rsq(__builtin_amdgcn_sqrt(xc));
+  const double y2 = y0 * y0;
+  const double e = __builtin_fma(-xc, y2 * y2, 1.0);
+  const double y = __builtin_fma(y0, e * __builtin_fma(e, 0.15625, 0.25), y0);
+  return (x * x) * (x * (y * (y * y)));
+}
+
+// kinetics_sl (phenopowerlaw.f90:444-483) with tau_pos = t, tau_neg = -t:
+// gamma_dot_s = sign(tau_s) gdot0 x_s^n, x_s = |tau_s| / xi_s, and its
+// derivative c_s = gdot0 n x_s^(n-1) / xi_s.  Gives pw_s = x_s^n and (DERIV)
+// pm_s = x_s^(n-1) / xi_s; sign, gdot0 and n are left to the caller, which
+// multiplies a sum by them instead of every term.  Takes the reciprocal slip
+// resistances rxi = 1/xi (xi is fixed during the Newton iteration, so the
+// divisions are done once per state iteration).  A compile-time exponent
+// takes both powers from one chain; there is no zero test on it: c_s of a
+// rate below 1e-306 is below 1e-290 and changes no Newton system.
+template <int NE4, bool DERIV>
+__device__ __forceinline__ void slip_powers(const double* tau, const double* rxi, double* pw, double* pm,
+                                            const MatConst& mc) {
+  constexpr double TINY10 = 2.2250738585072014e-308 * 10.0;
+#pragma unroll
+  for (int s = 0; s < NSLIP; ++s) {
+    const double t = fabs(tau[s]);
+    const double x = t * rxi[s];
+    if constexpr (NE4 >= 8) {
+      const double xm1 = powc<NE4 - 4>(x);
+      pw[s] = xm1 * x;
+      if constexpr (DERIV) pm[s] = xm1 * rxi[s];
+    } else {
+      pw[s] = powe<NE4>(x, mc.n_e4, mc.n);
+      if constexpr (DERIV) pm[s] = (mc.gdot0 * pw[s] <= TINY10) ? 0.0 : pw[s] / t;
+    }
+  }
+}
+
+// phenopowerlaw_dotState (phenopowerlaw.f90:351-394) at the slip resistances
+// xi, rxi = 1/xi
+template <int NE4, int AE4>
+__device__ __forceinline__ void dot_state(const double* S, const double* xi, const double* rxi, double* dot,
+                                          const MatConst& mc) {
+  double tau[NSLIP], dg[NSLIP];
+  resolved_shears(S, mc.v, tau);
+  slip_powers<NE4, false>(tau, rxi, dg, nullptr, mc);
+#pragma unroll
+  for (int s = 0; s < NSLIP; ++s) dg[s] = mc.gdot0 * dg[s];
+#pragma unroll
+  for (int s = 0; s < NSLIP; ++s) {
+    const double x = 1.0 - xi[s] * mc.rxi_inf;
+    const double p = AE4 == 9 ? pow_9_4(fabs(x)) : powe<AE4>(fabs(x), mc.a_e4, mc.a);
+    const double left = copysign(p, x);
+    double hg = 0.0;
+#pragma unroll
+    for (int k = 0; k < NSLIP; ++k) hg += mc.hv[HTYPE[s][k] - 1] * dg[k];
+    dot[s] = mc.h0 * left * hg;
+  }
+#pragma unroll
+  for (int s = 0; s < NSLIP; ++s) dot[NSLIP + s] = dg[s];
+}
+
+// The Newton system of the Lp iteration, J x = b, as a 5x5 system.
+//
+// A change x of Lp (traceless, as b and every P_s are) changes the stress by
+// dS = -dt C : sym(X), X = G x, G = Fe^T A, and the constitutive Lp by
+// sum_s c_s P_s (P_s : dS), so
+//   J x = x + dt sum_s c_s P_s (P_s : C : sym(X)).
+// P_s is traceless and C cubic: P_s : C : sym(X) is a combination of the five
+// numbers w(x) = (X00 - X22, X11 - X22, X01 + X10, X02 + X20, X12 + X21) with
+// the coefficients v kD sgn_s(0,0), v kD sgn_s(1,1), v kA k_s(0,1),
+// v kA k_s(0,2), v kA k_s(1,2) (kD = C11 - C12, kA = C44, P_s = v sgn_s).  With
+// f_s = dt v^2 c_s and the five matrices U_j = sum_s f_s sgn_s k_s(j) that is
+//   J x = x + sum_j kappa_j U_j w_j(x),
+// and applying w to J x = b leaves the 5x5 system
+//   (1/kappa_i delta_ij + w_i(U_j)) y_j = w_i(b),   x = b - sum_j U_j y_j,
+// y_i = kappa_i w_i(x).
+// The same solution as that of the 9x9 system (up to rounding), from 25
+// instead of 81 (traceless: 64) matrix entries.  G is near the identity, which
+// makes the 5x5 matrix near a symmetric positive definite one times a 2x2
+// block: its LU rarely needs row exchanges.  Every entry of every U_j is plus
+// or minus one of 23 sums of one or two of the Hadamard sums of the direction
+// groups' f_s (qhad), formed once.
+//
+// GENERAL: rows scaled by kappa_i instead of divided by it (any C44 and
+// C11 - C12, zero included); otherwise f_s carries kA and the first two
+// diagonal entries are kA / kD (30 multiplications fewer).
+constexpr int NW = 5;
+__device__ __forceinline__ constexpr int um(int j) { return j == 0 ? 0 : j == 1 ? 1 : j == 2 ? 0 : j == 3 ? 0 : 1; }
+__device__ __forceinline__ constexpr int ul(int j) { return j == 0 ? 0 : j == 1 ? 1 : j == 2 ? 1 : j == 3 ? 2 : 2; }
+// sign of the first term of U_j(r), so that entries equal up to their sign
+// are the same expression
+__device__ __forceinline__ constexpr int usign(int j, int r) {
+  for (int g = 0; g < 3; ++g) {
+    const int code = qhad(g, r, um(j), ul(j));
+    if (code != 0) return code > 0 ? 1 : -1;
+  }
+  return 1;
+}
+// the five numbers w of X = G x (x row-major 3x3)
+__device__ __forceinline__ void newton_w(const double* G, const double* x, double* w) {
+  const double x22 = G[6] * x[2] + G[7] * x[5] + G[8] * x[8];
+  w[0] = G[0] * x[0] + G[1] * x[3] + G[2] * x[6] - x22;
+  w[1] = G[3] * x[1] + G[4] * x[4] + G[5] * x[7] - x22;
+  w[2] = G[0] * x[1] + G[1] * x[4] + G[2] * x[7] + G[3] * x[0] + G[4] * x[3] + G[5] * x[6];
+  w[3] = G[0] * x[2] + G[1] * x[5] + G[2] * x[8] + G[6] * x[0] + G[7] * x[3] + G[8] * x[6];
+  w[4] = G[3] * x[2] + G[4] * x[5] + G[5] * x[8] + G[6] * x[1] + G[7] * x[4] + G[8] * x[7];
+}
+
+// Solves M y = b (NW x NW, row-major) by LU with partial pivoting (first
+// largest entry of the column, as LAPACK's idamax); false: singular.
+__device__ __forceinline__ bool solve_pivot(double* M, double* b) {
+#pragma unroll
+  for (int k = 0; k < NW; ++k) {
+    int p = k;
+    double mx = fabs(M[NW * k + k]);
+#pragma unroll
+    for (int i = k + 1; i < NW; ++i) {
+      const double v = fabs(M[NW * i + k]);
+      if (v > mx) {
+        mx = v;
+        p = i;
+      }
+    }
+    if (!(mx > 0.0)) return false;
+    // exchange rows k and p by selects over the candidate rows (static
+    // register indices; the columns left of k are not read again)
+#pragma unroll
+    for (int i = k + 1; i < NW; ++i) {
+      const bool sw = p == i;
+#pragma unroll
+      for (int c = k; c < NW; ++c) {
+        const double u = M[NW * k + c], w = M[NW * i + c];
+        M[NW * k + c] = sw ? w : u;
+        M[NW * i + c] = sw ? u : w;
+      }
+      const double u = b[k], w = b[i];
+      b[k] = sw ? w : u;
+      b[i] = sw ? u : w;
+    }
+    const double inv = 1.0 / M[NW * k + k];
+#pragma unroll
+    for (int i = k + 1; i < NW; ++i) {
+      const double l = M[NW * i + k] * inv;
+#pragma unroll
+      for (int c = k + 1; c < NW; ++c) M[NW * i + c] -= l * M[NW * k + c];
+      b[i] -= l * b[k];
+    }
+  }
+#pragma unroll
+  for (int i = NW - 1; i >= 0; --i) {
+    double s = b[i];
+#pragma unroll
+    for (int c = i + 1; c < NW; ++c) s -= M[NW * i + c] * b[c];
+    b[i] = s / M[NW * i + i];
+  }
+  return true;
+}
+
+// Solves M y = b by LU without row exchanges.  Refuses (returns false; b then
+// holds no meaning) when a multiplier exceeds 1e6 in magnitude or a pivot's
+// magnitude is below 2^-1000 (zero and NaN included: the pivot's reciprocal is
+// the corrected hardware one, so a pivot near the bottom of the range goes to
+// the pivoted solve and its exact division).  Multipliers up to 1e6 cost at
+// most a few of the 16 digits of a Newton step that needs 6, and the residual
+// test of the next iteration uses the exact residual.  Refusals are collected
+// and tested once at the end (what is computed after one is discarded): no
+// branches inside the unrolled elimination, and the multipliers' magnitudes
+// enter one running maximum (a NaN multiplier is ignored by the maximum).
+__device__ __forceinline__ bool solve_nopivot(double* M, double* b) {
+  bool refused = false;
+  double lmax = 0.0;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+#pragma unroll
+    for (int k = 0; k < i; ++k) {
+      const double l = M[NW * i + k] * M[NW * k + k];
+      lmax = fmax(lmax, fabs(l));
+#pragma unroll
+      for (int c = k + 1; c < NW; ++c) M[NW * i + c] -= l * M[NW * k + c];
+      b[i] -= l * b[k];
+    }
+    const double piv = M[NW * i + i];
+    refused = refused || !(fabs(piv) >= 0x1p-1000);
+    M[NW * i + i] = rcp_cubic(piv);
+  }
+#pragma unroll
+  for (int i = NW - 1; i >= 0; --i) {
+    double s = b[i];
+#pragma unroll
+    for (int c = i + 1; c < NW; ++c) s -= M[NW * i + c] * b[c];
+    b[i] = s * M[NW * i + i];
+  }
+  return !(refused || lmax > 1e6);
+}
+
+// kappa_i of a GENERAL system
+__device__ __forceinline__ double newton_kappa(int i, const MatConst& mc) {
+  return i < 2 ? mc.C11 - mc.C12 : mc.C44;
+}
+
+// The U_j and the 5x5 matrix for G and the derivatives pm of slip_powers
+template <bool GENERAL>
+__device__ __forceinline__ void newton_matrix(const double* G, const double* pm, double dt, double (*U)[9], double* M,
+                                              const MatConst& mc) {
+  // Hadamard sums of f_s over each direction group
+  const double f = dt * (GENERAL ? mc.newton_f : mc.newton_fA);
+  double H[3][4];
+#pragma unroll
+  for (int g = 0; g < 3; ++g) {
+    const double a = pm[g] * f, bb = pm[g + 3] * f, x = pm[g + 6] * f, y = pm[g + 9] * f;
+    const double ab = a + bb, amb = a - bb, xy = x + y, xmy = x - y;
+    H[g][0] = ab + xy;
+    H[g][1] = ab - xy;
+    H[g][2] = amb + xmy;
+    H[g][3] = amb - xmy;
+  }
+#pragma unroll
+  for (int j = 0; j < NW; ++j)
+#pragma unroll
+    for (int r = 0; r < 9; ++r) {
+      double t = 0.0;
+      bool first = true;
+#pragma unroll
+      for (int g = 0; g < 3; ++g) {
+        const int code = qhad(g, r, um(j), ul(j)) * usign(j, r);
+        if (code != 0) {
+          const double h = H[g][(code > 0 ? code : -code) - 1];
+          t = first ? h : (code > 0 ? t + h : t - h);
+          first = false;
+        }
+      }
+      U[j][r] = usign(j, r) > 0 ? t : -t;
+    }
+#pragma unroll
+  for (int j = 0; j < NW; ++j) {
+    double w[NW];
+    newton_w(G, U[j], w);
+#pragma unroll
+    for (int i = 0; i < NW; ++i) M[NW * i + j] = GENERAL ? newton_kappa(i, mc) * w[i] : w[i];
+  }
+#pragma unroll
+  for (int i = 0; i < NW; ++i) M[NW * i + i] += GENERAL || i >= 2 ? 1.0 : mc.newton_d;
+}
+
+// The Newton step x of J x = b, in place of b (row-major 3x3, traceless).
+// false: refused (without PIVOT) or singular.
+template <bool GENERAL, bool PIVOT>
+__device__ __forceinline__ bool newton_step(const double* Fe, const double* A, const double* pm, double dt,
+                                            double* b, const MatConst& mc) {
+  double G[9];
+#pragma unroll
+  for (int m = 0; m < 3; ++m)
+#pragma unroll
+    for (int p = 0; p < 3; ++p) G[3 * m + p] = Fe[m] * A[p] + Fe[3 + m] * A[3 + p] + Fe[6 + m] * A[6 + p];
+  double U[NW][9], M[NW * NW], y[NW];
+  newton_matrix<GENERAL>(G, pm, dt, U, M, mc);
+  b[8] = -(b[0] + b[4]);
+  newton_w(G, b, y);
+  if constexpr (GENERAL) {
+#pragma unroll
+    for (int i = 0; i < NW; ++i) y[i] *= newton_kappa(i, mc);
+  }
+  const bool ok = PIVOT ? solve_pivot(M, y) : solve_nopivot(M, y);
+#pragma unroll
+  for (int r = 0; r < 8; ++r)
+#pragma unroll
+    for (int j = 0; j < NW; ++j) b[r] -= U[j][r] * y[j];
+  b[8] = -(b[0] + b[4]);
+  // Where the rates are stiff (an overshot iterate), b and sum U y agree in
+  // many digits and x keeps a rounding error of the size of b's, which J
+  // multiplies.  J acts on the five numbers w(x) only, and those are known
+  // without cancellation: y_i / kappa_i.  The symmetric traceless matrix that
+  // has the difference for its five numbers (G taken as the identity) removes
+  // it to within |G - I|.  Without it 871 instead of 162 of the 4096 points of
+  // 2 % strain steps take other iteration counts than with a pivoted 9x9 LU.
+  double e[NW];
+  newton_w(G, b, e);
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    if constexpr (GENERAL) {
+      const double k = newton_kappa(i, mc);
+      e[i] = k != 0.0 ? y[i] / k - e[i] : 0.0;
+    } else {
+      e[i] = i < 2 ? mc.newton_d * y[i] - e[i] : y[i] - e[i];
+    }
+  }
+  const double tr = (e[0] + e[1]) * (-1.0 / 3.0);
+  b[0] += e[0] + tr;
+  b[4] += e[1] + tr;
+  b[1] += 0.5 * e[2];
+  b[3] += 0.5 * e[2];
+  b[2] += 0.5 * e[3];
+  b[6] += 0.5 * e[3];
+  b[5] += 0.5 * e[4];
+  b[7] += 0.5 * e[4];
+  b[8] = -(b[0] + b[4]);
+  return ok;
+}
+
+// Elastic deformation and constitutive velocity gradient at Lp: Fe = A (I -
+// dt Lp), pm (slip_powers) and Lpc = v gdot0 sum_s sign_s x_s^n d_s n_s^T
+template <int NE4>
+__device__ __forceinline__ void lp_constitutive(const double* A, double dt, const double* Lp, const double* rxi,
+                                                double* Fe, double* pm, double* Lpc, const MatConst& mc) {
+  double B[9], Sl[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) B[k] = (k % 4 == 0 ? 1.0 : 0.0) - dt * Lp[k];
+  mm33(A, B, Fe);  // Fe = A B invFi_new, invFi_new = I
+  hooke_S(Fe, Sl, mc);
+  double tau[NSLIP], g[NSLIP];
+  resolved_shears(Sl, mc.v, tau);
+  slip_powers<NE4, true>(tau, rxi, g, pm, mc);
+#pragma unroll
+  for (int s = 0; s < NSLIP; ++s) g[s] = copysign(g[s], tau[s]);
+  slip_sum(g, mc.newton_vg, Lpc);
+}
+
+// integrateStress (phase_mechanical.f90:380-604); returns 0 (integrated) or
+// 1 (broken).  Takes the reciprocal slip resistances of the state and updates
+// S and Lp in registers; Fe, P and Fp of the integration the state loop keeps
+// are formed and stored by store_integrated.
+//
+// A = F invFp0 of the (sub)step and invFp0 (both in LDS, lane t) are formed
+// once per substep by the caller: they do not change during the state fixed
+// point.
+//
+// A Newton system whose LU without row exchanges is refused (a steep or
+// singular one) is formed again and solved with partial pivoting, as LAPACK's
+// dgesv in the reference: a branch that a wave takes only when one of its
+// lanes does.
+template <int NE4>
+__device__ __forceinline__ int integrate_stress(const double (*hA)[64], const double (*invFp0)[64], int t, double dt,
+                                                const double* rxi, double* Lp, double* S, int& newton,
+                                                const MatConst& mc) {
+  constexpr bool GENERAL = NE4 < 0;
+  // A is read from LDS where it is used, not hoisted into the registers the
+  // Newton system needs: the lane index passes through an empty asm, so every
+  // call's nine ds_reads are new loads (issued together, one wait), not the
+  // serialised one-wait-each accesses a volatile read would be
+  auto loadA = [&](double* A) {
+    int tl = t;
+    asm volatile("" : "+v"(tl));
+#pragma unroll
+    for (int k = 0; k < 9; ++k) A[k] = hA[k][tl];
+  };
+  double Lpg_old[9], dLp[9];
+  double res_old_n2 = 0.0;  // squared norms: the tests compare non-negative values
+  double step = 1.0;
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {
+    Lpg_old[k] = Lp[k];
+    dLp[k] = 0.0;
+  }
+  int it = 0;
+  // B, Fe and S of an iteration are not carried across the linear solve: the
+  // converged ones are formed again from the converged Lp after the loop (S
+  // is an output only on success)
+  for (;;) {
+    it++;
+    if (it > mc.N_iter_Lp_max) return 1;
+    double A[9], Fe[9], pm[NSLIP], res[9];
+    loadA(A);
+    lp_constitutive<NE4>(A, dt, Lp, rxi, Fe, pm, res, mc);
+    // res holds Lp_constitutive here
+    double n2Lpc = 0.0, n2Lp = 0.0, n2res = 0.0;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      n2Lpc += res[k] * res[k];
+      n2Lp += Lp[k] * Lp[k];
+      res[k] = Lp[k] - res[k];
+      n2res += res[k] * res[k];
+    }
+    {
+      // |res| < max(eps_rel max(|Lp|, |Lp_c|), eps_abs), compared squared:
+      // |res|^2 < max(eps_rel^2 max(|Lp|^2, |Lp_c|^2), eps_abs^2), no square root
+      const double tol2 = fmax((mc.eps_rel_Lp * mc.eps_rel_Lp) * fmax(n2Lp, n2Lpc), mc.eps_abs_Lp * mc.eps_abs_Lp);
+      // a sum of squares is NaN exactly when one of its terms is
+      if (isnan(n2res)) return 1;
+      if (n2res < tol2) break;
+      if (it == 1 || n2res < res_old_n2) {
+        res_old_n2 = n2res;
+#pragma unroll
+        for (int k = 0; k < 9; ++k) Lpg_old[k] = Lp[k];
+        step = 1.0;
+      } else {
+        step = mc.r_linesearch_Lp * step;
+#pragma unroll
+        for (int k = 0; k < 9; ++k) Lp[k] = Lpg_old[k] + dLp[k] * step;
+        continue;
+      }
+    }
+    if (!newton_step<GENERAL, false>(Fe, A, pm, dt, res, mc)) {
+      // formed again from Lp (the same values: the same operations), so that
+      // nothing is held for this rare branch
+      loadA(A);
+      lp_constitutive<NE4>(A, dt, Lp, rxi, Fe, pm, res, mc);
+#pragma unroll
+      for (int k = 0; k < 9; ++k) res[k] = Lp[k] - res[k];
+      if (!newton_step<GENERAL, true>(Fe, A, pm, dt, res, mc)) return 1;  // singular
+    }
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      dLp[k] = -res[k];
+      Lp[k] = Lp[k] + dLp[k] * step;
+    }
+  }
+  newton += it;
+  double B[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) B[k] = (k % 4 == 0 ? 1.0 : 0.0) - dt * Lp[k];
+  double invFp_new[9], Fpn[9];
+  {
+    double iF0[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) iF0[k] = invFp0[k][t];
+    mm33(iF0, B, invFp_new);
+  }
+  if (!inv33(invFp_new, Fpn, nullptr)) return 1;
+  double T1[9], A[9];
+  loadA(A);
+  mm33(A, B, T1);  // F invFp_new (= Fe, invFi_new = I)
+  hooke_S(T1, S, mc);
+  return 0;
+}
+
+// Fe, P and Fp of the last successful integrate_stress (same operations on
+// the same Lp, A and invFp0, hence the same values), stored when the state
+// fixed point leaves with it; integrations that a later state iteration
+// supersedes store nothing
+__device__ __forceinline__ void store_integrated(const double (*hA)[64], const double (*invFp0)[64], int t,
+                                                 double dt, const double* Lp, const double* S, ConstArgs* ap,
+                                                 Lane l) {
+  const MpState io = ap->s;
+  const int64_t N = io.N;
+  double A[9], B[9], invFp_new[9], Fpn[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {
+    A[k] = hA[k][t];
+    B[k] = (k % 4 == 0 ? 1.0 : 0.0) - dt * Lp[k];
+  }
+  {
+    double iF0[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) iF0[k] = invFp0[k][t];
+    mm33(iF0, B, invFp_new);
+  }
+  inv33(invFp_new, Fpn, nullptr);  // invertible: integrate_stress checked it
+  double T1[9];
+  mm33(A, B, T1);
+  store33(io.Fe, N, l, T1);
+  {
+    double iFt[9], T2[9], P[9];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) iFt[3 * i + j] = invFp_new[3 * j + i];
+    mm33(S, iFt, T2);
+    mm33(T1, T2, P);
+    store33(io.P, N, l, P);
+  }
+  const double d = pow(det33(Fpn), 1.0 / 3.0);
+  const double rd = rcp_refined(d);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) Fpn[k] = div_rcp(Fpn[k], d, rd);
+  store33(io.Fp, N, l, Fpn);
+}
+
+// 0.75 + 0.25 tanh(x) (phase_mechanical.f90:674-691), tanh x = 1 - 2 / (e^2x + 1)
+// to an absolute rounding error, which is what the sum with 0.75 keeps (a
+// third of the library tanh's instructions); tanh 20 is 1 in double precision,
+// and a NaN stays one
+__device__ __forceinline__ double damping(double x) {
+  const double e = exp(2.0 * (x > 20.0 ? 20.0 : x));
+  return __builtin_fma(-0.5, rcp_cubic(e + 1.0), 1.0);
+}
+
+// per-lane LDS columns of one 64-lane block: the state fixed point's rate
+// history (dotState_last(:,1), its difference to dotState_last(:,2)) and the
+// (sub)step's matrices, which stay in LDS while the Lp Newton iteration needs
+// the registers
+struct MpLds {
+  double last1[NSTATE][64];
+  double d12[NSTATE][64];
+  double iFp0[9][64];  // invFp0 of the current (sub)step
+  double A[9][64];     // F_(sub)step invFp0
+};
+
+template <int NE4, int AE4>
+__device__ __forceinline__ void mp_point(ConstArgs* ap, const int64_t c, MpLds& sh) {
+  const MatConst mc = ap->mc;
+  const double dt = ap->dt;
+  const int64_t N = ap->s.N;
+  const int t = threadIdx.x;
+  double (&h_last1)[NSTATE][64] = sh.last1;
+  double (&h_d12)[NSTATE][64] = sh.d12;
+  const Lane l{(uint32_t)(c * 8)};
+  // state (xi, gamma) at the start of the (sub)step; after a converged one, at
+  // its end
+  double s0[NSTATE];
+  double Lp[9], S[9];
+  double Fi[9], F0i[9];  // F and F0 of the increment (not written here), loaded once
+  double fp0v[9];        // Fp0 of the (sub)step about to be integrated (planes in order)
+  // every value of the whole step (phase_restore: S = S0, Fp = Fp0, state =
+  // state0) is loaded before the first one is used: one memory round trip,
+  // which nothing else hides (one wave per SIMD)
+  {
+    const MpState s = ap->s;
+    const int64_t n = stride_here(N);
+    load33(s.F, n, l, Fi);
+    load33(s.F0, n, l, F0i);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) fp0v[k] = ld(s.Fp0 + k * n, l);
+    load33(s.S0, n, l, S);
+#pragma unroll
+    for (int k = 0; k < NSLIP; ++k) {
+      s0[k] = ld(s.xi0 + k * n, l);
+      s0[NSLIP + k] = ld(s.gamma0 + k * n, l);
+    }
+    load33(s.Lp, n, l, Lp);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // substep start values live in memory: the increment's converged values
+  // (F0, Lp0, Fp0, state0) until a partial substep succeeded, then the
+  // substep scratch planes
+  bool in_sub = false;
+  int newton = 0, fpi = 0;
+  double stepFrac = 0.0, step = mc.r_cutback * (1.0 / mc.r_cutback);
+  bool converged = false;
+  if (step < 1.0) load33(here(ap)->s.Lp0, N, l, Lp);  // 1 / r_cutback may round down
+  bool todo = step > mc.r_cutback_min;
+  if (!todo) {  // leaves with the restored values
+    double* Fp = here(ap)->s.Fp;
+    const int64_t n = stride_here(N);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) st(Fp + k * n, l, fp0v[k]);
+  }
+  while (todo) {
+    // A = F_(sub)step invFp0 and invFp0 are fixed during the state fixed
+    // point (integrateStress, phase_mechanical.f90:425-432)
+    bool fp0_singular;
+    {
+      // F of the (sub)step: F0l + step (F - F0), phase_mechanical.f90:1093-1096
+      double Fl[9], Fp0[9], iF0[9], A[9], F0l[9];
+      double* sub = ap->sub;
+      const int64_t n = stride_here(N);
+      if (in_sub) {
+        load33(sub + SUB_F0 * n, n, l, F0l);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) F0l[k] = F0i[k];
+      }
+#pragma unroll
+      for (int k = 0; k < 9; ++k) Fl[k] = F0l[k] + step * (Fi[k] - F0i[k]);
+      if (step < 1.0) store33(sub + SUB_FLOC * n, n, l, Fl);  // start of the next substep
+#pragma unroll
+      for (int k = 0; k < 9; ++k) Fp0[rm(k)] = fp0v[k];
+      fp0_singular = !inv33(Fp0, iF0, nullptr);
+      mm33(Fl, iF0, A);
+#pragma unroll
+      for (int k = 0; k < 9; ++k) {
+        sh.iFp0[k][t] = iF0[k];
+        sh.A[k][t] = A[k];
+      }
+    }
+    const double sdt = step * dt;
+    // integrateStateFPI (phase_mechanical.f90:611-693).  Pass 0 predicts the
+    // state from the start values' rate, pass it > 0 follows the it-th stress
+    // integration; the rate, the history and the state update are the same
+    // code in both (a loop of two thirds of the instructions that separate
+    // copies take: a small launch pays for fetching each of them).  The
+    // current state is s0 + last1 sdt throughout, so only xi, which the
+    // kinetics read, is held.
+    bool broken;
+    double xi[NSLIP], rxi[NSLIP];
+#pragma unroll
+    for (int k = 0; k < NSLIP; ++k) xi[k] = s0[k];
+    for (int it = 0;; ++it) {
+      double dot[NSTATE];
+#pragma unroll
+      for (int k = 0; k < NSLIP; ++k) rxi[k] = rcp_cubic(xi[k]);
+      if (it > 0) {
+        fpi++;
+        broken = fp0_singular || integrate_stress<NE4>(sh.A, sh.iFp0, t, sdt, rxi, Lp, S, newton, mc) != 0;
+        if (broken) break;
+      }
+      dot_state<NE4, AE4>(S, xi, rxi, dot, mc);
+      bool nan = false;
+#pragma unroll
+      for (int k = 0; k < NSLIP; ++k) nan = nan || __builtin_isunordered(dot[k], dot[NSLIP + k]);
+      if (nan) {  // after an integration: leaves with it
+        broken = it == 0;
+        break;
+      }
+      // the rate history is read from LDS in one batch before the sums
+      // (issued together: one wait instead of one per state variable)
+      double l1v[NSTATE], zeta = 1.0;
+      if (it > 0) {
+        double d12v[NSTATE];
+#pragma unroll
+        for (int k = 0; k < NSTATE; ++k) {
+          l1v[k] = h_last1[k][t];
+          d12v[k] = h_d12[k][t];
+        }
+        double dp12 = 0.0, dp22 = 0.0, dp01 = 0.0;
+#pragma unroll
+        for (int k = 0; k < NSTATE; ++k) {
+          dp12 += (dot[k] - l1v[k]) * d12v[k];
+          dp22 += d12v[k] * d12v[k];
+          dp01 += dot[k] * l1v[k];
+        }
+        if (fmin(dp01, dp12) < 0.0 && dp22 > 0.0) zeta = damping(2.0 + 4.0 * dp12 / dp22);
+      } else {
+#pragma unroll
+        for (int k = 0; k < NSTATE; ++k) l1v[k] = 0.0;
+      }
+      bool conv = it > 0;
+      const double omz = 1.0 - zeta;
+#pragma unroll
+      for (int k = 0; k < NSTATE; ++k) {
+        const double l1 = l1v[k];
+        // the damped rate replaces dotState: it is dotState_last(:,1) of
+        // the next iteration (phase_mechanical.f90:653-655)
+        const double dk = dot[k] * zeta + l1 * omz;
+        h_d12[k][t] = dk - l1;  // dotState_last(:,1) - dotState_last(:,2) of the next iteration
+        h_last1[k][t] = dk;
+        const double nw = __builtin_fma(dk, sdt, s0[k]);
+        const double r = __builtin_fma(l1, sdt, s0[k]) - nw;
+        if (k < NSLIP) xi[k] = nw;
+        const double at = (k < NSLIP) ? mc.atol_xi : mc.atol_gamma;
+        conv = conv && (fabs(r) <= fmax(at, mc.eps_rel_state * fabs(nw)));
+      }
+      // converged, or the last iteration (integrateStateFPI then returns the
+      // last integration's broken = false)
+      if (conv || it >= mc.N_iter_state_max) {
+        broken = it == 0;
+        break;
+      }
+    }
+    converged = !broken;
+    // step control: the next substep after a converged one, else a cut-back
+    // step from the restored start values
+    ConstArgs* p = here(ap);
+    const MpState s = p->s;
+    double* sub = p->sub;
+    const int64_t n = stride_here(N);
+    if (converged) {
+      store_integrated(sh.A, sh.iFp0, t, sdt, Lp, S, p, l);
+#pragma unroll
+      for (int k = 0; k < NSTATE; ++k) s0[k] = __builtin_fma(h_last1[k][t], sdt, s0[k]);
+      stepFrac = stepFrac + step;
+      step = fmin(1.0 - stepFrac, mc.r_increase * step);
+      todo = step > 0.0;
+      if (todo) {
+        // all loads before the stores: the compiler cannot tell the planes
+        // apart, and a load after a store would wait for the one before it
+        double fl[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+          fl[k] = ld(sub + (SUB_FLOC + k) * n, l);
+          fp0v[k] = ld(s.Fp + (k) * n, l);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // all issued before the first store (one round trip)
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+          st(sub + (SUB_F0 + k) * n, l, fl[k]);
+          st(sub + (SUB_LP0 + k) * n, l, Lp[rm(k)]);
+          st(sub + (SUB_FP0 + k) * n, l, fp0v[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < NSTATE; ++k) st(sub + (SUB_ST0 + k) * n, l, s0[k]);
+        in_sub = true;
+      }
+    } else {
+      step = mc.r_cutback * step;
+      load33(s.S0, n, l, S);
+#pragma unroll
+      for (int k = 0; k < 9; ++k) fp0v[k] = ldv((in_sub ? sub + SUB_FP0 * n : s.Fp0) + k * n, l);
+      if (step < 1.0) load33_sel(in_sub, sub + SUB_LP0 * n, s.Lp0, n, l, Lp);
+#pragma unroll
+      for (int k = 0; k < NSLIP; ++k) {
+        s0[k] = ldv((in_sub ? sub + SUB_ST0 * n : s.xi0) + k * n, l);
+        s0[NSLIP + k] = ldv((in_sub ? sub + (SUB_ST0 + NSLIP) * n : s.gamma0) + k * n, l);
+      }
+      todo = step > mc.r_cutback_min;
+      // the restored Fp is stored only by a point that leaves with it: an
+      // integrated one stores its own
+      if (!todo) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) st(s.Fp + (k) * n, l, fp0v[k]);
+      }
+    }
+  }
+  ConstArgs* p = here(ap);
+  const MpState s = p->s;
+  store33(s.Lp, N, l, Lp);
+  store33(s.S, N, l, S);
+  const int64_t n = stride_here(N);
+#pragma unroll
+  for (int k = 0; k < NSLIP; ++k) {
+    st(s.xi + (k) * n, l, s0[k]);
+    st(s.gamma + (k) * n, l, s0[NSLIP + k]);
+  }
+  if (s.iters) {
+    s.iters[c] = newton;
+    s.iters[N + c] = fpi;
+  }
+  if (p->broken) p->broken[c] = converged ? 0 : 1;
+  if (!converged && p->ill) atomicOr(p->ill, 1);
+}
+
+// the arguments of a kernel whose only parameter they are, and a table's entry
+__device__ __forceinline__ ConstArgs* kernel_args() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (ConstArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+#else
+  return nullptr;
+#endif
+}
+__device__ __forceinline__ ConstArgs* table_args(const KernelArgs* p) { return (ConstArgs*)p; }
+
+template <int NE4, int AE4>
+__global__ void __launch_bounds__(64) mp_points_kernel(KernelArgs) {
+  __shared__ MpLds sh;
+  ConstArgs* a = kernel_args();
+  const int64_t c = a->c_begin + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= a->c_end) return;
+  mp_point<NE4, AE4>(a, c, sh);
+}
+
+// ---------------------------------------------------------------------------
+// Consistent tangent dPdF (phase_mechanical_dPdF, phase_mechanical.f90:1137-1258)
+// with Fi = I, dLi/dS = 0.  Output: 81 planes of N doubles, plane index
+// i+3j+9k+27l for dPdF(i,j,k,l) (column-major as the reference).
+//
+// Column (p,o) of dS/dF solves dS + dt sum_s c_s U_s (P_s : dS) = C : X with
+// X = Fe(p,:) (x) invFp(o,:), U_s = C : (H P_s), H = Fe^T F invFp0.  P_s : dS
+// is a combination of five numbers of dS, so with the U_j and the diagonal of
+// the Newton system (newton_step, H in the place of G)
+//   (diag + w(H U_j)) y = w(X),   V = sum_j U_j y_j,   dS = C : (X - H V),
+// and dFp^-1/dF = -invFp0 V.  The 5x5 matrix is inverted once (partial
+// pivoting) for the nine columns: 5730 instead of 8400 instructions, no 9x9
+// elimination in one dependent chain (28 -> 17 us for a call of one wave).
+// ---------------------------------------------------------------------------
+
+// inverse of M (NW x NW, row-major) by Gauss-Jordan with partial pivoting
+__device__ __forceinline__ void invert_pivot(double* M, double* R) {
+#pragma unroll
+  for (int k = 0; k < NW * NW; ++k) R[k] = k % (NW + 1) == 0 ? 1.0 : 0.0;
+#pragma unroll
+  for (int k = 0; k < NW; ++k) {
+    int p = k;
+    double mx = fabs(M[NW * k + k]);
+#pragma unroll
+    for (int i = k + 1; i < NW; ++i) {
+      const double v = fabs(M[NW * i + k]);
+      if (v > mx) {
+        mx = v;
+        p = i;
+      }
+    }
+#pragma unroll
+    for (int i = k + 1; i < NW; ++i) {
+      const bool sw = p == i;
+#pragma unroll
+      for (int c = k; c < NW; ++c) {
+        const double u = M[NW * k + c], w = M[NW * i + c];
+        M[NW * k + c] = sw ? w : u;
+        M[NW * i + c] = sw ? u : w;
+      }
+#pragma unroll
+      for (int c = 0; c < NW; ++c) {
+        const double u = R[NW * k + c], w = R[NW * i + c];
+        R[NW * k + c] = sw ? w : u;
+        R[NW * i + c] = sw ? u : w;
+      }
+    }
+    const double inv = 1.0 / M[NW * k + k];
+#pragma unroll
+    for (int c = k + 1; c < NW; ++c) M[NW * k + c] *= inv;
+#pragma unroll
+    for (int c = 0; c < NW; ++c) R[NW * k + c] *= inv;
+#pragma unroll
+    for (int i = 0; i < NW; ++i)
+      if (i != k) {
+        const double l = M[NW * i + k];
+#pragma unroll
+        for (int c = k + 1; c < NW; ++c) M[NW * i + c] -= l * M[NW * k + c];
+#pragma unroll
+        for (int c = 0; c < NW; ++c) R[NW * i + c] -= l * R[NW * k + c];
+      }
+  }
+}
+
+struct TangentArgs {
+  MpState s;
+  MatConst mc;
+  double dt;
+  double* dPdF;  // 81 planes of N (plane k+3l+9p+27o)
+  int64_t c_begin, c_end;
+};
+
+template <int NE4>
+__global__ void __launch_bounds__(64) mp_points_tangent_kernel(TangentArgs a) {
+  constexpr bool GENERAL = NE4 < 0;
+  const MatConst& mc = a.mc;
+  const int64_t N = a.s.N;
+  const int64_t c = a.c_begin + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= a.c_end) return;
+  const Lane l{(uint32_t)(c * 8)};
+  double F[9], Fe[9], S[9], invFp[9], invFp0[9], cs[NSLIP];
+  {
+    double Fp[9], Fp0[9], xi[NSLIP], rxi[NSLIP], tau[NSLIP], pw[NSLIP];
+    load33(a.s.F, N, l, F);
+    load33(a.s.Fp, N, l, Fp);
+    load33(a.s.Fp0, N, l, Fp0);
+    load33(a.s.S, N, l, S);
+    load33(a.s.Fe, N, l, Fe);
+#pragma unroll
+    for (int k = 0; k < NSLIP; ++k) xi[k] = ld(a.s.xi + k * N, l);
+    if (!inv33(Fp, invFp, nullptr)) {
+#pragma unroll
+      for (int k = 0; k < 9; ++k) invFp[k] = 0.0;
+    }
+    if (!inv33(Fp0, invFp0, nullptr)) {
+#pragma unroll
+      for (int k = 0; k < 9; ++k) invFp0[k] = 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < NSLIP; ++k) rxi[k] = 1.0 / xi[k];
+    resolved_shears(S, mc.v, tau);
+    slip_powers<NE4, true>(tau, rxi, pw, cs, mc);
+  }
+  double T2[9], H[9], U[NW][9], Mi[NW * NW];
+  mm33(F, invFp0, T2);
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) H[3 * i + j] = Fe[i] * T2[j] + Fe[3 + i] * T2[3 + j] + Fe[6 + i] * T2[6 + j];
+  {
+    double M[NW * NW];
+    newton_matrix<GENERAL>(H, cs, a.dt, U, M, mc);
+    invert_pivot(M, Mi);
+  }
+  double iFt[9], SiT[9], FiFp[9], u3[9], G[9];
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) iFt[3 * i + j] = invFp[3 * j + i];
+  mm33(S, iFt, SiT);     // S invFp^T
+  mm33(F, invFp, FiFp);  // F invFp
+  mm33(FiFp, S, u3);     // F invFp S
+  mm33(invFp, SiT, G);   // invFp S invFp^T
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+#pragma unroll
+    for (int o = 0; o < 3; ++o) {
+      double X[9], w[NW], V[9];
+#pragma unroll
+      for (int m = 0; m < 3; ++m)
+#pragma unroll
+        for (int r = 0; r < 3; ++r) X[3 * m + r] = Fe[3 * p + m] * invFp[3 * o + r];
+      w[0] = X[0] - X[8];
+      w[1] = X[4] - X[8];
+      w[2] = X[1] + X[3];
+      w[3] = X[2] + X[6];
+      w[4] = X[5] + X[7];
+      if constexpr (GENERAL) {
+#pragma unroll
+        for (int i = 0; i < NW; ++i) w[i] *= newton_kappa(i, mc);
+      }
+#pragma unroll
+      for (int k = 0; k < 9; ++k) V[k] = 0.0;
+#pragma unroll
+      for (int j = 0; j < NW; ++j) {
+        double y = 0.0;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) y += Mi[NW * j + i] * w[i];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) V[k] += U[j][k] * y;
+      }
+      V[8] = -(V[0] + V[4]);
+      double HV[9], dS[9], diFp[9], B1[9], B2[9], B3[9], D[9];
+      mm33(H, V, HV);
+#pragma unroll
+      for (int k = 0; k < 9; ++k) X[k] -= HV[k];
+      cubic_contract(X, dS, mc);
+      mm33(invFp0, V, diFp);  // -dFp^-1
+      mm33(T2, V, B1);        // -F dFp^-1
+      mm33(B1, S, B2);
+      mm33(FiFp, dS, B3);
+#pragma unroll
+      for (int k = 0; k < 9; ++k) B3[k] -= B2[k];
+      mm33(B3, iFt, D);       // (F dFp^-1 S + F invFp dS) invFp^T
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          double v = D[3 * k + q];
+#pragma unroll
+          for (int m = 0; m < 3; ++m) v -= u3[3 * k + m] * diFp[3 * q + m];  // F invFp S dFp^-T
+          if (k == p) v += G[3 * o + q];  // dF invFp S invFp^T
+          st(a.dPdF + (int64_t)(k + 3 * q + 9 * p + 27 * o) * N, l, v);
+        }
+    }
+}
+
+// clears the terminally-ill flag of one call
+__global__ void ill_reset_kernel(int* ill) { *ill = 0; }
+
+}  // namespace
+
+// The exponents of the example material (n_sl = 20, a_sl = 2.25) are compiled
+// in, with the Newton system divided by its stiffness scales, which must not
+// vanish; any other material runs the runtime-exponent instantiation.
+static bool example_class(const MatConst& mc) {
+  return mc.n_e4 == 80 && mc.a_e4 == 9 && std::isfinite(mc.newton_d) && mc.newton_d != 0.0;
+}
+// lanes address planes by a 32-bit byte offset (cell index * 8)
+static void check_range(const MpState& s, int64_t& c_begin, int64_t& c_end) {
+  if (c_end < 0) c_end = s.N;
+  if (c_begin < 0 || c_end > s.N || c_begin > c_end) throw std::runtime_error("material-point range out of bounds");
+  if (s.N > ((int64_t)1 << 29)) throw std::runtime_error("material-point planes longer than 2^29 cells");
+}
+
+void launch_mp_points(const MpState& s, const MatConst& mc, double dt, int* d_ill, double* d_sub, hipStream_t st,
+                      int* d_broken, int64_t c_begin, int64_t c_end) {
+  check_range(s, c_begin, c_end);
+  if (c_begin == c_end) return;
+  const KernelArgs a{s, mc, dt, d_ill, d_broken, d_sub, c_begin, c_end};
+  const dim3 grid((unsigned)((c_end - c_begin + 63) / 64));
+  if (d_ill) hipLaunchKernelGGL(ill_reset_kernel, dim3(1), dim3(1), 0, st, d_ill);
+  if (example_class(mc)) hipLaunchKernelGGL((mp_points_kernel<80, 9>), grid, dim3(64), 0, st, a);
+  else hipLaunchKernelGGL((mp_points_kernel<-1, -1>), grid, dim3(64), 0, st, a);
+  SCA_HIP(hipGetLastError());
+}
+
+void launch_mp_tangent(const MpState& s, const MatConst& mc, double dt, double* dPdF, hipStream_t st,
+                       int64_t c_begin, int64_t c_end) {
+  check_range(s, c_begin, c_end);
+  if (c_begin == c_end) return;
+  const TangentArgs a{s, mc, dt, dPdF, c_begin, c_end};
+  const dim3 grid((unsigned)((c_end - c_begin + 63) / 64));
+  if (example_class(mc)) hipLaunchKernelGGL(mp_points_tangent_kernel<80>, grid, dim3(64), 0, st, a);
+  else hipLaunchKernelGGL(mp_points_tangent_kernel<-1>, grid, dim3(64), 0, st, a);
+  SCA_HIP(hipGetLastError());
+}
+
+}  // namespace sca

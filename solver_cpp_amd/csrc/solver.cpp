@@ -367,6 +367,7 @@ void Rve::setup(const sc_rve_desc& d, bool residual_graphs) {
   mp.xi = dalloc(12 * N);
   mp.gamma = dalloc(12 * N);
   mp.iters = static_cast<int*>(dev_alloc(2 * N * sizeof(int)));
+  mp.repivot = static_cast<int*>(dev_alloc((N + 1) * sizeof(int)));
   sub = dalloc((size_t)mp_sub_planes() * N);
   X = dalloc(9 * N);
   F_last_inc = dalloc(9 * N);
@@ -476,7 +477,9 @@ void Rve::release() {
   for (double* p : allocs) dev_free(p);
   allocs.clear();
   dev_free(mp.iters);
+  dev_free(mp.repivot);
   mp.iters = nullptr;
+  mp.repivot = nullptr;
   dev_free(d_minmax_i);
   d_minmax_i = nullptr;
   fft.release();
