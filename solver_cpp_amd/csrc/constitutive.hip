@@ -1278,7 +1278,12 @@ __global__ void mp_init_kernel(MpState s, const double* Fp_init, double xi_0) {
 int mp_partial_blocks(int64_t N) { return (int)((N + PAV_CELLS - 1) / PAV_CELLS); }
 int mp_sub_planes() { return SUB_PLANES; }
 
-void launch_mp_response(const MpState& s, const MatConst& mc, double dt, int* d_ill, double* d_sub, hipStream_t st) {
+void launch_response_reset(int* repivot, int* d_ill, hipStream_t st) {
+  hipLaunchKernelGGL(repivot_reset_kernel, dim3(1), dim3(1), 0, st, repivot, d_ill);
+}
+
+void launch_mp_response(const MpState& s, const MatConst& mc, double dt, int* d_ill, double* d_sub, hipStream_t st,
+                        bool clear) {
   if (s.N < 1) return;
   // lanes address planes by a 32-bit byte offset (cell index * 8)
   if (s.N > ((int64_t)1 << 29)) throw std::runtime_error("material-point planes longer than 2^29 cells");
@@ -1290,7 +1295,7 @@ void launch_mp_response(const MpState& s, const MatConst& mc, double dt, int* d_
   // second pass: a fixed grid striding over the list (it holds at most the
   // range's points)
   const int blocks2 = std::min(blocks, 1024);
-  hipLaunchKernelGGL(repivot_reset_kernel, dim3(1), dim3(1), 0, st, s.repivot, d_ill);
+  if (clear) launch_response_reset(s.repivot, d_ill, st);
   if (mc.n_e4 == 80 && mc.a_e4 == 9) {
     hipLaunchKernelGGL((mp_response_kernel<80, 9>), dim3(blocks), dim3(64), 0, st, a);
     hipLaunchKernelGGL((mp_repivot_kernel<80, 9>), dim3(blocks2), dim3(64), 0, st, a);

@@ -211,20 +211,34 @@ __device__ __forceinline__ const cpx<T>* stage_tw(cpx<T>* lds_tw, const cpx<T>* 
 
 // strided complex pass (y or z): pencil (o, i) starts at
 // (o / d1) * s1 + (o % d1) * s2 + i with element stride es; a block takes P
-// consecutive i of one o, the pencil index fastest across lanes
-template <typename T, int N, int SIGN>
+// consecutive i of one o, the pencil index fastest across lanes.  The first
+// side.blocks() blocks do the side job's work instead (Side: NoSide, or a few
+// sums of the evaluation that would otherwise be launches of their own).
+// Blocks go to the 8 XCDs in turn: each XCD gets a contiguous eighth of the
+// pencils, since neighbouring blocks of a y pass share the cache lines at
+// their ends (rows of N/2 + 1 entries start anywhere in a line): y pass of
+// 9 x 128^3, forward / inverse 68 / 68 -> 62 / 48 us, in single precision
+// 39 / 40 -> 28 / 28; z pass 46 -> 45.
+template <typename T, int N, int SIGN, typename Side>
 __global__ void __launch_bounds__(MAX_PENCIL_BLOCK) strided_kernel(cpx<T>* data, int ni, int64_t npen, int d1,
                                                                    int64_t s1, int64_t s2, int64_t es,
-                                                                   const cpx<T>* tw_g) {
+                                                                   const cpx<T>* tw_g, Side side) {
   using S = Shape<T, N>;
   extern __shared__ unsigned char smem_raw[];
+  if constexpr (Side::blocks() > 0) {
+    if (blockIdx.x < Side::blocks()) {
+      side.run((int)blockIdx.x, reinterpret_cast<double*>(smem_raw));
+      return;
+    }
+  }
   cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem_raw);
   const int P = blockDim.x / S::TP;  // a power of two
   const cpx<T>* tw = stage_tw<T, N>(lds + P * S::LD, tw_g);
   const int p = threadIdx.x & (P - 1), t = threadIdx.x >> __builtin_ctz(P);
   // pencils (o, i) numbered with i fastest across the whole launch, so that a
   // block does not hold a mostly empty row of i (ni = N/2 + 1 is odd)
-  const int64_t pen = (int64_t)blockIdx.x * P + p;
+  const unsigned nb = gridDim.x - Side::blocks(), b = blockIdx.x - Side::blocks();  // nb: a multiple of 8
+  const int64_t pen = (int64_t)((b & 7) * (nb >> 3) + (b >> 3)) * P + p;
   const int64_t o = pen / ni;
   const int i = (int)(pen - o * ni);
   const int64_t base = (o / d1) * s1 + (o % d1) * s2 + i;
@@ -237,6 +251,60 @@ __global__ void __launch_bounds__(MAX_PENCIL_BLOCK) strided_kernel(cpx<T>* data,
 #pragma unroll
     for (int j = 0; j < S::E; ++j) data[base + (int64_t)(t + S::TP * j) * es] = v[j];
   }
+}
+
+// Forward z pass and an operation on the nine components of each wavevector
+// in one kernel: the spectrum is read and written once instead of twice.  A
+// block holds the z pencils of all nine components for W consecutive (x, y)
+// frequencies (their index q = i + nr y is contiguous in memory) in LDS: TP
+// threads a pencil as in the strided pass, the same stages on the same points,
+// so every transform has the strided pass's bits.  (The inverse transform
+// starts with y, so its z pass is not in here.)
+//
+// W: the smallest power of two with W N >= 256 (an operation for every thread,
+// and no more blocks than the operation's own kernel has) and 64 contiguous
+// bytes; at most 80 KB of LDS, so that two blocks share a CU and one's memory
+// phase overlaps the other's transforms.
+template <typename T, int N>
+struct ZShape {
+  using S = Shape<T, N>;
+  static constexpr int width() {
+    int w = 64 / (2 * (int)sizeof(T));
+    while (w * N < 256) w *= 2;
+    return w;
+  }
+  static constexpr int W = width();
+  static constexpr int PENCILS = 9 * W;
+  static constexpr int THREADS = PENCILS * S::TP;
+  static constexpr int ENTRIES = PENCILS * S::LD + N;
+  static constexpr bool fits = THREADS <= 1024 && (size_t)ENTRIES * 2 * sizeof(T) <= 80000;
+};
+
+template <typename T, int N, typename Op>
+__device__ __forceinline__ void zop_block(cpx<T>* data, int64_t K, int64_t nq, int64_t block, const cpx<T>* tw_g,
+                                          const Op& op, cpx<T>* lds) {
+  using S = Shape<T, N>;
+  using Z = ZShape<T, N>;
+  const cpx<T>* tw = stage_tw<T, N>(lds + Z::PENCILS * S::LD, tw_g);
+  const int p = threadIdx.x % Z::W, ct = threadIdx.x / Z::W;
+  const int c = ct % 9, t = ct / 9;
+  const int64_t q0 = block * Z::W, q = q0 + p;
+  const bool ok = q < nq;
+  cpx<T>* row = lds + (c * Z::W + p) * S::LD;
+  const cpx<T>* base = data + c * K + q;
+  cpx<T> v[S::E];
+#pragma unroll
+  for (int j = 0; j < S::E; ++j) v[j] = ok ? base[(int64_t)(t + S::TP * j) * nq] : cpx<T>{(T)0, (T)0};
+  stages<T, N, S::E, -1, 1>(v, t, row, tw);
+  __syncthreads();  // the stages' last reads of the rows are done
+#pragma unroll
+  for (int j = 0; j < S::E; ++j) row[t + S::TP * j] = v[j];
+  __syncthreads();
+  for (int f = threadIdx.x; f < Z::W * N; f += Z::THREADS) {
+    const int fp = f % Z::W, z = f / Z::W;
+    if (q0 + fp < nq) op.point(q0 + fp, z, lds + fp * S::LD + z, Z::W * S::LD, data + q0 + fp + (int64_t)z * nq);
+  }
+  op.finish();
 }
 
 // Rows of the pencil that pairs rows ra and rb of a set of set_rows rows

@@ -164,6 +164,7 @@ class Rve {
   // (null: on this context's own stream)
   Batcher* batch = nullptr;
   GammaHost gamma_host(bool do_gamma) const;
+  bool fused_gamma() const;
 
   // descriptor and geometry
   sc_rve_desc desc;
@@ -226,6 +227,9 @@ class Rve {
   hipGraphExec_t g_exec = nullptr;
   std::vector<char> g_sig, g_seen;
   int64_t stats_graph_captures = 0, stats_graph_updates = 0;
+  // the pivoting list and the ill flag are cleared (by the last evaluation's
+  // end): the next response need not clear them
+  bool response_clean = false;
   bool scal_pending = false, scal_rotate = false, scal_residual = false, scal_reused = false;
 
   // MechBase state (mech_base.h:75-107), column-major

@@ -520,6 +520,7 @@ void Rve::constitutive_response(const double* Fdev, double dt) {
   f_eval = Fdev;
   kt.begin(SC_KT_RESPONSE, st);
   launch_mp_response(s, mc, dt, d_ill, sub, st);
+  response_clean = false;
   kt.end(SC_KT_RESPONSE, N, st);
   kt.begin(SC_KT_REDUCE, st);
   launch_pav_partial(mp.P, N, partial, st);
@@ -662,6 +663,12 @@ void Rve::tangent() {
   kt.flush();
 }
 
+// whether an evaluation's forward z pass and convolution are one kernel: pencil
+// lengths that fit it, and an imaginary xi (continuous, central differences)
+bool Rve::fused_gamma() const {
+  return desc.grid_num.derivative != 2 && (use32 ? fft32.fused_gamma_available() : fft.fused_gamma_available());
+}
+
 GammaHost Rve::gamma_host(bool do_gamma) const {
   GammaHost g;
   for (int p = 0; p < 3; ++p) {
@@ -691,7 +698,7 @@ void Rve::launch_residual(const double* Fdev, void* rdev) {
   MpState s = mp;
   s.F = const_cast<double*>(Fdev);  // read only
   kt.begin(SC_KT_RESPONSE, st);
-  launch_mp_response(s, mc, delta_t, d_ill, sub, st);
+  launch_mp_response(s, mc, delta_t, d_ill, sub, st, !fused_gamma());
   kt.end(SC_KT_RESPONSE, N, st);
   if (!xsums) {  // else the forward transform gives the P sums
     kt.begin(SC_KT_REDUCE, st);
@@ -724,6 +731,27 @@ void Rve::launch_spectral(void* rdev) {
     launch_bc_aim(small + SM_SUMS, S, Rrm, wgt, 1, small + SM_AIM, st);
   };
   double* rowsum = xsums ? d_rowsum : nullptr;
+  if (fused_gamma()) {
+    // eight launches an evaluation instead of fourteen: the forward z pass
+    // and the convolution in one kernel, the small sums in blocks of the y
+    // passes
+    const RowSumItem sums{d_rowsum, (int64_t)cells[1] * cells[2], small + SM_SUMS};
+    auto stages = [&](auto& plan, auto* sp, auto* r) {
+      kt.begin(SC_KT_FFT_FWD, st);
+      plan.forward_xy(mp.P, sp, st, d_rowsum, sums);
+      kt.end(SC_KT_FFT_FWD, N, st);
+      kt.begin(SC_KT_GAMMA, st);
+      const int nb = launch_zgamma(plan, sp, gamma_host(true), d_xi_tab, small + SM_SUMS, S, Rrm, wgt, partial, st);
+      kt.end(SC_KT_GAMMA, K, st);
+      kt.begin(SC_KT_FFT_BWD, st);
+      plan.backward_fin(sp, r, st, FinishItem{partial, nb, small + SM_SUMS, SM_DIV - SM_SUMS, kt.on ? 13 : 11, h_scal,
+                                             d_ill, mp.repivot});
+      kt.end(SC_KT_FFT_BWD, N, st);
+    };
+    if (use32) stages(fft32, spec32, static_cast<float*>(rdev));
+    else stages(fft, spec, static_cast<double*>(rdev));
+    return;
+  }
   if (use32) {  // FP32 transforms and spectrum from the FP64 P; r out in FP32 (exactly the transform's values)
     kt.begin(SC_KT_FFT_FWD, st);
     fft32.forward(mp.P, spec32, 9, st, 0, rowsum);
@@ -835,6 +863,9 @@ void Rve::form_residual(const double* Fdev, void* rdev) {
   if (total_iter - iter_base <= snes_iter) total_iter += 1;
   const bool reused = reuse_response;
   reuse_response = false;
+  // a fused evaluation clears the response's flags for the next one; others leave them as they are
+  if (!reused && !batch && fused_gamma() && !response_clean) launch_response_reset(mp.repivot, d_ill, st);
+  response_clean = !batch && fused_gamma();
   if (reused) {
     launch_spectral(rdev);
   } else if (batch) {

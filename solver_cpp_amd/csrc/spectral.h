@@ -9,6 +9,26 @@ namespace sca {
 
 constexpr int MAX_RED_VEC = 96;
 
+// the 9 sums of a field from its x-pass row sums: out[q] = sum of the rows
+// q * nrow .. (q + 1) * nrow - 1, in a fixed order (one block per q)
+struct RowSumItem {
+  const double* rowsum;
+  int64_t nrow;  // rows per component (Ny x Nz)
+  double* out;
+};
+// end of an evaluation: scal[div] = sum of the nb partials (as
+// launch_final_reduce), the n scalars to host (pinned), *ill and repivot[0]
+// cleared
+struct FinishItem {
+  const double* partial;
+  int nb;
+  double* scal;
+  int div, n;
+  double* host;
+  int* ill;
+  int* repivot;
+};
+
 // 3D FFT of `ncomp` real planes (N each) <-> half spectra (K complex each)
 template <typename T>
 struct cpx;
@@ -42,12 +62,23 @@ struct FftPlan {
   void backward(T* spec, TO* real, int ncomp, double scale, hipStream_t st,
                 int set_comp = 0) const;  // spec is clobbered
   void strided_passes(void* spec, int ncomp, int sign, hipStream_t st) const;
+  // The transforms of a 9-component field around launch_zgamma, which holds
+  // the forward z pass: x and y forward, with the field's sums (SumSide)
+  // formed in the y pass; the inverse (scale 1), with the end of the
+  // evaluation in its y pass.  Available when x and y have pencil kernels and z's fit.
+  bool fused_gamma_available() const;
+  void forward_xy(const double* real, T* spec, hipStream_t st, double* rowsum, const RowSumItem& sums) const;
+  template <typename TO>
+  void backward_fin(T* spec, TO* real, hipStream_t st, const FinishItem& fin) const;
 
  private:
   int shape(int axis) const;
   void x_pass_fwd(const void* real, bool real_is_double, cpx<T>* S, int ncomp, int shp, hipStream_t st,
                   int set_comp, double* rowsum = nullptr) const;
-  void strided_pass(cpx<T>* S, int ncomp, int sign, int axis, int shp, hipStream_t st) const;
+  void strided_pass(cpx<T>* S, int ncomp, int sign, int axis, int shp, hipStream_t st,
+                    const RowSumItem* sum = nullptr, const FinishItem* fin = nullptr) const;
+  template <typename TO>
+  void x_pass_bwd(const cpx<T>* S, TO* real, int ncomp, T scale, int shp, hipStream_t st, int set_comp) const;
 };
 
 struct GammaHost {
@@ -62,6 +93,14 @@ int gamma_blocks(int64_t K);
 template <typename T>
 void launch_gamma_div(T* spec, int64_t K, const GammaHost& g, const double* d_aim, const double* d_xi_tab,
                       double* div_partial, hipStream_t st);
+
+// z forward and launch_gamma_div with the aim of launch_bc_aim(sums, S, R, wgt,
+// 1) in one kernel (plan.fused_gamma_available(), derivative 0 or
+// 1): the spectrum has the bits of the separate launches.  Returns the number
+// of divergence partials (at most gamma_blocks(K)).
+template <typename T>
+int launch_zgamma(const FftPlan<T>& plan, T* spec, const GammaHost& g, const double* d_xi_tab, const double* sums,
+                  const double S[81], const double R[9], double wgt, double* div_partial, hipStream_t st);
 
 // base_update_coords: F_hat -> u_hat (planes 0..2) and the 9 sums of F;
 // then node / cell-centre coordinates from u (3 planes of N) and the sums
@@ -95,13 +134,6 @@ void tangent_select_norms(const double* n2, int64_t N, double* pv, long long* pi
 void launch_bc_aim(const double* sums, const double S[81], const double R[9], double wgt, int rotate, double* aim,
                    hipStream_t st);
 void launch_final_reduce(const double* partial, int nvec, int nb, double* out, hipStream_t st);
-// the 9 sums of a field from its x-pass row sums: out[q] = sum of the rows
-// q * nrow .. (q + 1) * nrow - 1, in a fixed order (one block per q)
-struct RowSumItem {
-  const double* rowsum;
-  int64_t nrow;  // rows per component (Ny x Nz)
-  double* out;
-};
 void launch_rowsum_reduce(const RowSumItem& item, hipStream_t st);
 
 void launch_fwd_field(const double* last, const double* rate, double dt, double* out, int64_t n, hipStream_t st);

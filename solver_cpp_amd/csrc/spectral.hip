@@ -36,6 +36,11 @@ __device__ __forceinline__ cpx<T> csub(cpx<T> a, cpx<T> b) {
   return {a.x - b.x, a.y - b.y};
 }
 
+// side job of a strided pass (fft_pencil.h): none
+struct NoSide {
+  static constexpr int blocks() { return 0; }
+};
+
 }  // namespace sca
 #include "fft_pencil.h"
 namespace sca {
@@ -425,6 +430,186 @@ __global__ void __launch_bounds__(256) gamma_div_batch_kernel(const GammaBatchEn
   gamma_div_block<T>(reinterpret_cast<cpx<T>*>(e.data), K, e.g, e.div_partial, blockIdx.x, red);
 }
 
+
+// The same with the forward z transforms in one kernel (pencil::zop_block),
+// for derivatives whose xi is imaginary (continuous and central differences):
+// every product with a real part of xi is then a zero, and the convolution is
+// real arithmetic on the two parts of P_hat.  Each value has the roundings of
+// gamma_div_block's (where its complex products keep the compiler from fusing
+// a multiplication with the next addition, so do the rounded products here),
+// so P_hat has its bits; only the divergence sum is added in another order.
+// Bound: HBM (two passes over the spectrum instead of four) and, at 128^3 in
+// single precision, the one block a CU has registers for.  At 128^3: 92 us
+// (3.3 TB/s) after 54 + 52 apart, without the XCD order 112; at 64^3 17 after
+// 10 + 9; at 16^3 8 after 5 + 5 and the two launches between them.
+__device__ __forceinline__ double rnd_mul(double a, double b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+struct BcArgs {
+  double S[81];  // (i,j,k,l) column-major
+  double R[9];   // row-major
+  double wgt;
+  int rotate;
+};
+__device__ __forceinline__ void bc_aim_body(const double* sums, const BcArgs& b, double* aim);
+
+template <typename T>
+struct GammaOp {
+  const GammaArgs& g;
+  int64_t K, nq;
+  double* div_partial;
+  unsigned blk;
+  double* red;        // one double per wave
+  const double* aim;  // LDS, block 0
+  mutable double contrib;
+  // component c of the wavevector: from v[c * stride] to out[c * K]
+  __device__ __forceinline__ void point(int64_t q, int z, const cpx<T>* v, int stride, cpx<T>* out) const {
+    const int i = (int)(q % g.nr), y = (int)(q / g.nr);
+    double xi[3];
+    if (g.derivative == 0) {
+      const int ks[3] = {i, (y > g.Ny / 2) ? y - g.Ny : y, (z > g.Nz / 2) ? z - g.Nz : z};
+      const int idx[3] = {i, y, z};
+      const int cells[3] = {g.Nx, g.Ny, g.Nz};
+      const double TAU = 6.283185307179586476925286766559;
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        const bool nyq = (cells[p] % 2 == 0) && (idx[p] == cells[p] / 2);
+        xi[p] = nyq ? 0.0 : TAU * ks[p] / g.size[p];
+      }
+    } else {
+      const int64_t kk = q + nq * z;
+#pragma unroll
+      for (int p = 0; p < 3; ++p) xi[p] = g.xi_tab[6 * kk + 2 * p + 1];
+    }
+    double Px[9], Py[9];
+#pragma unroll
+    for (int c = 0; c < 9; ++c) {
+      const cpx<T> a = v[c * stride];
+      Px[c] = (double)a.x;
+      Py[c] = (double)a.y;
+    }
+    // divergence: |P_hat . conj(xi) L/L_scaled|^2, weight 2 for 0 < i < nr-1
+    {
+      double s = 0.0;
+#pragma unroll
+      for (int m = 0; m < 3; ++m) {
+        double re = 0.0, im = 0.0;
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+          const double k = xi[n] * g.rescale[n];
+          re += Py[m + 3 * n] * k;
+          im -= Px[m + 3 * n] * k;
+        }
+        s += re * re + im * im;
+      }
+      contrib += ((i > 0 && i < g.nr - 1) ? 2.0 : 1.0) * s;
+    }
+    if (q == 0 && z == 0) {
+#pragma unroll
+      for (int c = 0; c < 9; ++c) out[c * K] = {(T)aim[c], (T)0};
+      return;
+    }
+    // Z(l,m) = sum_no C_ref(l,n,m,o) dy(n,o), dy = conj(-xi_n) xi_o
+    double dy[9], Z[9];
+#pragma unroll
+    for (int n = 0; n < 3; ++n)
+#pragma unroll
+      for (int o = 0; o < 3; ++o) dy[3 * n + o] = -rnd_mul(xi[n], xi[o]);
+#pragma unroll
+    for (int l = 0; l < 3; ++l)
+#pragma unroll
+      for (int m = 0; m < 3; ++m) {
+        double s = 0.0;
+#pragma unroll
+        for (int n = 0; n < 3; ++n)
+#pragma unroll
+          for (int o = 0; o < 3; ++o) s = __builtin_fma(g.C_ref[27 * l + 9 * n + 3 * m + o], dy[3 * n + o], s);
+        Z[3 * l + m] = s;
+      }
+    // cofactors, differences of rounded products
+    double cof[9];
+    cof[0] = rnd_mul(Z[4], Z[8]) - rnd_mul(Z[5], Z[7]);
+    cof[3] = rnd_mul(Z[5], Z[6]) - rnd_mul(Z[3], Z[8]);
+    cof[6] = rnd_mul(Z[3], Z[7]) - rnd_mul(Z[4], Z[6]);
+    cof[1] = rnd_mul(Z[2], Z[7]) - rnd_mul(Z[1], Z[8]);
+    cof[4] = rnd_mul(Z[0], Z[8]) - rnd_mul(Z[2], Z[6]);
+    cof[7] = rnd_mul(Z[1], Z[6]) - rnd_mul(Z[0], Z[7]);
+    cof[2] = rnd_mul(Z[1], Z[5]) - rnd_mul(Z[2], Z[4]);
+    cof[5] = rnd_mul(Z[2], Z[3]) - rnd_mul(Z[0], Z[5]);
+    cof[8] = rnd_mul(Z[0], Z[4]) - rnd_mul(Z[1], Z[3]);
+    const double det = (rnd_mul(Z[0], cof[0]) + rnd_mul(Z[1], cof[3])) + rnd_mul(Z[2], cof[6]);
+    const double detRe = Z[0] * (Z[4] * Z[8] - Z[5] * Z[7]) - Z[1] * (Z[3] * Z[8] - Z[5] * Z[6]) +
+                         Z[2] * (Z[3] * Z[7] - Z[4] * Z[6]);
+    if (!(fabs(detRe) > 1e-16)) {
+#pragma unroll
+      for (int c = 0; c < 9; ++c) out[c * K] = {(T)0, (T)0};
+      return;
+    }
+    const double idet = det / rnd_mul(det, det);
+    // w_n = sum_o P(n,o) conj(-xi_o); u = Z^-1 w; out(l,m) = u_l xi_m
+    double wx[3], wy[3];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      double sx = 0.0, sy = 0.0;
+#pragma unroll
+      for (int o = 0; o < 3; ++o) {
+        sx = sx - rnd_mul(Py[n + 3 * o], xi[o]);
+        sy = sy + rnd_mul(Px[n + 3 * o], xi[o]);
+      }
+      wx[n] = sx;
+      wy[n] = sy;
+    }
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+      double ux = 0.0, uy = 0.0;
+#pragma unroll
+      for (int n = 0; n < 3; ++n) {
+        const double a = rnd_mul(cof[3 * l + n], idet);
+        ux = ux + rnd_mul(a, wx[n]);
+        uy = uy + rnd_mul(a, wy[n]);
+      }
+#pragma unroll
+      for (int m = 0; m < 3; ++m) out[(l + 3 * m) * K] = {(T)(-rnd_mul(uy, xi[m])), (T)rnd_mul(ux, xi[m])};
+    }
+  }
+  // the block's divergence sum: lanes of a wave, then the waves in order
+  __device__ __forceinline__ void finish() const {
+    double s = contrib;
+    for (int w = 32; w > 0; w >>= 1) {
+      const double o = __shfl_xor(s, w);
+      if ((threadIdx.x ^ w) < blockDim.x) s += o;  // the last wave may be partly empty
+    }
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const int nw = ((int)blockDim.x + 63) >> 6;
+      double t = red[0];
+      for (int w = 1; w < nw; ++w) t += red[w];
+      div_partial[blk] = t;
+    }
+  }
+};
+
+template <typename T, int N>
+__global__ void __launch_bounds__((pencil::ZShape<T, N>::THREADS))
+    zgamma_kernel(cpx<T>* data, int64_t K, GammaArgs g, const double* sums, BcArgs bc, const cpx<T>* tw,
+                  double* div_partial) {
+  using Z = pencil::ZShape<T, N>;
+  __shared__ cpx<T> lds[Z::ENTRIES];
+  __shared__ double red[16], aim[9];
+  const int64_t nq = (int64_t)g.nr * g.Ny;
+  // neighbouring blocks read and write the two halves of a cache line: they
+  // run on the same XCD (blocks go to the 8 of them in turn)
+  const unsigned blk = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (blk * Z::W >= nq) return;
+  // the convolution's mean (block 0 holds wavevector 0), ready after the first
+  // barrier of the transforms
+  if (blk == 0 && threadIdx.x == 0) bc_aim_body(sums, bc, aim);
+  const GammaOp<T> op{g, K, nq, div_partial, blk, red, aim, 0.0};
+  pencil::zop_block<T, N>(data, K, nq, blk, tw, op, lds);
+}
+
 // ---------------------------------------------------------------------------
 // Cell and node coordinates (base_update_coords, mech_base.cpp:45-154)
 // ---------------------------------------------------------------------------
@@ -748,6 +933,65 @@ __global__ void __launch_bounds__(256) rowsum_reduce_batch_kernel(const RowSumIt
   rowsum_block(tab[blockIdx.y], blockIdx.x, red);
 }
 
+// Side jobs of the y passes (fft_pencil.h).  256 virtual threads whatever the
+// block size, so that the sums have the bits of the kernels they stand for.
+__device__ __forceinline__ void side_tree(double* red) {
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    for (int v = threadIdx.x; v < w; v += blockDim.x) red[v] += red[v + w];
+    __syncthreads();
+  }
+}
+// rowsum_reduce_kernel: the nine sums of a field from its x-pass row sums
+struct SumSide {
+  RowSumItem e;
+  static constexpr int blocks() { return 9; }
+  __device__ __forceinline__ void run(int q, double* red) const {
+    const double* r = e.rowsum + (int64_t)q * e.nrow;
+    for (int v = threadIdx.x; v < 256; v += blockDim.x) {
+      double s = 0.0;
+      constexpr int U = 16;
+      for (int64_t t0 = v; t0 < e.nrow; t0 += 256 * U) {
+        double x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = (t0 + 256 * u < e.nrow) ? r[t0 + 256 * u] : 0.0;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (t0 + 256 * u < e.nrow) s += x[u];
+      }
+      red[v] = s;
+    }
+    side_tree(red);
+    if (threadIdx.x == 0) e.out[q] = red[0];
+  }
+};
+// final_reduce_kernel of the divergence partials, then the evaluation's n
+// scalars (scal, the divergence sum at div) to pinned host memory; the flag
+// and the pivoting list's count are cleared for the next evaluation
+struct FinishSide {
+  FinishItem e;
+  static constexpr int blocks() { return 1; }
+  __device__ __forceinline__ void run(int, double* red) const {
+    for (int v = threadIdx.x; v < 256; v += blockDim.x) {
+      double s = 0.0;
+      for (int t = v; t < e.nb; t += 256) s += e.partial[t];
+      red[v] = s;
+    }
+    side_tree(red);
+    if (threadIdx.x < (unsigned)e.n) {
+      const double x = (int)threadIdx.x == e.div ? red[0] : e.scal[threadIdx.x];
+      if ((int)threadIdx.x == e.div) e.scal[threadIdx.x] = x;
+      e.host[threadIdx.x] = x;
+      __threadfence_system();  // read by the host once the stream is done
+    }
+    __syncthreads();  // the flag is among the scalars
+    if (threadIdx.x == 0) {
+      *e.ill = 0;
+      e.repivot[0] = 0;
+    }
+  }
+};
+
 // copies of a batch (gathers and scatters between RVE buffers and a group's
 // contiguous arena): blockIdx.y is the entry
 __global__ void __launch_bounds__(256) copy_batch_kernel(const BatchCopy* __restrict__ tab) {
@@ -1027,22 +1271,31 @@ static bool pencil_x_c2r(int n, const cpx<T>* in, TO* out, int64_t rows, int64_t
   }
 }
 
+// side jobs run in blocks of the pass (SumSide: forward, FinishSide: inverse)
 template <typename T>
 static bool pencil_strided(int n, int sign, cpx<T>* data, int ni, unsigned no, int d1, int64_t s1, int64_t s2,
-                           int64_t es, const cpx<T>* tw, int bs, hipStream_t st) {
+                           int64_t es, const cpx<T>* tw, int bs, hipStream_t st, const RowSumItem* sum = nullptr,
+                           const FinishItem* fin = nullptr) {
   switch (n) {
 #define SCA_CASE(N)                                                                                          \
   case N: {                                                                                                  \
     using S = pencil::Shape<T, N>;                                                                              \
     const int P = bs / S::TP;                                                                                \
     const int64_t npen = (int64_t)ni * no;                                                                   \
-    const dim3 grid((unsigned)((npen + P - 1) / P));                                                         \
-    if (sign < 0)                                                                                            \
-      hipLaunchKernelGGL((pencil::strided_kernel<T, N, -1>), grid, dim3(bs), (pencil_lds<T, N>(bs)), st, data, \
-                         ni, npen, d1, s1, s2, es, tw);                                                      \
+    const unsigned nb = (unsigned)((npen + P - 1) / P + 7) / 8 * 8;                                          \
+    const size_t lds = std::max<size_t>(pencil_lds<T, N>(bs), sum || fin ? 256 * sizeof(double) : 0);        \
+    if (sign < 0 && sum)                                                                                     \
+      hipLaunchKernelGGL((pencil::strided_kernel<T, N, -1, SumSide>), dim3(nb + SumSide::blocks()), dim3(bs), lds, \
+                         st, data, ni, npen, d1, s1, s2, es, tw, SumSide{*sum});                             \
+    else if (sign < 0)                                                                                       \
+      hipLaunchKernelGGL((pencil::strided_kernel<T, N, -1, NoSide>), dim3(nb), dim3(bs), lds, st, data, ni, npen, \
+                         d1, s1, s2, es, tw, NoSide{});                                                      \
+    else if (fin)                                                                                            \
+      hipLaunchKernelGGL((pencil::strided_kernel<T, N, 1, FinishSide>), dim3(nb + FinishSide::blocks()),     \
+                         dim3(bs), lds, st, data, ni, npen, d1, s1, s2, es, tw, FinishSide{*fin});           \
     else                                                                                                     \
-      hipLaunchKernelGGL((pencil::strided_kernel<T, N, 1>), grid, dim3(bs), (pencil_lds<T, N>(bs)), st, data,  \
-                         ni, npen, d1, s1, s2, es, tw);                                                      \
+      hipLaunchKernelGGL((pencil::strided_kernel<T, N, 1, NoSide>), dim3(nb), dim3(bs), lds, st, data, ni, npen, \
+                         d1, s1, s2, es, tw, NoSide{});                                                      \
     return true;                                                                                             \
   }
     SCA_PENCIL_LENGTHS(SCA_CASE)
@@ -1149,7 +1402,8 @@ void FftPlan<T>::forward(const TI* real, T* spec, int ncomp, hipStream_t st, int
 }
 
 template <typename T>
-void FftPlan<T>::strided_pass(cpx<T>* S, int ncomp, int sign, int axis, int shp, hipStream_t st) const {
+void FftPlan<T>::strided_pass(cpx<T>* S, int ncomp, int sign, int axis, int shp, hipStream_t st,
+                              const RowSumItem* sum, const FinishItem* fin) const {
   const int Ny = cells[1], Nz = cells[2];
   const int n = cells[axis];
   // y: pencils (c, z, i) with element stride nr; z: pencils (c, y, i), stride nr*Ny
@@ -1158,7 +1412,8 @@ void FftPlan<T>::strided_pass(cpx<T>* S, int ncomp, int sign, int axis, int shp,
   const int64_t s2 = axis == 1 ? (int64_t)nr * Ny : (int64_t)nr;
   const int64_t es = axis == 1 ? (int64_t)nr : (int64_t)nr * Ny;
   const cpx<T>* t = reinterpret_cast<const cpx<T>*>(tw[axis]);
-  if (!pencil_strided<T>(n, sign, S, nr, no, d1, K, s2, es, t, shp, st)) {
+  if (!pencil_strided<T>(n, sign, S, nr, no, d1, K, s2, es, t, shp, st, sum, fin)) {
+    if (sum || fin) throw std::runtime_error("FFT: side job on a generic pass");
     FftPassDesc d = make_desc(n, sign);
     dim3 grid((nr + shp - 1) / shp, no);
     hipLaunchKernelGGL(fft_strided<T>, grid, dim3(256), 2 * (size_t)shp * (n + 1) * sizeof(cpx<T>), st, S, nr, d1, K,
@@ -1174,25 +1429,61 @@ void FftPlan<T>::strided_passes(void* Sv, int ncomp, int sign, hipStream_t st) c
   if (cells[2] > 1) strided_pass(S, ncomp, sign, 2, shape(2), st);
 }
 
+// lengths whose z pencils of nine components fit a block (pencil::ZShape)
+#define SCA_ZGAMMA_LENGTHS(X) X(8) X(16) X(32) X(64) X(128) X(12) X(24) X(48) X(96) X(18) X(36) X(72) X(27)
+
+template <typename T>
+bool FftPlan<T>::fused_gamma_available() const {
+  if (!row_sums_available() || cells[1] < 2 || pencil_tp<T>(cells[1]) == 0) return false;
+  switch (cells[2]) {
+#define SCA_CASE(N) \
+  case N: return pencil::ZShape<T, N>::fits;
+    SCA_ZGAMMA_LENGTHS(SCA_CASE)
+#undef SCA_CASE
+    default: return false;
+  }
+}
+
+template <typename T>
+void FftPlan<T>::forward_xy(const double* real, T* spec, hipStream_t st, double* rowsum, const RowSumItem& sums) const {
+  cpx<T>* S = reinterpret_cast<cpx<T>*>(spec);
+  x_pass_fwd(real, true, S, 9, shape(0), st, 0, rowsum);
+  strided_pass(S, 9, -1, 1, shape(1), st, &sums, nullptr);
+}
+
+template <typename T>
+template <typename TO>
+void FftPlan<T>::backward_fin(T* spec, TO* real, hipStream_t st, const FinishItem& fin) const {
+  cpx<T>* S = reinterpret_cast<cpx<T>*>(spec);
+  strided_pass(S, 9, +1, 1, shape(1), st, nullptr, &fin);
+  strided_pass(S, 9, +1, 2, shape(2), st);
+  x_pass_bwd(S, real, 9, (T)1, shape(0), st, 0);
+}
+
 template <typename T>
 template <typename TO>
 void FftPlan<T>::backward(T* spec, TO* real, int ncomp, double scale, hipStream_t st, int set_comp) const {
-  const int Nx = cells[0], Ny = cells[1], Nz = cells[2];
+  const int Ny = cells[1], Nz = cells[2];
   cpx<T>* S = reinterpret_cast<cpx<T>*>(spec);
   const int64_t set_rows = (int64_t)(set_comp > 0 ? set_comp : ncomp) * Ny * Nz;
   if (((int64_t)ncomp * Ny * Nz) % set_rows != 0) throw std::runtime_error("FFT: components not a multiple of the field size");
   strided_passes(S, ncomp, +1, st);
-  const int shp = shape(0);
-  if (pencil_x_c2r<T, TO>(Nx, S, real, (int64_t)ncomp * Ny * Nz, set_rows, reinterpret_cast<const cpx<T>*>(tw[0]),
-                          (T)scale, shp, st)) {
-    SCA_HIP(hipGetLastError());
-    return;
-  }
-  FftPassDesc d = make_desc(Nx, +1);
+  x_pass_bwd(S, real, ncomp, (T)scale, shape(0), st, set_comp);
+}
+
+template <typename T>
+template <typename TO>
+void FftPlan<T>::x_pass_bwd(const cpx<T>* S, TO* real, int ncomp, T scale, int shp, hipStream_t st,
+                            int set_comp) const {
+  const int Nx = cells[0], Ny = cells[1], Nz = cells[2];
   const int64_t rows = (int64_t)ncomp * Ny * Nz;
-  const size_t sh = 2 * (size_t)shp * Nx * sizeof(cpx<T>);
-  hipLaunchKernelGGL((fft_x_c2r<T, TO>), dim3(nblk(rows, shp)), dim3(256), sh, st, S, real, rows, d,
-                     reinterpret_cast<const cpx<T>*>(tw[0]), (T)scale, shp);
+  const int64_t set_rows = (int64_t)(set_comp > 0 ? set_comp : ncomp) * Ny * Nz;
+  const cpx<T>* t0 = reinterpret_cast<const cpx<T>*>(tw[0]);
+  if (!pencil_x_c2r<T, TO>(Nx, S, real, rows, set_rows, t0, scale, shp, st)) {
+    FftPassDesc d = make_desc(Nx, +1);
+    const size_t sh = 2 * (size_t)shp * Nx * sizeof(cpx<T>);
+    hipLaunchKernelGGL((fft_x_c2r<T, TO>), dim3(nblk(rows, shp)), dim3(256), sh, st, S, real, rows, d, t0, scale, shp);
+  }
   SCA_HIP(hipGetLastError());
 }
 
@@ -1289,6 +1580,8 @@ template void FftPlan<float>::forward<double>(const double*, float*, int, hipStr
 template void FftPlan<float>::backward<double>(float*, double*, int, double, hipStream_t, int) const;
 template void FftPlan<float>::forward<float>(const float*, float*, int, hipStream_t, int, double*) const;
 template void FftPlan<float>::backward<float>(float*, float*, int, double, hipStream_t, int) const;
+template void FftPlan<double>::backward_fin<double>(double*, double*, hipStream_t, const FinishItem&) const;
+template void FftPlan<float>::backward_fin<float>(float*, float*, hipStream_t, const FinishItem&) const;
 
 static GammaArgs gamma_args(const GammaHost& gh, const double* d_xi_tab, const double* d_aim) {
   GammaArgs g;
@@ -1321,6 +1614,46 @@ template void launch_gamma_div<double>(double*, int64_t, const GammaHost&, const
 template void launch_gamma_div<float>(float*, int64_t, const GammaHost&, const double*, const double*, double*,
                                       hipStream_t);
 int gamma_blocks(int64_t K) { return (int)((K + 255) / 256); }
+
+static BcArgs bc_args(const double S[81], const double R[9], double wgt, int rotate) {
+  BcArgs b;
+  for (int i = 0; i < 81; ++i) b.S[i] = S[i];
+  for (int i = 0; i < 9; ++i) b.R[i] = R[i];
+  b.wgt = wgt;
+  b.rotate = rotate;
+  return b;
+}
+
+template <typename T>
+int launch_zgamma(const FftPlan<T>& plan, T* spec, const GammaHost& gh, const double* d_xi_tab, const double* sums,
+                  const double S[81], const double R[9], double wgt, double* div_partial, hipStream_t st) {
+  if (gh.derivative == 2 || !gh.do_gamma) throw std::runtime_error("fused Gamma convolution: unsupported form");
+  const GammaArgs g = gamma_args(gh, d_xi_tab, nullptr);
+  const BcArgs bc = bc_args(S, R, wgt, 1);
+  const int64_t nq = (int64_t)plan.nr * plan.cells[1];
+  const cpx<T>* tw = reinterpret_cast<const cpx<T>*>(plan.tw[2]);
+  int nb = 0;
+  switch (plan.cells[2]) {
+#define SCA_CASE(N)                                                                                                 \
+  case N:                                                                                                           \
+    if constexpr (pencil::ZShape<T, N>::fits) {                                                                     \
+      nb = (int)((nq + pencil::ZShape<T, N>::W - 1) / pencil::ZShape<T, N>::W);                                     \
+      hipLaunchKernelGGL((zgamma_kernel<T, N>), dim3((nb + 7) / 8 * 8), dim3(pencil::ZShape<T, N>::THREADS), 0, st,               \
+                         reinterpret_cast<cpx<T>*>(spec), plan.K, g, sums, bc, tw, div_partial);                    \
+    }                                                                                                               \
+    break;
+    SCA_ZGAMMA_LENGTHS(SCA_CASE)
+#undef SCA_CASE
+    default: break;
+  }
+  if (nb == 0) throw std::runtime_error("fused Gamma convolution: unsupported z length");
+  SCA_HIP(hipGetLastError());
+  return nb;
+}
+template int launch_zgamma<double>(const FftPlan<double>&, double*, const GammaHost&, const double*, const double*,
+                                   const double*, const double*, double, double*, hipStream_t);
+template int launch_zgamma<float>(const FftPlan<float>&, float*, const GammaHost&, const double*, const double*,
+                                  const double*, const double*, double, double*, hipStream_t);
 
 void launch_coords_uhat(double* spec, int64_t K, const GammaHost& gh, const double* d_xi_tab, double* fsum,
                         hipStream_t st) {
@@ -1543,12 +1876,6 @@ static void select_from_extremes(const double* n2, int64_t N, double* pv, long l
 }
 // dF_aim on the device: P_av = wgt * sums (rotated R P R^T when rotating),
 // dF = S : P_av in the load frame, aim = R^T dF R in the field frame (active)
-struct BcArgs {
-  double S[81];  // (i,j,k,l) column-major
-  double R[9];   // row-major
-  double wgt;
-  int rotate;
-};
 struct BcBatchEntry {
   const double* sums;
   BcArgs b;
@@ -1593,12 +1920,7 @@ __global__ void bc_aim_batch_kernel(const BcBatchEntry* __restrict__ tab, int n)
 
 void launch_bc_aim(const double* sums, const double S[81], const double R[9], double wgt, int rotate, double* aim,
                    hipStream_t st) {
-  BcArgs b;
-  for (int i = 0; i < 81; ++i) b.S[i] = S[i];
-  for (int i = 0; i < 9; ++i) b.R[i] = R[i];
-  b.wgt = wgt;
-  b.rotate = rotate;
-  hipLaunchKernelGGL(bc_aim_kernel, dim3(1), dim3(64), 0, st, sums, b, aim);
+  hipLaunchKernelGGL(bc_aim_kernel, dim3(1), dim3(64), 0, st, sums, bc_args(S, R, wgt, rotate), aim);
   SCA_HIP(hipGetLastError());
 }
 

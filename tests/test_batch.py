@@ -12,8 +12,8 @@ import pytest
 
 from conftest import GOLDEN, PRODUCT_SO, tail_close
 from solver_cpp_amd.capi import Library
-from solver_cpp_amd.geometry import EXAMPLE_NUMERICS
-from solver_cpp_amd.rve import tension_x
+from solver_cpp_amd.geometry import EXAMPLE_NUMERICS, uniform_orientations, voronoi
+from solver_cpp_amd.rve import RveSpec, tension_x
 from solver_cpp_amd.serving import Server, batched_specs
 
 pytestmark = pytest.mark.gpu
@@ -73,6 +73,34 @@ def test_batched_odd_grid_equals_alone(lib):
         for a, b in zip(a_job, b_job):
             assert a.status == 0 and b.status == 0
             assert (a.iterations, a.evaluations) == (b.iterations, b.evaluations)
+            np.testing.assert_array_equal(np.array(a.P_av), np.array(b.P_av))
+    for x, y in zip(fa, fb):
+        for k in x:
+            np.testing.assert_array_equal(x[k], y[k], err_msg=k)
+
+
+@pytest.mark.parametrize("cells,derivative,precision", [
+    ((8, 8, 8), 1, 0),        # smallest z pencil, central differences
+    ((18, 27, 12), 0, 0),   # an odd y, (x, y) frequencies no multiple of a block's
+    ((8, 12, 18), 1, 1), ((12, 8, 27), 0, 1), ((27, 8, 36), 0, 0),
+    ((8, 8, 72), 0, 1), ((8, 16, 96), 1, 0), ((8, 8, 128), 0, 0), ((12, 8, 128), 1, 1),
+    ((16, 8, 20), 0, 0),      # no z pencil: separate launches
+])
+def test_alone_evaluation_equals_joint_launches(lib, cells, derivative, precision):
+    """A job alone takes its forward z transforms and the convolution in one
+    kernel and its sums in blocks of the y passes; a batch runs them as
+    separate launches.  Two increments of a four-grain RVE give bitwise the same
+    counts, <P> and fields either way."""
+    size = [1e-5 * c / 8 for c in cells]
+    specs = [(RveSpec(lib, cells, size, voronoi(cells, size, 4, 5 + i), uniform_orientations(4, 6 + i),
+                      derivative=derivative, precision=precision, **EXAMPLE_NUMERICS), None) for i in range(2)]
+    loads = [[tension_x(t=1.0, N=2)] for _ in specs]
+    print(f"[alone] {cells} derivative {derivative} precision {precision}", flush=True)
+    alone, fa, _ = _run(lib, specs, loads, 2, batched=False, workers=1)
+    batch, fb, _ = _run(lib, specs, loads, 2, batched=True, workers=2)
+    for a_job, b_job in zip(alone, batch):
+        for a, b in zip(a_job, b_job):
+            assert (a.status, a.iterations, a.evaluations) == (b.status, b.iterations, b.evaluations)
             np.testing.assert_array_equal(np.array(a.P_av), np.array(b.P_av))
     for x, y in zip(fa, fb):
         for k in x:
