@@ -53,7 +53,17 @@ struct FftPassDesc {
   int nrad;        // number of radix passes
   int rad[16];     // radices 4, 2, 3, 5, 7, 11, 13
   int sign;        // -1 forward, +1 inverse
+  // quotients by launch constants: quot_of(x, inv(d)) = x / d
+  unsigned inv_n, inv_nr, inv_pb;      // n, n / 2 + 1, pencils per block
+  unsigned inv_nb[16], inv_ns[16];     // butterflies and span of each pass
 };
+// x / d for x d < 2^32 (a block's work items and lengths are below 2^16):
+// with inv = floor(2^32 / d) + 1 the product exceeds x 2^32 / d by less than
+// x < 2^32 / d.  inv = 0 stands for d = 1.  A division in hardware is some 30
+// instructions, three to an item of each pass: x passes of 9 x 108 x 96 x 72,
+// r2c / c2r: 97 / 100 us with them, 75 / 78 with the quotients.
+static unsigned inv_of(int d) { return d <= 1 ? 0u : (unsigned)(((uint64_t)1 << 32) / (unsigned)d + 1); }
+__device__ __forceinline__ int quot_of(int x, unsigned inv) { return inv ? (int)__umulhi((unsigned)x, inv) : x; }
 
 // R-point DFT in registers for R = 2, 3, 4; generic R by direct summation
 // with the length-n table (exp(sign 2 pi i q k / R) = tw[q k n / R mod n]).
@@ -102,12 +112,12 @@ __device__ __forceinline__ void dft_r(cpx<T>* v, int sign, const cpx<T>* tw, int
 // one Stockham radix-R pass over PB pencils (a -> b)
 template <typename T, int R>
 __device__ __forceinline__ void stockham_pass(const cpx<T>* a, cpx<T>* b, int PB, int ps, int n, int Ns, int sign,
-                                              const cpx<T>* tw) {
+                                              const cpx<T>* tw, unsigned inv_nb, unsigned inv_ns) {
   const int nb = n / R;
   const int step = n / (Ns * R);
   for (int idx = threadIdx.x; idx < PB * nb; idx += blockDim.x) {
-    const int j = idx / nb, jj = idx % nb;
-    const int k = jj % Ns;
+    const int j = quot_of(idx, inv_nb), jj = idx - j * nb;
+    const int s = quot_of(jj, inv_ns), k = jj - s * Ns;
     cpx<T> v[R];
     const cpx<T>* src = a + j * ps;
 #pragma unroll
@@ -121,7 +131,7 @@ __device__ __forceinline__ void stockham_pass(const cpx<T>* a, cpx<T>* b, int PB
       v[q] = x;
     }
     dft_r<T, R>(v, sign, tw, n);
-    const int idxD = (jj / Ns) * Ns * R + k;
+    const int idxD = s * Ns * R + k;
     cpx<T>* dst = b + j * ps;
 #pragma unroll
     for (int q = 0; q < R; ++q) dst[idxD + q * Ns] = v[q];
@@ -138,13 +148,13 @@ __device__ cpx<T>* stockham(cpx<T>* a, cpx<T>* b, int PB, int ps, const FftPassD
   for (int p = 0; p < d.nrad; ++p) {
     const int R = d.rad[p];
     switch (R) {
-      case 4: stockham_pass<T, 4>(a, b, PB, ps, n, Ns, d.sign, tw); break;
-      case 2: stockham_pass<T, 2>(a, b, PB, ps, n, Ns, d.sign, tw); break;
-      case 3: stockham_pass<T, 3>(a, b, PB, ps, n, Ns, d.sign, tw); break;
-      case 5: stockham_pass<T, 5>(a, b, PB, ps, n, Ns, d.sign, tw); break;
-      case 7: stockham_pass<T, 7>(a, b, PB, ps, n, Ns, d.sign, tw); break;
-      case 11: stockham_pass<T, 11>(a, b, PB, ps, n, Ns, d.sign, tw); break;
-      default: stockham_pass<T, 13>(a, b, PB, ps, n, Ns, d.sign, tw); break;
+      case 4: stockham_pass<T, 4>(a, b, PB, ps, n, Ns, d.sign, tw, d.inv_nb[p], d.inv_ns[p]); break;
+      case 2: stockham_pass<T, 2>(a, b, PB, ps, n, Ns, d.sign, tw, d.inv_nb[p], d.inv_ns[p]); break;
+      case 3: stockham_pass<T, 3>(a, b, PB, ps, n, Ns, d.sign, tw, d.inv_nb[p], d.inv_ns[p]); break;
+      case 5: stockham_pass<T, 5>(a, b, PB, ps, n, Ns, d.sign, tw, d.inv_nb[p], d.inv_ns[p]); break;
+      case 7: stockham_pass<T, 7>(a, b, PB, ps, n, Ns, d.sign, tw, d.inv_nb[p], d.inv_ns[p]); break;
+      case 11: stockham_pass<T, 11>(a, b, PB, ps, n, Ns, d.sign, tw, d.inv_nb[p], d.inv_ns[p]); break;
+      default: stockham_pass<T, 13>(a, b, PB, ps, n, Ns, d.sign, tw, d.inv_nb[p], d.inv_ns[p]); break;
     }
     __syncthreads();
     cpx<T>* t = a;
@@ -166,14 +176,14 @@ __global__ void __launch_bounds__(256) fft_x_r2c(const TI* in, cpx<T>* out, int6
   cpx<T>* b = a + PB * n;
   const int64_t r0 = (int64_t)blockIdx.x * PB;
   for (int f = threadIdx.x; f < PB * n; f += blockDim.x) {
-    const int j = f / n, e = f % n;
+    const int j = quot_of(f, d.inv_n), e = f - j * n;
     const int64_t r = r0 + j;
     a[f] = {(r < nrows) ? (T)in[r * n + e] : (T)0, (T)0};
   }
   __syncthreads();
   cpx<T>* res = stockham(a, b, PB, n, d, tw);
   for (int f = threadIdx.x; f < PB * nr; f += blockDim.x) {
-    const int j = f / nr, e = f % nr;
+    const int j = quot_of(f, d.inv_nr), e = f - j * nr;
     const int64_t r = r0 + j;
     if (r < nrows) out[r * nr + e] = res[j * n + e];
   }
@@ -189,7 +199,7 @@ __global__ void __launch_bounds__(256) fft_x_c2r(const cpx<T>* in, TO* out, int6
   cpx<T>* b = a + PB * n;
   const int64_t r0 = (int64_t)blockIdx.x * PB;
   for (int f = threadIdx.x; f < PB * n; f += blockDim.x) {
-    const int j = f / n, e = f % n;
+    const int j = quot_of(f, d.inv_n), e = f - j * n;
     const int64_t r = r0 + j;
     cpx<T> v = {(T)0, (T)0};
     if (r < nrows) {
@@ -206,7 +216,7 @@ __global__ void __launch_bounds__(256) fft_x_c2r(const cpx<T>* in, TO* out, int6
   __syncthreads();
   cpx<T>* res = stockham(a, b, PB, n, d, tw);
   for (int f = threadIdx.x; f < PB * n; f += blockDim.x) {
-    const int j = f / n, e = f % n;
+    const int j = quot_of(f, d.inv_n), e = f - j * n;
     const int64_t r = r0 + j;
     if (r < nrows) out[r * n + e] = (TO)(res[j * n + e].x * scale);
   }
@@ -227,14 +237,14 @@ __global__ void __launch_bounds__(256) fft_strided(cpx<T>* data, int ni, int d1,
   const int64_t o = blockIdx.y;
   const int64_t base = (o / d1) * s1 + (o % d1) * s2;
   for (int f = threadIdx.x; f < PB * n; f += blockDim.x) {
-    const int j = f % PB, e = f / PB;
+    const int e = quot_of(f, d.inv_pb), j = f - e * PB;
     const int i = i0 + j;
     a[j * ps + e] = (i < ni) ? data[base + i + e * es] : cpx<T>{(T)0, (T)0};
   }
   __syncthreads();
   cpx<T>* res = stockham(a, b, PB, ps, d, tw);
   for (int f = threadIdx.x; f < PB * n; f += blockDim.x) {
-    const int j = f % PB, e = f / PB;
+    const int e = quot_of(f, d.inv_pb), j = f - e * PB;
     const int i = i0 + j;
     if (i < ni) data[base + i + e * es] = res[j * ps + e];
   }
@@ -1164,7 +1174,7 @@ __global__ void f32_to_f64_kernel(const float* a, double* b, int64_t n) {
 // ---------------------------------------------------------------------------
 static inline unsigned nblk(int64_t n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
-static FftPassDesc make_desc(int n, int sign) {
+static FftPassDesc make_desc(int n, int sign, int pb) {
   FftPassDesc d{};
   d.n = n;
   d.sign = sign;
@@ -1184,6 +1194,13 @@ static FftPassDesc make_desc(int n, int sign) {
     }
   if (m != 1) throw std::runtime_error("FFT length " + std::to_string(n) + " has a prime factor above 13");
   d.nrad = k;
+  d.inv_n = inv_of(n);
+  d.inv_nr = inv_of(n / 2 + 1);
+  d.inv_pb = inv_of(pb);
+  for (int p = 0, ns = 1; p < k; ns *= d.rad[p++]) {
+    d.inv_nb[p] = inv_of(n / d.rad[p]);
+    d.inv_ns[p] = inv_of(ns);
+  }
   return d;
 }
 
@@ -1343,7 +1360,7 @@ void FftPlan<T>::init(const int cells_[3]) {
     tw[p] = static_cast<T*>(dev_alloc(2 * n * sizeof(T)));
     SCA_HIP(hipMemcpyAsync(tw[p], h.data(), 2 * n * sizeof(T), hipMemcpyHostToDevice, hipStreamPerThread));
     SCA_HIP(hipStreamSynchronize(hipStreamPerThread));
-    make_desc(n, -1);  // validate
+    make_desc(n, -1, 1);  // validate
   }
 }
 template <typename T>
@@ -1381,7 +1398,7 @@ void FftPlan<T>::x_pass_fwd(const void* real, bool real_is_double, cpx<T>* S, in
     done = pencil_x_r2c<T, double>(Nx, static_cast<const double*>(real), S, rows, set_rows, t0, shp, st, rowsum);
   else done = pencil_x_r2c<T, T>(Nx, static_cast<const T*>(real), S, rows, set_rows, t0, shp, st, nullptr);
   if (!done) {
-    FftPassDesc d = make_desc(Nx, -1);
+    FftPassDesc d = make_desc(Nx, -1, shp);
     const size_t sh = 2 * (size_t)shp * Nx * sizeof(cpx<T>);
     if (real_is_double)
       hipLaunchKernelGGL((fft_x_r2c<T, double>), dim3(nblk(rows, shp)), dim3(256), sh, st,
@@ -1414,7 +1431,7 @@ void FftPlan<T>::strided_pass(cpx<T>* S, int ncomp, int sign, int axis, int shp,
   const cpx<T>* t = reinterpret_cast<const cpx<T>*>(tw[axis]);
   if (!pencil_strided<T>(n, sign, S, nr, no, d1, K, s2, es, t, shp, st, sum, fin)) {
     if (sum || fin) throw std::runtime_error("FFT: side job on a generic pass");
-    FftPassDesc d = make_desc(n, sign);
+    FftPassDesc d = make_desc(n, sign, shp);
     dim3 grid((nr + shp - 1) / shp, no);
     hipLaunchKernelGGL(fft_strided<T>, grid, dim3(256), 2 * (size_t)shp * (n + 1) * sizeof(cpx<T>), st, S, nr, d1, K,
                        s2, es, d, t, shp);
@@ -1480,7 +1497,7 @@ void FftPlan<T>::x_pass_bwd(const cpx<T>* S, TO* real, int ncomp, T scale, int s
   const int64_t set_rows = (int64_t)(set_comp > 0 ? set_comp : ncomp) * Ny * Nz;
   const cpx<T>* t0 = reinterpret_cast<const cpx<T>*>(tw[0]);
   if (!pencil_x_c2r<T, TO>(Nx, S, real, rows, set_rows, t0, scale, shp, st)) {
-    FftPassDesc d = make_desc(Nx, +1);
+    FftPassDesc d = make_desc(Nx, +1, shp);
     const size_t sh = 2 * (size_t)shp * Nx * sizeof(cpx<T>);
     hipLaunchKernelGGL((fft_x_c2r<T, TO>), dim3(nblk(rows, shp)), dim3(256), sh, st, S, real, rows, d, t0, scale, shp);
   }
