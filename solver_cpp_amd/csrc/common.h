@@ -171,6 +171,10 @@ void launch_mp_tangent_cells(const MpState& s, const MatConst& mc, double dt, co
 void launch_mp_forward(const MpState& s, hipStream_t st);
 // what = 1: F0 <- F, Lp0 <- Lp; what = 2: Fp, S, xi, gamma <- their start values
 void launch_mp_copy(const MpState& s, int what, hipStream_t st);
+// d_Fp_init may be s.Fp
 void launch_mp_init(const MpState& s, const double* d_Fp_init /*(9,N)*/, double xi0, hipStream_t st);
+// the planes of each cell's orientation matrix, from the material map (N) and
+// the materials' matrices (9 each)
+void launch_orientation_planes(const int* d_map, const double* d_om, double* d_Fp, int64_t N, hipStream_t st);
 
 }  // namespace sca

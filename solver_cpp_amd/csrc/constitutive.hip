@@ -1274,6 +1274,16 @@ __global__ void mp_init_kernel(MpState s, const double* Fp_init, double xi_0) {
   }
 }
 
+// planes of each cell's orientation matrix: material map (N) and the materials'
+// matrices (9 doubles each)
+__global__ void orientation_planes_kernel(const int* map, const double* om, double* Fp, int64_t N) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= N) return;
+  const double* o = om + 9 * (int64_t)map[c];
+#pragma unroll
+  for (int q = 0; q < 9; ++q) Fp[q * N + c] = o[q];
+}
+
 // ---- launchers ---------------------------------------------------------------
 int mp_partial_blocks(int64_t N) { return (int)((N + PAV_CELLS - 1) / PAV_CELLS); }
 int mp_sub_planes() { return SUB_PLANES; }
@@ -1442,6 +1452,11 @@ void launch_mp_copy(const MpState& s, int what, hipStream_t st) {
   SCA_HIP(hipGetLastError());
 }
 
+void launch_orientation_planes(const int* d_map, const double* d_om, double* d_Fp, int64_t N, hipStream_t st) {
+  hipLaunchKernelGGL(orientation_planes_kernel, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, d_map, d_om, d_Fp,
+                     N);
+  SCA_HIP(hipGetLastError());
+}
 void launch_mp_init(const MpState& s, const double* d_Fp_init, double xi0, hipStream_t st) {
   hipLaunchKernelGGL(mp_init_kernel, dim3((unsigned)((s.N + 255) / 256)), dim3(256), 0, st, s, d_Fp_init, xi0);
   SCA_HIP(hipGetLastError());

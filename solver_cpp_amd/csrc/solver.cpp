@@ -428,18 +428,19 @@ void Rve::setup(const sc_rve_desc& d, bool residual_graphs) {
   }
   // mechanical_init: F = I, Fp = O_0, Fe = Fp^T, Lp = S = 0, xi = xi_0, gamma = 0
   {
-    std::vector<double> fp(9 * N);
+    // the planes are formed on the device, from the map (in range:
+    // validate_rve_desc; it waits in the iteration counts' plane, which the
+    // first update writes) and one matrix a material: 4 bytes a cell to
+    // compute and send instead of 72
     std::vector<double> om(9 * (size_t)d.n_materials);
     for (int m = 0; m < d.n_materials; ++m) qu2om_host(&orientations[4 * m], &om[9 * m]);
-    for (int64_t c = 0; c < N; ++c) {
-      const int ma = material_at[c];  // in range: validate_rve_desc
-      for (int q = 0; q < 9; ++q) fp[q * N + c] = om[9 * ma + q];
-    }
-    double* d_fp = dalloc(9 * N);
-    SCA_HIP(hipMemcpyAsync(d_fp, fp.data(), fp.size() * sizeof(double), hipMemcpyHostToDevice, st));
-    launch_mp_init(mp, d_fp, d.material.xi_0_sl, st);
+    double* d_om = dalloc(om.size());
+    SCA_HIP(hipMemcpyAsync(d_om, om.data(), om.size() * sizeof(double), hipMemcpyHostToDevice, st));
+    SCA_HIP(hipMemcpyAsync(mp.iters, material_at.data(), N * sizeof(int), hipMemcpyHostToDevice, st));
+    launch_orientation_planes(mp.iters, d_om, mp.Fp, N, st);
+    launch_mp_init(mp, mp.Fp, d.material.xi_0_sl, st);
     SCA_HIP(hipStreamSynchronize(st));
-    dev_free(d_fp);
+    dev_free(d_om);
     allocs.pop_back();
   }
   std::memset(C_ref, 0, sizeof C_ref);
@@ -1403,12 +1404,7 @@ void Rve::load(const std::vector<char>& blob) {
 }
 
 void Rve::init() {
-  std::vector<double> eye(9 * N);
-  for (int q = 0; q < 9; ++q)
-    for (int64_t c = 0; c < N; ++c) eye[q * N + c] = (q % 4 == 0) ? 1.0 : 0.0;
-  SCA_HIP(hipMemcpyAsync(F_last_inc, eye.data(), 9 * N * sizeof(double), hipMemcpyHostToDevice, st));
-  SCA_HIP(hipMemcpyAsync(X, eye.data(), 9 * N * sizeof(double), hipMemcpyHostToDevice, st));
-  SCA_HIP(hipStreamSynchronize(st));
+  launch_identity_planes(F_last_inc, X, N, st);
   x_uniform = last_uniform = true;
   rate_uniform = false;
   for (int q = 0; q < 9; ++q) x_value[q] = last_value[q] = (q % 4 == 0) ? 1.0 : 0.0;

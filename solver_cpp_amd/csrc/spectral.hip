@@ -1143,6 +1143,13 @@ __global__ void __launch_bounds__(256) lincomb_norms_kernel(CombNormArgs r, doub
   }
 }
 
+// the identity in every cell of two fields (9 planes of N)
+__global__ void identity_planes_kernel(double* a, double* b, int64_t N) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= N) return;
+#pragma unroll
+  for (int q = 0; q < 9; ++q) a[q * N + c] = b[q * N + c] = (q % 4 == 0) ? 1.0 : 0.0;
+}
 // SoA (9 planes of N, component q = i+3j) <-> AoS (3,3,N) column-major
 __global__ void soa_to_aos_kernel(const double* soa, double* aos, int64_t N, int ncomp) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2111,6 +2118,10 @@ bool launch_lincomb_norms(const double* XM, double c0, int l, const double* beta
   }
   SCA_HIP(hipGetLastError());
   return true;
+}
+void launch_identity_planes(double* a, double* b, int64_t N, hipStream_t st) {
+  hipLaunchKernelGGL(identity_planes_kernel, dim3(nblk(N)), dim3(256), 0, st, a, b, N);
+  SCA_HIP(hipGetLastError());
 }
 void launch_soa_to_aos(const double* soa, double* aos, int64_t N, int ncomp, hipStream_t st) {
   hipLaunchKernelGGL(soa_to_aos_kernel, dim3(nblk(ncomp * N)), dim3(256), 0, st, soa, aos, N, ncomp);
