@@ -378,7 +378,12 @@ void Rve::setup(const sc_rve_desc& d, bool residual_graphs) {
   if (xsums) d_rowsum = dalloc((size_t)9 * cells[1] * cells[2]);
   partial = dalloc((size_t)std::max<int64_t>(red_blocks() * MAX_RED_VEC, 9 * mp_partial_blocks(N)) +
                    gamma_blocks(K));
-  if (residual_graphs && N <= RESIDUAL_GRAPH_MAX_CELLS) {  // staging of the captured residual evaluation
+  // staging of the captured residual evaluation.  A fused evaluation (eight
+  // launches) is not captured: the graph's launch and the copies into and out
+  // of its buffers cost more than the launches (a re-solved increment of 16^3:
+  // 1818 us captured, 1699 launched; 64^3: 5.46 and 5.18 ms); one of fourteen launches is.
+  const bool fused = d.grid_num.derivative != 2 && fft.fused_gamma_available() && (!mixed || fft32.fused_gamma_available());
+  if (residual_graphs && !fused && N <= RESIDUAL_GRAPH_MAX_CELLS) {
     g_in = dalloc(9 * N);
     g_out = dalloc(9 * N);
   }
