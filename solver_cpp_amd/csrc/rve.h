@@ -11,9 +11,6 @@
 
 struct sc_rve;
 
-// grids up to this many cells evaluate their residual as one HIP graph
-constexpr int64_t RESIDUAL_GRAPH_MAX_CELLS = 64 * 64 * 64;
-
 // mixed precision: the FP32 stage's relative divergence tolerance is never
 // tighter than this (about 170 FP32 rounding units)
 constexpr double MIXED_FP32_REL_DIV_MIN = 1.0e-5;
@@ -122,9 +119,7 @@ struct LoadCursor {
 
 class Rve {
  public:
-  // residual_graphs: grids of at most RESIDUAL_GRAPH_MAX_CELLS cells
-  // evaluate their residual as a HIP graph
-  explicit Rve(const sc_rve_desc& d, bool residual_graphs = true);
+  explicit Rve(const sc_rve_desc& d);
   ~Rve();
   Rve(const Rve&) = delete;
   Rve& operator=(const Rve&) = delete;
@@ -138,8 +133,6 @@ class Rve {
   void form_residual(const double* Fdev, void* rdev);
   void launch_residual(const double* Fdev, void* rdev);
   void launch_spectral(void* rdev);
-  bool ensure_residual_graph();  // false: evaluate eagerly this time
-  void release_residual_graph();
   void constitutive_response(const double* Fdev, double dt);
   void fetch_response_scalars(bool rotate);
   void request_response_scalars(bool rotate, bool residual);
@@ -219,14 +212,6 @@ class Rve {
   double* d_scr_partial = nullptr;  // partial sums of the iteration counters
   const double* f_eval = nullptr;   // F of the last response, until sync_response_F
   double* h_scal = nullptr;  // pinned: response scalars in flight
-  // residual evaluation as a HIP graph (grids of at most
-  // RESIDUAL_GRAPH_MAX_CELLS cells): staging of F and r, the graph and the
-  // arguments it was captured with
-  double *g_in = nullptr, *g_out = nullptr;
-  hipGraph_t g_graph = nullptr;
-  hipGraphExec_t g_exec = nullptr;
-  std::vector<char> g_sig, g_seen;
-  int64_t stats_graph_captures = 0, stats_graph_updates = 0;
   // the pivoting list and the ill flag are cleared (by the last evaluation's
   // end): the next response need not clear them
   bool response_clean = false;
@@ -254,7 +239,7 @@ class Rve {
 
  private:
   std::vector<double*> allocs;
-  void setup(const sc_rve_desc& d, bool residual_graphs);
+  void setup(const sc_rve_desc& d);
   void release();
   double* dalloc(size_t n);
   int converged() const;

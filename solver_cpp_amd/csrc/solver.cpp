@@ -294,17 +294,17 @@ void validate_rve_desc(const sc_rve_desc& d) {
     bad("unknown divergence correction");
 }
 
-Rve::Rve(const sc_rve_desc& d, bool residual_graphs) {
+Rve::Rve(const sc_rve_desc& d) {
   validate_rve_desc(d);
   try {
-    setup(d, residual_graphs);
+    setup(d);
   } catch (...) {
     release();  // a throwing constructor runs no destructor
     throw;
   }
 }
 
-void Rve::setup(const sc_rve_desc& d, bool residual_graphs) {
+void Rve::setup(const sc_rve_desc& d) {
   desc = d;
   for (int p = 0; p < 3; ++p) {
     cells[p] = d.cells[p];
@@ -378,15 +378,6 @@ void Rve::setup(const sc_rve_desc& d, bool residual_graphs) {
   if (xsums) d_rowsum = dalloc((size_t)9 * cells[1] * cells[2]);
   partial = dalloc((size_t)std::max<int64_t>(red_blocks() * MAX_RED_VEC, 9 * mp_partial_blocks(N)) +
                    gamma_blocks(K));
-  // staging of the captured residual evaluation.  A fused evaluation (eight
-  // launches) is not captured: the graph's launch and the copies into and out
-  // of its buffers cost more than the launches (a re-solved increment of 16^3:
-  // 1818 us captured, 1699 launched; 64^3: 5.46 and 5.18 ms); one of fourteen launches is.
-  const bool fused = d.grid_num.derivative != 2 && fft.fused_gamma_available() && (!mixed || fft32.fused_gamma_available());
-  if (residual_graphs && !fused && N <= RESIDUAL_GRAPH_MAX_CELLS) {
-    g_in = dalloc(9 * N);
-    g_out = dalloc(9 * N);
-  }
   small = dalloc(512);
   d_u = dalloc(3 * N);
   d_xp = dalloc(3 * N);
@@ -470,7 +461,6 @@ Rve::~Rve() { release(); }
 void Rve::release() {
   // the blocks go back to the library's caches: nothing may still use them
   if (st) (void)hipStreamSynchronize(st);
-  release_residual_graph();
   delete ngm;
   ngm = nullptr;
   if (wait_ev) (void)hipEventDestroy(wait_ev);
@@ -696,9 +686,12 @@ GammaHost Rve::gamma_host(bool do_gamma) const {
 // The device work of one residual evaluation on st, without host
 // synchronisation: material-point update at F, P sums, the aim of the
 // convolution, forward transform, Gamma convolution with the divergence,
-// inverse transform into r, and the asynchronous copy of the response
-// scalars.  Its launches depend on F, r, delta_t, the compliance S, the load
-// rotation, C_ref and the precision phase only, so it can be captured.
+// inverse transform into r, and the response scalars' way to the host.
+// Launched, not replayed from a captured graph, on grids of every size: a
+// graph needs F copied in and r out of its own buffers, and the forward step
+// could not exchange the state's.  Re-solved increments, captured / launched:
+// 16^3 1818 / 1699 us, 64^3 5.46 / 5.18 ms, 27 x 40 x 22 mixed (fourteen
+// launches an evaluation) 2.69 / 2.59 ms.
 void Rve::launch_residual(const double* Fdev, void* rdev) {
   state_stale = false;  // the update writes the current set of every cell
   MpState s = mp;
@@ -788,76 +781,7 @@ void Rve::launch_spectral(void* rdev) {
   SCA_HIP(hipMemcpyAsync(h_scal, small + SM_SUMS, (kt.on ? 13 : 11) * sizeof(double), hipMemcpyDeviceToHost, st));
 }
 
-// Graph of launch_residual(g_in, g_out) for the current arguments.  A
-// signature seen for the first time is evaluated eagerly (returns false): a
-// capture pays off only when the arguments repeat.  A new capture updates the
-// executable graph in place when only kernel arguments changed (the launch
-// sequence is the same), instead of instantiating it again.
-bool Rve::ensure_residual_graph() {
-  struct Sig {
-    double dt, S[81], rot_q[4], C_ref[81];
-    int use32;
-  } sig{};
-  sig.dt = delta_t;
-  std::memcpy(sig.S, S, sizeof sig.S);
-  std::memcpy(sig.rot_q, rot_q, sizeof sig.rot_q);
-  std::memcpy(sig.C_ref, C_ref, sizeof sig.C_ref);
-  sig.use32 = use32 ? 1 : 0;
-  const char* sb = reinterpret_cast<const char*>(&sig);
-  auto same = [&](const std::vector<char>& v) { return v.size() == sizeof sig && std::memcmp(v.data(), sb, sizeof sig) == 0; };
-  if (g_exec && same(g_sig)) return true;
-  if (!same(g_seen)) {
-    g_seen.assign(sb, sb + sizeof sig);
-    return false;
-  }
-  SCA_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-  try {
-    launch_residual(g_in, g_out);
-  } catch (...) {
-    hipGraph_t broken = nullptr;
-    (void)hipStreamEndCapture(st, &broken);
-    if (broken) (void)hipGraphDestroy(broken);
-    throw;
-  }
-  hipGraph_t graph = nullptr;
-  SCA_HIP(hipStreamEndCapture(st, &graph));
-  if (g_exec) {
-    hipGraphNode_t err_node = nullptr;
-    hipGraphExecUpdateResult res;
-    if (hipGraphExecUpdate(g_exec, graph, &err_node, &res) == hipSuccess && res == hipGraphExecUpdateSuccess) {
-      if (g_graph) (void)hipGraphDestroy(g_graph);
-      g_graph = graph;
-      g_sig.assign(sb, sb + sizeof sig);
-      stats_graph_updates++;
-      return true;
-    }
-    (void)hipGetLastError();  // a refused update leaves no error behind
-  }
-  hipGraphExec_t exec = nullptr;
-  const hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-  if (e != hipSuccess) {
-    (void)hipGraphDestroy(graph);
-    SCA_HIP(e);
-  }
-  release_residual_graph();
-  g_graph = graph;
-  g_exec = exec;
-  g_sig.assign(sb, sb + sizeof sig);
-  stats_graph_captures++;
-  return true;
-}
-
-void Rve::release_residual_graph() {
-  if (g_exec) (void)hipGraphExecDestroy(g_exec);
-  if (g_graph) (void)hipGraphDestroy(g_graph);
-  g_exec = nullptr;
-  g_graph = nullptr;
-  g_sig.clear();
-}
-
-// MechSolverBasic::formResidual (mech_solver_basic.cpp:286-339).  Small grids
-// are bound by launch latency: there the evaluation is one graph launch
-// between copies of F in and r out (not while kernels are being timed).
+// MechSolverBasic::formResidual (mech_solver_basic.cpp:286-339).
 //
 // reuse_response (mixed precision, first evaluation of the FP64 finish): the
 // material point was last updated, in FP64, at exactly this F (the point the
@@ -878,11 +802,6 @@ void Rve::form_residual(const double* Fdev, void* rdev) {
     SCA_HIP(hipStreamSynchronize(st));  // F and everything before it complete
     state_stale = false;                 // the joint update writes the current set
     batch->evaluate(this, Fdev, rdev);   // the response scalars land in h_scal
-  } else if (g_in && !kt.on && ensure_residual_graph()) {
-    SCA_HIP(hipMemcpyAsync(g_in, Fdev, 9 * N * sizeof(double), hipMemcpyDeviceToDevice, st));
-    SCA_HIP(hipGraphLaunch(g_exec, st));
-    SCA_HIP(hipMemcpyAsync(rdev, g_out, 9 * N * (use32 ? sizeof(float) : sizeof(double)), hipMemcpyDeviceToDevice,
-                           st));
   } else {
     launch_residual(Fdev, rdev);
   }
@@ -1355,8 +1274,6 @@ void Rve::load(const std::vector<char>& blob) {
     throw std::runtime_error("checkpoint of another microstructure, material or numerics");
   // nothing of this context's last evaluation may land on the restored state
   complete_response_scalars();
-  release_residual_graph();
-  g_seen.clear();
   state_stale = false;  // both sets of the state are restored
   const std::vector<std::pair<double*, int64_t>> planes = {
       {mp.F, 9 * N},       {mp.F0, 9 * N},    {mp.Fp0, 9 * N},   {mp.Lp0, 9 * N},   {mp.S0, 9 * N},
@@ -1452,18 +1369,12 @@ void Rve::forward(bool cutBack, bool guess, double dt, double dt_old, double t_r
     // by exchanging the buffers' roles (the next evaluation writes the
     // current set before anything reads it; refresh_state() copies it back
     // for a reader that comes first); F and Lp stay in use and are copied.
-    // A captured residual graph holds the buffer addresses: with it the
-    // whole state is copied.
-    if (g_in) {
-      launch_mp_forward(mp, st);
-    } else {
-      launch_mp_copy(mp, 1, st);
-      std::swap(mp.Fp, mp.Fp0);
-      std::swap(mp.S, mp.S0);
-      std::swap(mp.xi, mp.xi0);
-      std::swap(mp.gamma, mp.gamma0);
-      state_stale = true;
-    }
+    launch_mp_copy(mp, 1, st);
+    std::swap(mp.Fp, mp.Fp0);
+    std::swap(mp.S, mp.S0);
+    std::swap(mp.xi, mp.xi0);
+    std::swap(mp.gamma, mp.gamma0);
+    state_stale = true;
   }
   for (int q = 0; q < 9; ++q) F_aim[q] = F_aim_last_inc[q] + F_aim_dot[q] * dt;
   for (int q = 0; q < 9; ++q)
