@@ -179,7 +179,7 @@ void f_materialpoint_initDamask(void) {
     b.dPdF_dev = b.dalloc(81 * (size_t)N);
     b.sub = b.dalloc((size_t)mp_sub_planes() * N);
     SCA_HIP(hipMalloc(&mp.iters, 2 * N * sizeof(int)));
-    SCA_HIP(hipMalloc(&b.d_ill, 2 * sizeof(int)));
+    SCA_HIP(hipMalloc(&b.d_ill, sizeof(int)));
     // Fp0 = orientation matrix of each cell's material (material.f90:155)
     std::vector<double> om(9 * (size_t)nm), fp(9 * (size_t)N);
     for (int m = 0; m < nm; ++m) qu2om_host(&b.mat.orientations[4 * m], &om[9 * m]);

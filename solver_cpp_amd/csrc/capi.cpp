@@ -857,7 +857,7 @@ int sc_mp_update(int64_t n, double dt, const sc_material* m, const sc_phase_nume
     double** t12[4] = {&st.xi0, &st.gamma0, &st.xi, &st.gamma};
     for (int k = 0; k < 4; ++k) *t12[k] = b + (int64_t)90 * n + (int64_t)12 * n * k;
     int *d_ill = nullptr, *d_br = nullptr, *d_it = nullptr;
-    SCA_HIP(hipMalloc(&d_ill, 2 * sizeof(int)));
+    SCA_HIP(hipMalloc(&d_ill, sizeof(int)));
     std::unique_ptr<int, void (*)(int*)> g1(d_ill, [](int* p) { (void)hipFree(p); });
     SCA_HIP(hipMalloc(&d_br, n * sizeof(int)));
     std::unique_ptr<int, void (*)(int*)> g2(d_br, [](int* p) { (void)hipFree(p); });

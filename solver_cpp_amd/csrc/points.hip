@@ -800,7 +800,7 @@ __global__ void __launch_bounds__(64) mp_points_kernel(KernelArgs) {
 //   (diag + w(H U_j)) y = w(X),   V = sum_j U_j y_j,   dS = C : (X - H V),
 // and dFp^-1/dF = -invFp0 V.  The 5x5 matrix is inverted once (partial
 // pivoting) for the nine columns: 5730 instead of 8400 instructions, no 9x9
-// elimination in one dependent chain (28 -> 17 us for a call of one wave).
+// elimination in one dependent chain (26 -> 13 us for 4097 points).
 // ---------------------------------------------------------------------------
 
 // inverse of M (NW x NW, row-major) by Gauss-Jordan with partial pivoting
