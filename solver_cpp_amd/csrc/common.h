@@ -144,10 +144,9 @@ struct MpBatchPav {
 void launch_mp_points(const MpState& s, const MatConst& mc, double dt, int* d_ill, double* d_sub, hipStream_t st,
                       int* d_broken = nullptr, int64_t c_begin = 0, int64_t c_end = -1);
 // the grid solver's update of all cells (needs s.repivot); *d_ill as above.
-// clear = false: the list's count and the flag are zero already (launch_response_reset)
+// clear = false: the list's count and the flag are zero already
 void launch_mp_response(const MpState& s, const MatConst& mc, double dt, int* d_ill, double* d_sub, hipStream_t st,
                         bool clear = true);
-void launch_response_reset(int* repivot, int* d_ill, hipStream_t st);
 int mp_partial_blocks(int64_t N);
 // Material-point updates of n RVEs in one launch (and their pivoting passes
 // and P block sums), each RVE's results bitwise those of launch_mp_response

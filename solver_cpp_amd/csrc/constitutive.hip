@@ -1288,10 +1288,6 @@ __global__ void orientation_planes_kernel(const int* map, const double* om, doub
 int mp_partial_blocks(int64_t N) { return (int)((N + PAV_CELLS - 1) / PAV_CELLS); }
 int mp_sub_planes() { return SUB_PLANES; }
 
-void launch_response_reset(int* repivot, int* d_ill, hipStream_t st) {
-  hipLaunchKernelGGL(repivot_reset_kernel, dim3(1), dim3(1), 0, st, repivot, d_ill);
-}
-
 void launch_mp_response(const MpState& s, const MatConst& mc, double dt, int* d_ill, double* d_sub, hipStream_t st,
                         bool clear) {
   if (s.N < 1) return;
@@ -1305,7 +1301,7 @@ void launch_mp_response(const MpState& s, const MatConst& mc, double dt, int* d_
   // second pass: a fixed grid striding over the list (it holds at most the
   // range's points)
   const int blocks2 = std::min(blocks, 1024);
-  if (clear) launch_response_reset(s.repivot, d_ill, st);
+  if (clear) hipLaunchKernelGGL(repivot_reset_kernel, dim3(1), dim3(1), 0, st, s.repivot, d_ill);
   if (mc.n_e4 == 80 && mc.a_e4 == 9) {
     hipLaunchKernelGGL((mp_response_kernel<80, 9>), dim3(blocks), dim3(64), 0, st, a);
     hipLaunchKernelGGL((mp_repivot_kernel<80, 9>), dim3(blocks2), dim3(64), 0, st, a);

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "common.h"
+#include "response_flags.h"
 #include "spectral.h"
 
 struct sc_rve;
@@ -131,7 +132,7 @@ class Rve {
   int next_increment(const sc_loadstep* steps, int n_steps, LoadCursor& cur, int* iterations, int* evaluations);
   // r: floats during the FP32 stage of the mixed form (use32), doubles otherwise
   void form_residual(const double* Fdev, void* rdev);
-  void launch_residual(const double* Fdev, void* rdev);
+  void launch_residual(const double* Fdev, void* rdev, bool clear);
   void launch_spectral(void* rdev);
   void constitutive_response(const double* Fdev, double dt);
   void fetch_response_scalars(bool rotate);
@@ -212,9 +213,7 @@ class Rve {
   double* d_scr_partial = nullptr;  // partial sums of the iteration counters
   const double* f_eval = nullptr;   // F of the last response, until sync_response_F
   double* h_scal = nullptr;  // pinned: response scalars in flight
-  // the pivoting list and the ill flag are cleared (by the last evaluation's
-  // end): the next response need not clear them
-  bool response_clean = false;
+  ResponseFlags response_flags;  // of the pivoting list and the ill flag
   bool scal_pending = false, scal_rotate = false, scal_residual = false, scal_reused = false;
 
   // MechBase state (mech_base.h:75-107), column-major

@@ -515,8 +515,8 @@ void Rve::constitutive_response(const double* Fdev, double dt) {
   s.F = const_cast<double*>(Fdev);  // read only
   f_eval = Fdev;
   kt.begin(SC_KT_RESPONSE, st);
+  response_flags.written();
   launch_mp_response(s, mc, dt, d_ill, sub, st);
-  response_clean = false;
   kt.end(SC_KT_RESPONSE, N, st);
   kt.begin(SC_KT_REDUCE, st);
   launch_pav_partial(mp.P, N, partial, st);
@@ -692,12 +692,13 @@ GammaHost Rve::gamma_host(bool do_gamma) const {
 // could not exchange the state's.  Re-solved increments, captured / launched:
 // 16^3 1818 / 1699 us, 64^3 5.46 / 5.18 ms, 27 x 40 x 22 mixed (fourteen
 // launches an evaluation) 2.69 / 2.59 ms.
-void Rve::launch_residual(const double* Fdev, void* rdev) {
+// clear: the pivoting list and the ill flag are not clear yet.
+void Rve::launch_residual(const double* Fdev, void* rdev, bool clear) {
   state_stale = false;  // the update writes the current set of every cell
   MpState s = mp;
   s.F = const_cast<double*>(Fdev);  // read only
   kt.begin(SC_KT_RESPONSE, st);
-  launch_mp_response(s, mc, delta_t, d_ill, sub, st, !fused_gamma());
+  launch_mp_response(s, mc, delta_t, d_ill, sub, st, clear);
   kt.end(SC_KT_RESPONSE, N, st);
   if (!xsums) {  // else the forward transform gives the P sums
     kt.begin(SC_KT_REDUCE, st);
@@ -794,17 +795,17 @@ void Rve::form_residual(const double* Fdev, void* rdev) {
   const bool reused = reuse_response;
   reuse_response = false;
   // a fused evaluation clears the response's flags for the next one; others leave them as they are
-  if (!reused && !batch && fused_gamma() && !response_clean) launch_response_reset(mp.repivot, d_ill, st);
-  response_clean = !batch && fused_gamma();
-  if (reused) {
-    launch_spectral(rdev);
-  } else if (batch) {
-    SCA_HIP(hipStreamSynchronize(st));  // F and everything before it complete
-    state_stale = false;                 // the joint update writes the current set
-    batch->evaluate(this, Fdev, rdev);   // the response scalars land in h_scal
-  } else {
-    launch_residual(Fdev, rdev);
-  }
+  response_flags.evaluation(!batch && fused_gamma(), [&](bool clear) {
+    if (reused) {
+      launch_spectral(rdev);
+    } else if (batch) {
+      SCA_HIP(hipStreamSynchronize(st));  // F and everything before it complete
+      state_stale = false;                 // the joint update writes the current set
+      batch->evaluate(this, Fdev, rdev);   // the response scalars land in h_scal
+    } else {
+      launch_residual(Fdev, rdev, clear);
+    }
+  });
   f_eval = Fdev;
   last_dt = delta_t;
   // P_av, err_div, F_aim and err_BC of this evaluation are completed at the
