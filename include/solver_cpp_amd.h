@@ -228,7 +228,10 @@ int sc_rve_form_residual(sc_rve* rve, const double* F, double* r);
  * solver arithmetic against a recorded trace. */
 int sc_ngmres_replay(int64_t n, int m, const double* x0, int n_evals, const double* r_rec, double* x_eval);
 
-/* Field / state access (host copies, (3,3,N) column-major). */
+/* Field / state access (host copies, (3,3,N) column-major).  sc_rve_get_field
+ * writes nothing of the context: several threads may read one context at once,
+ * and beside a running sc_rve_calculate_solution (they then see the planes of
+ * an evaluation that may be unfinished); not beside the other calls. */
 enum {
   SC_FIELD_F = 0,        /* solver deformation gradient (F_PETSc) */
   SC_FIELD_P = 1,        /* first Piola-Kirchhoff stress of the last evaluation */

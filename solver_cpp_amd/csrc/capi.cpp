@@ -58,6 +58,25 @@ struct DBuf {
   }
 };
 
+// a block of the library's allocator for work on st; given back when that work
+// has completed (finish(), or where an error left it unfinished)
+struct Staging {
+  double* p;
+  hipStream_t st;
+  bool done = false;
+  Staging(size_t n, hipStream_t st_) : p(static_cast<double*>(sca::dev_alloc(n * sizeof(double)))), st(st_) {}
+  ~Staging() {
+    if (!done) (void)hipStreamSynchronize(st);
+    sca::dev_free(p);
+  }
+  void finish() {
+    SCA_HIP(hipStreamSynchronize(st));
+    done = true;
+  }
+  Staging(const Staging&) = delete;
+  Staging& operator=(const Staging&) = delete;
+};
+
 struct Stream {
   hipStream_t s = nullptr;
   Stream() { SCA_HIP(hipStreamCreate(&s)); }
@@ -450,23 +469,27 @@ int sc_rve_get_field(sc_rve* R, int field, double* out, int64_t n) {
 
 }  // extern "C"
 
-// host copy of a field in the reference's layout (sc_rve_get_field)
+// host copy of a field in the reference's layout (sc_rve_get_field).  A read
+// writes nothing of the context, so that threads may read one context beside
+// each other and beside a solve.  After a forward step that exchanged the
+// current and start buffers of Fp, S, xi and gamma, the current values are the
+// start ones until the next update.
 int sca::rve_get_field(sca::Rve& v, int field, double* out, int64_t n) {
-  v.refresh_state();
   {
     const int64_t N = v.N;
+    const bool stale = v.state_stale;
     const double* src = nullptr;
     int ncomp = 9;
     switch (field) {
       case SC_FIELD_F: src = v.X; break;
       case SC_FIELD_P: src = v.mp.P; break;
-      case SC_FIELD_FP: src = v.mp.Fp; break;
+      case SC_FIELD_FP: src = stale ? v.mp.Fp0 : v.mp.Fp; break;
       case SC_FIELD_LP: src = v.mp.Lp; break;
-      case SC_FIELD_S: src = v.mp.S; break;
+      case SC_FIELD_S: src = stale ? v.mp.S0 : v.mp.S; break;
       case SC_FIELD_FE: src = v.mp.Fe; break;
       case SC_FIELD_F_LAST_INC: src = v.F_last_inc; break;
-      case SC_FIELD_XI: src = v.mp.xi; ncomp = 12; break;
-      case SC_FIELD_GAMMA: src = v.mp.gamma; ncomp = 12; break;
+      case SC_FIELD_XI: src = stale ? v.mp.xi0 : v.mp.xi; ncomp = 12; break;
+      case SC_FIELD_GAMMA: src = stale ? v.mp.gamma0 : v.mp.gamma; ncomp = 12; break;
       case SC_FIELD_ITERATIONS: {
         if (n < 2 * N) throw std::runtime_error("output buffer too small");
         std::vector<int> it(2 * N);
@@ -491,17 +514,13 @@ int sca::rve_get_field(sca::Rve& v, int field, double* out, int64_t n) {
       default: throw std::runtime_error("unknown field");
     }
     if (n < ncomp * N) throw std::runtime_error("output buffer too small");
-    // cells at a time through the spectrum's buffer (18 K doubles, scratch
-    // between evaluations; all cells at once for nine components): hipMalloc
-    // and hipFree of a buffer cost 2 x 0.3 ms at 128^3
-    const int64_t chunk = 18 * v.K / ncomp;
-    for (int64_t c0 = 0; c0 < N; c0 += chunk) {
-      const int64_t m = std::min(chunk, N - c0);
-      sca::launch_soa_to_aos(src + c0, v.spec, N, ncomp, v.st, m);
-      SCA_HIP(hipMemcpyAsync(out + ncomp * c0, v.spec, (size_t)(ncomp * m) * sizeof(double), hipMemcpyDeviceToHost,
-                             v.st));
-    }
-    SCA_HIP(hipStreamSynchronize(v.st));
+    // through a buffer of this call's own from the library's allocator (one
+    // size for every field: hipMalloc and hipFree of it, once a call, cost
+    // 2 x 0.3 ms at 128^3)
+    Staging buf((size_t)12 * N, v.st);
+    sca::launch_soa_to_aos(src, buf.p, N, ncomp, v.st);
+    SCA_HIP(hipMemcpyAsync(out, buf.p, (size_t)(ncomp * N) * sizeof(double), hipMemcpyDeviceToHost, v.st));
+    buf.finish();
     return 0;
   }
 }

@@ -1,6 +1,7 @@
 // One representative volume element resident on the GPU (solver.cpp).
 #pragma once
 #include <algorithm>
+#include <atomic>
 #include <complex>
 #include <functional>
 #include <string>
@@ -176,7 +177,7 @@ class Rve {
   double* d_rowsum = nullptr;  // 9 Ny Nz
   // after a forward step that exchanged the roles of the current and start
   // buffers of Fp, S, xi, gamma, until the next material-point update
-  bool state_stale = false;
+  std::atomic<bool> state_stale{false};  // field reads look at it from other threads
   void refresh_state();  // makes the current set readable (a copy, if stale)
   // polling waits (wait_stream); the job server's contexts wait blocking
   bool spin_wait = true;

@@ -152,8 +152,7 @@ void launch_lincomb(const double* XM, double c0, int l, const double* beta, cons
 bool launch_lincomb_norms(const double* XM, double c0, int l, const double* beta, const double* const* X,
                           double* XA, int64_t n, double* partial, hipStream_t st);
 void launch_identity_planes(double* a, double* b, int64_t N, hipStream_t st);
-// m (-1: N): only the first m cells
-void launch_soa_to_aos(const double* soa, double* aos, int64_t N, int ncomp, hipStream_t st, int64_t m = -1);
+void launch_soa_to_aos(const double* soa, double* aos, int64_t N, int ncomp, hipStream_t st);
 void launch_aos_to_soa(const double* aos, double* soa, int64_t N, int ncomp, hipStream_t st);
 void launch_f64_to_f32(const double* a, float* b, int64_t n, hipStream_t st);
 void launch_f32_to_f64(const float* a, double* b, int64_t n, hipStream_t st);

@@ -1151,9 +1151,9 @@ __global__ void identity_planes_kernel(double* a, double* b, int64_t N) {
   for (int q = 0; q < 9; ++q) a[q * N + c] = b[q * N + c] = (q % 4 == 0) ? 1.0 : 0.0;
 }
 // SoA (9 planes of N, component q = i+3j) <-> AoS (3,3,N) column-major
-__global__ void soa_to_aos_kernel(const double* soa, double* aos, int64_t N, int ncomp, int64_t m) {
+__global__ void soa_to_aos_kernel(const double* soa, double* aos, int64_t N, int ncomp) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < ncomp * m) {
+  if (t < ncomp * N) {
     const int64_t c = t / ncomp;
     const int q = (int)(t % ncomp);
     aos[t] = soa[q * N + c];
@@ -2123,9 +2123,8 @@ void launch_identity_planes(double* a, double* b, int64_t N, hipStream_t st) {
   hipLaunchKernelGGL(identity_planes_kernel, dim3(nblk(N)), dim3(256), 0, st, a, b, N);
   SCA_HIP(hipGetLastError());
 }
-void launch_soa_to_aos(const double* soa, double* aos, int64_t N, int ncomp, hipStream_t st, int64_t m) {
-  if (m < 0) m = N;
-  hipLaunchKernelGGL(soa_to_aos_kernel, dim3(nblk(ncomp * m)), dim3(256), 0, st, soa, aos, N, ncomp, m);
+void launch_soa_to_aos(const double* soa, double* aos, int64_t N, int ncomp, hipStream_t st) {
+  hipLaunchKernelGGL(soa_to_aos_kernel, dim3(nblk(ncomp * N)), dim3(256), 0, st, soa, aos, N, ncomp);
   SCA_HIP(hipGetLastError());
 }
 void launch_aos_to_soa(const double* aos, double* soa, int64_t N, int ncomp, hipStream_t st) {

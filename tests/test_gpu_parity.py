@@ -6,6 +6,7 @@ plain GPU form has to meet against the reference solver.
 """
 import ctypes as C
 import os
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -338,6 +339,53 @@ def test_state_read_between_forward_and_solve(product):
             np.testing.assert_array_equal(rs[0].field(k), before[k], err_msg=k)
         sa, sb = rs[0].calculate_solution(), rs[1].calculate_solution()
         assert (sa.required_iterations, sa.residual_evaluations) == (sb.required_iterations, sb.residual_evaluations)
+        for k in ["F", "P", "Fp", "S", "xi", "gamma"]:
+            np.testing.assert_array_equal(rs[0].field(k), rs[1].field(k), err_msg=k)
+    finally:
+        for r in rs:
+            r.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_field_reads_beside_each_other_and_a_solve(product, precision):
+    """sc_rve_get_field writes nothing of the context.  Four threads read four
+    fields of one context at once, each the same values every time; then two
+    threads read P and the slip resistances while a third solves an increment:
+    counts, scalars and fields are bitwise those of a context left alone."""
+    cells = (24, 18, 16)
+    print(f"concurrent reads: cells {cells} precision {precision}", flush=True)
+    mat, ori, size = polycrystal(cells, 6, seed=15, ori_seed=16)
+    load = tension_x(t=10.0, N=20)
+    rs = [Rve(product, cells, size, mat, ori, precision=precision, **EXAMPLE_NUMERICS) for _ in range(2)]
+    try:
+        for r in rs:
+            r.init()
+            r.forward(False, False, 0.5, 1.0, 10.0, load)
+            r.calculate_solution()
+        names = ["P", "xi", "Fe", "gamma"]
+        want = {k: rs[0].field(k) for k in names}
+        with ThreadPoolExecutor(4) as ex:
+            for k, got in ex.map(lambda k: (k, [rs[0].field(k) for _ in range(25)]), names):
+                for g in got:
+                    np.testing.assert_array_equal(g, want[k], err_msg=k)
+        for r in rs:
+            r.forward(False, True, 0.5, 0.5, 9.5, load)
+        with ThreadPoolExecutor(3) as ex:
+            solve = ex.submit(rs[0].calculate_solution)
+
+            def watch(k):
+                reads = 0
+                while reads < 500 and not (solve.done() and reads):
+                    rs[0].field(k)
+                    reads += 1
+                return reads
+
+            reads = [ex.submit(watch, k) for k in ("P", "xi")]
+            sa = solve.result()
+            assert all(f.result() > 0 for f in reads)
+        sb = rs[1].calculate_solution()
+        assert (sa.required_iterations, sa.residual_evaluations) == (sb.required_iterations, sb.residual_evaluations)
+        assert (sa.err_div, sa.err_BC) == (sb.err_div, sb.err_BC)
         for k in ["F", "P", "Fp", "S", "xi", "gamma"]:
             np.testing.assert_array_equal(rs[0].field(k), rs[1].field(k), err_msg=k)
     finally:
