@@ -212,8 +212,8 @@ __device__ __forceinline__ const cpx<T>* stage_tw(cpx<T>* lds_tw, const cpx<T>* 
 // strided complex pass (y or z): pencil (o, i) starts at
 // (o / d1) * s1 + (o % d1) * s2 + i with element stride es; a block takes P
 // consecutive i of one o, the pencil index fastest across lanes.  The first
-// side.blocks() blocks do the side job's work instead (Side: NoSide, or a few
-// sums of the evaluation that would otherwise be launches of their own).
+// side.blocks() blocks do the side job's work instead (Side: NoSide, or sums
+// of the evaluation that would otherwise be launches of their own).
 // Blocks go to the 8 XCDs in turn: each XCD gets a contiguous eighth of the
 // pencils, since neighbouring blocks of a y pass share the cache lines at
 // their ends (rows of N/2 + 1 entries start anywhere in a line): y pass of
@@ -225,8 +225,9 @@ __global__ void __launch_bounds__(MAX_PENCIL_BLOCK) strided_kernel(cpx<T>* data,
                                                                    const cpx<T>* tw_g, Side side) {
   using S = Shape<T, N>;
   extern __shared__ unsigned char smem_raw[];
-  if constexpr (Side::blocks() > 0) {
-    if (blockIdx.x < Side::blocks()) {
+  const unsigned sb = side.blocks();
+  if constexpr (Side::active) {
+    if (blockIdx.x < sb) {
       side.run((int)blockIdx.x, reinterpret_cast<double*>(smem_raw));
       return;
     }
@@ -237,7 +238,7 @@ __global__ void __launch_bounds__(MAX_PENCIL_BLOCK) strided_kernel(cpx<T>* data,
   const int p = threadIdx.x & (P - 1), t = threadIdx.x >> __builtin_ctz(P);
   // pencils (o, i) numbered with i fastest across the whole launch, so that a
   // block does not hold a mostly empty row of i (ni = N/2 + 1 is odd)
-  const unsigned nb = gridDim.x - Side::blocks(), b = blockIdx.x - Side::blocks();  // nb: a multiple of 8
+  const unsigned nb = gridDim.x - sb, b = blockIdx.x - sb;  // nb: a multiple of 8
   const int64_t pen = (int64_t)((b & 7) * (nb >> 3) + (b >> 3)) * P + p;
   const int64_t o = pen / ni;
   const int i = (int)(pen - o * ni);
@@ -304,7 +305,6 @@ __device__ __forceinline__ void zop_block(cpx<T>* data, int64_t K, int64_t nq, i
     const int fp = f % Z::W, z = f / Z::W;
     if (q0 + fp < nq) op.point(q0 + fp, z, lds + fp * S::LD + z, Z::W * S::LD, data + q0 + fp + (int64_t)z * nq);
   }
-  op.finish();
 }
 
 // Rows of the pencil that pairs rows ra and rb of a set of set_rows rows

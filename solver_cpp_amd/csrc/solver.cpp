@@ -734,18 +734,21 @@ void Rve::launch_spectral(void* rdev) {
   if (fused_gamma()) {
     // eight launches an evaluation instead of fourteen: the forward z pass
     // and the convolution in one kernel, the small sums in blocks of the y
-    // passes
+    // and z passes.  The divergence terms (K <= N) wait in the substep
+    // scratch, which only the material-point update uses.
+    double* terms = sub;
     const RowSumItem sums{d_rowsum, (int64_t)cells[1] * cells[2], small + SM_SUMS};
     auto stages = [&](auto& plan, auto* sp, auto* r) {
       kt.begin(SC_KT_FFT_FWD, st);
       plan.forward_xy(mp.P, sp, st, d_rowsum, sums);
       kt.end(SC_KT_FFT_FWD, N, st);
       kt.begin(SC_KT_GAMMA, st);
-      const int nb = launch_zgamma(plan, sp, gamma_host(true), d_xi_tab, small + SM_SUMS, S, Rrm, wgt, partial, st);
+      launch_zgamma(plan, sp, gamma_host(true), d_xi_tab, small + SM_SUMS, S, Rrm, wgt, terms, st);
       kt.end(SC_KT_GAMMA, K, st);
       kt.begin(SC_KT_FFT_BWD, st);
-      plan.backward_fin(sp, r, st, FinishItem{partial, nb, small + SM_SUMS, SM_DIV - SM_SUMS, kt.on ? 13 : 11, h_scal,
-                                             d_ill, mp.repivot});
+      plan.backward_fin(sp, r, st, DivItem{terms, K, partial},
+                        FinishItem{partial, gamma_blocks(K), small + SM_SUMS, SM_DIV - SM_SUMS, kt.on ? 13 : 11, h_scal,
+                                   d_ill, mp.repivot});
       kt.end(SC_KT_FFT_BWD, N, st);
     };
     if (use32) stages(fft32, spec32, static_cast<float*>(rdev));

@@ -16,6 +16,13 @@ struct RowSumItem {
   int64_t nrow;  // rows per component (Ny x Nz)
   double* out;
 };
+// the divergence sum's partials (256 consecutive wavevectors each, gamma_blocks(K)
+// of them, as launch_gamma_div's) from its K terms
+struct DivItem {
+  const double* terms;
+  int64_t K;
+  double* partial;
+};
 // end of an evaluation: scal[div] = sum of the nb partials (as
 // launch_final_reduce), the n scalars to host (pinned), *ill and repivot[0]
 // cleared
@@ -27,6 +34,12 @@ struct FinishItem {
   double* host;
   int* ill;
   int* repivot;
+};
+// the side job of a strided pass (at most one)
+struct SideJobs {
+  const RowSumItem* sum = nullptr;
+  const DivItem* div = nullptr;
+  const FinishItem* fin = nullptr;
 };
 
 // 3D FFT of `ncomp` real planes (N each) <-> half spectra (K complex each)
@@ -64,19 +77,19 @@ struct FftPlan {
   void strided_passes(void* spec, int ncomp, int sign, hipStream_t st) const;
   // The transforms of a 9-component field around launch_zgamma, which holds
   // the forward z pass: x and y forward, with the field's sums (SumSide)
-  // formed in the y pass; the inverse (scale 1), with the end of the
-  // evaluation in its y pass.  Available when x and y have pencil kernels and z's fit.
+  // formed in the y pass; the inverse (scale 1), with the divergence partials
+  // in its y pass and the end of the evaluation in its z pass.  Available when x and y have pencil kernels and z's fit.
   bool fused_gamma_available() const;
   void forward_xy(const double* real, T* spec, hipStream_t st, double* rowsum, const RowSumItem& sums) const;
   template <typename TO>
-  void backward_fin(T* spec, TO* real, hipStream_t st, const FinishItem& fin) const;
+  void backward_fin(T* spec, TO* real, hipStream_t st, const DivItem& div, const FinishItem& fin) const;
 
  private:
   int shape(int axis) const;
   void x_pass_fwd(const void* real, bool real_is_double, cpx<T>* S, int ncomp, int shp, hipStream_t st,
                   int set_comp, double* rowsum = nullptr) const;
   void strided_pass(cpx<T>* S, int ncomp, int sign, int axis, int shp, hipStream_t st,
-                    const RowSumItem* sum = nullptr, const FinishItem* fin = nullptr) const;
+                    const SideJobs& job = SideJobs()) const;
   template <typename TO>
   void x_pass_bwd(const cpx<T>* S, TO* real, int ncomp, T scale, int shp, hipStream_t st, int set_comp) const;
 };
@@ -96,11 +109,11 @@ void launch_gamma_div(T* spec, int64_t K, const GammaHost& g, const double* d_ai
 
 // z forward and launch_gamma_div with the aim of launch_bc_aim(sums, S, R, wgt,
 // 1) in one kernel (plan.fused_gamma_available(), derivative 0 or
-// 1): the spectrum has the bits of the separate launches.  Returns the number
-// of divergence partials (at most gamma_blocks(K)).
+// 1): the spectrum and the K terms of the divergence sum have the bits of the
+// separate launches.
 template <typename T>
-int launch_zgamma(const FftPlan<T>& plan, T* spec, const GammaHost& g, const double* d_xi_tab, const double* sums,
-                  const double S[81], const double R[9], double wgt, double* div_partial, hipStream_t st);
+void launch_zgamma(const FftPlan<T>& plan, T* spec, const GammaHost& g, const double* d_xi_tab, const double* sums,
+                   const double S[81], const double R[9], double wgt, double* div_terms, hipStream_t st);
 
 // base_update_coords: F_hat -> u_hat (planes 0..2) and the 9 sums of F;
 // then node / cell-centre coordinates from u (3 planes of N) and the sums

@@ -38,7 +38,8 @@ __device__ __forceinline__ cpx<T> csub(cpx<T> a, cpx<T> b) {
 
 // side job of a strided pass (fft_pencil.h): none
 struct NoSide {
-  static constexpr int blocks() { return 0; }
+  static constexpr bool active = false;
+  __host__ __device__ static constexpr unsigned blocks() { return 0; }
 };
 
 }  // namespace sca
@@ -447,7 +448,11 @@ __global__ void __launch_bounds__(256) gamma_div_batch_kernel(const GammaBatchEn
 // real arithmetic on the two parts of P_hat.  Each value has the roundings of
 // gamma_div_block's (where its complex products keep the compiler from fusing
 // a multiplication with the next addition, so do the rounded products here),
-// so P_hat has its bits; only the divergence sum is added in another order.
+// so P_hat and the wavevectors' terms of the divergence sum have its bits.  The
+// terms are stored (8 bytes a wavevector, 3 % of the spectrum's traffic) and
+// added in the order of the separate launches by side blocks of the inverse y
+// and z passes (DivSide, FinishSide): the divergence decides convergence, and a
+// context alone stops where a batch of it does.
 // Bound: HBM (two passes over the spectrum instead of four) and, at 128^3 in
 // single precision, the one block a CU has registers for.  At 128^3: 92 us
 // (3.3 TB/s) after 54 + 52 apart, without the XCD order 112; at 64^3 17 after
@@ -468,11 +473,8 @@ template <typename T>
 struct GammaOp {
   const GammaArgs& g;
   int64_t K, nq;
-  double* div_partial;
-  unsigned blk;
-  double* red;        // one double per wave
+  double* div_terms;  // K: the wavevectors' terms of the divergence sum
   const double* aim;  // LDS, block 0
-  mutable double contrib;
   // component c of the wavevector: from v[c * stride] to out[c * K]
   __device__ __forceinline__ void point(int64_t q, int z, const cpx<T>* v, int stride, cpx<T>* out) const {
     const int i = (int)(q % g.nr), y = (int)(q / g.nr);
@@ -501,19 +503,20 @@ struct GammaOp {
     }
     // divergence: |P_hat . conj(xi) L/L_scaled|^2, weight 2 for 0 < i < nr-1
     {
-      double s = 0.0;
+      double re2 = 0.0, im2 = 0.0;
 #pragma unroll
       for (int m = 0; m < 3; ++m) {
         double re = 0.0, im = 0.0;
 #pragma unroll
         for (int n = 0; n < 3; ++n) {
-          const double k = xi[n] * g.rescale[n];
-          re += Py[m + 3 * n] * k;
-          im -= Px[m + 3 * n] * k;
+          const double k = rnd_mul(xi[n], g.rescale[n]);
+          re = re + rnd_mul(Py[m + 3 * n], k);
+          im = im - rnd_mul(Px[m + 3 * n], k);
         }
-        s += re * re + im * im;
+        re2 = __builtin_fma(re, re, re2);
+        im2 = __builtin_fma(im, im, im2);
       }
-      contrib += ((i > 0 && i < g.nr - 1) ? 2.0 : 1.0) * s;
+      div_terms[q + nq * z] = ((i > 0 && i < g.nr - 1) ? 2.0 : 1.0) * (re2 + im2);
     }
     if (q == 0 && z == 0) {
 #pragma unroll
@@ -583,31 +586,15 @@ struct GammaOp {
       for (int m = 0; m < 3; ++m) out[(l + 3 * m) * K] = {(T)(-rnd_mul(uy, xi[m])), (T)rnd_mul(ux, xi[m])};
     }
   }
-  // the block's divergence sum: lanes of a wave, then the waves in order
-  __device__ __forceinline__ void finish() const {
-    double s = contrib;
-    for (int w = 32; w > 0; w >>= 1) {
-      const double o = __shfl_xor(s, w);
-      if ((threadIdx.x ^ w) < blockDim.x) s += o;  // the last wave may be partly empty
-    }
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const int nw = ((int)blockDim.x + 63) >> 6;
-      double t = red[0];
-      for (int w = 1; w < nw; ++w) t += red[w];
-      div_partial[blk] = t;
-    }
-  }
 };
 
 template <typename T, int N>
 __global__ void __launch_bounds__((pencil::ZShape<T, N>::THREADS))
     zgamma_kernel(cpx<T>* data, int64_t K, GammaArgs g, const double* sums, BcArgs bc, const cpx<T>* tw,
-                  double* div_partial) {
+                  double* div_terms) {
   using Z = pencil::ZShape<T, N>;
   __shared__ cpx<T> lds[Z::ENTRIES];
-  __shared__ double red[16], aim[9];
+  __shared__ double aim[9];
   const int64_t nq = (int64_t)g.nr * g.Ny;
   // neighbouring blocks read and write the two halves of a cache line: they
   // run on the same XCD (blocks go to the 8 of them in turn)
@@ -616,7 +603,7 @@ __global__ void __launch_bounds__((pencil::ZShape<T, N>::THREADS))
   // the convolution's mean (block 0 holds wavevector 0), ready after the first
   // barrier of the transforms
   if (blk == 0 && threadIdx.x == 0) bc_aim_body(sums, bc, aim);
-  const GammaOp<T> op{g, K, nq, div_partial, blk, red, aim, 0.0};
+  const GammaOp<T> op{g, K, nq, div_terms, aim};
   pencil::zop_block<T, N>(data, K, nq, blk, tw, op, lds);
 }
 
@@ -943,7 +930,7 @@ __global__ void __launch_bounds__(256) rowsum_reduce_batch_kernel(const RowSumIt
   rowsum_block(tab[blockIdx.y], blockIdx.x, red);
 }
 
-// Side jobs of the y passes (fft_pencil.h).  256 virtual threads whatever the
+// Side jobs of the strided passes (fft_pencil.h).  256 virtual threads whatever the
 // block size, so that the sums have the bits of the kernels they stand for.
 __device__ __forceinline__ void side_tree(double* red) {
   __syncthreads();
@@ -955,7 +942,8 @@ __device__ __forceinline__ void side_tree(double* red) {
 // rowsum_reduce_kernel: the nine sums of a field from its x-pass row sums
 struct SumSide {
   RowSumItem e;
-  static constexpr int blocks() { return 9; }
+  static constexpr bool active = true;
+  __host__ __device__ static constexpr unsigned blocks() { return 9; }
   __device__ __forceinline__ void run(int q, double* red) const {
     const double* r = e.rowsum + (int64_t)q * e.nrow;
     for (int v = threadIdx.x; v < 256; v += blockDim.x) {
@@ -975,12 +963,37 @@ struct SumSide {
     if (threadIdx.x == 0) e.out[q] = red[0];
   }
 };
+// the block sums of gamma_div_block from the stored terms: 256 wavevectors a
+// wave at a time, lane t holding the tree's t, t + 64, t + 128 and t + 192
+struct DivSide {
+  DivItem e;
+  unsigned nblocks;
+  static constexpr bool active = true;
+  __host__ __device__ unsigned blocks() const { return nblocks; }
+  __device__ __forceinline__ void run(int blk, double*) const {
+    const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+    const int64_t nb = (e.K + 255) / 256;
+    for (int64_t b = (int64_t)blk * waves + (threadIdx.x >> 6); b < nb; b += (int64_t)nblocks * waves) {
+      double x[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t k = 256 * b + lane + 64 * j;
+        x[j] = k < e.K ? e.terms[k] : 0.0;
+      }
+      double s = (x[0] + x[2]) + (x[1] + x[3]);
+#pragma unroll
+      for (int w = 32; w > 0; w >>= 1) s += __shfl_down(s, w);
+      if (lane == 0) e.partial[b] = s;
+    }
+  }
+};
 // final_reduce_kernel of the divergence partials, then the evaluation's n
 // scalars (scal, the divergence sum at div) to pinned host memory; the flag
 // and the pivoting list's count are cleared for the next evaluation
 struct FinishSide {
   FinishItem e;
-  static constexpr int blocks() { return 1; }
+  static constexpr bool active = true;
+  __host__ __device__ static constexpr unsigned blocks() { return 1; }
   __device__ __forceinline__ void run(int, double* red) const {
     for (int v = threadIdx.x; v < 256; v += blockDim.x) {
       double s = 0.0;
@@ -1295,11 +1308,17 @@ static bool pencil_x_c2r(int n, const cpx<T>* in, TO* out, int64_t rows, int64_t
   }
 }
 
-// side jobs run in blocks of the pass (SumSide: forward, FinishSide: inverse)
+// four sums a wave: a 16th of the blocks that the sums' own launch had go ahead
+// of the pass's own (one a wave: the same within 1 % at 16^3 and 64^3)
+static unsigned div_side_blocks(int64_t K, int bs) {
+  const int per = 4 * (bs / 64);  // block sizes are multiples of 64
+  return (unsigned)((gamma_blocks(K) + per - 1) / per);
+}
+// side jobs run in blocks of the pass (SumSide: forward, DivSide and
+// FinishSide: inverse; at most one)
 template <typename T>
 static bool pencil_strided(int n, int sign, cpx<T>* data, int ni, unsigned no, int d1, int64_t s1, int64_t s2,
-                           int64_t es, const cpx<T>* tw, int bs, hipStream_t st, const RowSumItem* sum = nullptr,
-                           const FinishItem* fin = nullptr) {
+                           int64_t es, const cpx<T>* tw, int bs, hipStream_t st, const SideJobs& job) {
   switch (n) {
 #define SCA_CASE(N)                                                                                          \
   case N: {                                                                                                  \
@@ -1307,19 +1326,21 @@ static bool pencil_strided(int n, int sign, cpx<T>* data, int ni, unsigned no, i
     const int P = bs / S::TP;                                                                                \
     const int64_t npen = (int64_t)ni * no;                                                                   \
     const unsigned nb = (unsigned)((npen + P - 1) / P + 7) / 8 * 8;                                          \
-    const size_t lds = std::max<size_t>(pencil_lds<T, N>(bs), sum || fin ? 256 * sizeof(double) : 0);        \
-    if (sign < 0 && sum)                                                                                     \
-      hipLaunchKernelGGL((pencil::strided_kernel<T, N, -1, SumSide>), dim3(nb + SumSide::blocks()), dim3(bs), lds, \
-                         st, data, ni, npen, d1, s1, s2, es, tw, SumSide{*sum});                             \
+    auto go = [&](auto kernel, const auto& side, size_t side_lds) {                                          \
+      hipLaunchKernelGGL(kernel, dim3(nb + side.blocks()), dim3(bs),                                         \
+                         (std::max<size_t>(pencil_lds<T, N>(bs), side_lds)), st, data, ni, npen, d1, s1, s2, es, tw, \
+                         side);                                                                              \
+    };                                                                                                       \
+    if (sign < 0 && job.sum)                                                                                 \
+      go(pencil::strided_kernel<T, N, -1, SumSide>, SumSide{*job.sum}, 256 * sizeof(double));                \
     else if (sign < 0)                                                                                       \
-      hipLaunchKernelGGL((pencil::strided_kernel<T, N, -1, NoSide>), dim3(nb), dim3(bs), lds, st, data, ni, npen, \
-                         d1, s1, s2, es, tw, NoSide{});                                                      \
-    else if (fin)                                                                                            \
-      hipLaunchKernelGGL((pencil::strided_kernel<T, N, 1, FinishSide>), dim3(nb + FinishSide::blocks()),     \
-                         dim3(bs), lds, st, data, ni, npen, d1, s1, s2, es, tw, FinishSide{*fin});           \
+      go(pencil::strided_kernel<T, N, -1, NoSide>, NoSide{}, 0);                                             \
+    else if (job.div)                                                                                        \
+      go(pencil::strided_kernel<T, N, 1, DivSide>, DivSide{*job.div, div_side_blocks(job.div->K, bs)}, 0);   \
+    else if (job.fin)                                                                                        \
+      go(pencil::strided_kernel<T, N, 1, FinishSide>, FinishSide{*job.fin}, 256 * sizeof(double));           \
     else                                                                                                     \
-      hipLaunchKernelGGL((pencil::strided_kernel<T, N, 1, NoSide>), dim3(nb), dim3(bs), lds, st, data, ni, npen, \
-                         d1, s1, s2, es, tw, NoSide{});                                                      \
+      go(pencil::strided_kernel<T, N, 1, NoSide>, NoSide{}, 0);                                              \
     return true;                                                                                             \
   }
     SCA_PENCIL_LENGTHS(SCA_CASE)
@@ -1427,7 +1448,7 @@ void FftPlan<T>::forward(const TI* real, T* spec, int ncomp, hipStream_t st, int
 
 template <typename T>
 void FftPlan<T>::strided_pass(cpx<T>* S, int ncomp, int sign, int axis, int shp, hipStream_t st,
-                              const RowSumItem* sum, const FinishItem* fin) const {
+                              const SideJobs& job) const {
   const int Ny = cells[1], Nz = cells[2];
   const int n = cells[axis];
   // y: pencils (c, z, i) with element stride nr; z: pencils (c, y, i), stride nr*Ny
@@ -1436,8 +1457,8 @@ void FftPlan<T>::strided_pass(cpx<T>* S, int ncomp, int sign, int axis, int shp,
   const int64_t s2 = axis == 1 ? (int64_t)nr * Ny : (int64_t)nr;
   const int64_t es = axis == 1 ? (int64_t)nr : (int64_t)nr * Ny;
   const cpx<T>* t = reinterpret_cast<const cpx<T>*>(tw[axis]);
-  if (!pencil_strided<T>(n, sign, S, nr, no, d1, K, s2, es, t, shp, st, sum, fin)) {
-    if (sum || fin) throw std::runtime_error("FFT: side job on a generic pass");
+  if (!pencil_strided<T>(n, sign, S, nr, no, d1, K, s2, es, t, shp, st, job)) {
+    if (job.sum || job.div || job.fin) throw std::runtime_error("FFT: side job on a generic pass");
     FftPassDesc d = make_desc(n, sign, shp);
     dim3 grid((nr + shp - 1) / shp, no);
     hipLaunchKernelGGL(fft_strided<T>, grid, dim3(256), 2 * (size_t)shp * (n + 1) * sizeof(cpx<T>), st, S, nr, d1, K,
@@ -1472,15 +1493,15 @@ template <typename T>
 void FftPlan<T>::forward_xy(const double* real, T* spec, hipStream_t st, double* rowsum, const RowSumItem& sums) const {
   cpx<T>* S = reinterpret_cast<cpx<T>*>(spec);
   x_pass_fwd(real, true, S, 9, shape(0), st, 0, rowsum);
-  strided_pass(S, 9, -1, 1, shape(1), st, &sums, nullptr);
+  strided_pass(S, 9, -1, 1, shape(1), st, SideJobs{&sums, nullptr, nullptr});
 }
 
 template <typename T>
 template <typename TO>
-void FftPlan<T>::backward_fin(T* spec, TO* real, hipStream_t st, const FinishItem& fin) const {
+void FftPlan<T>::backward_fin(T* spec, TO* real, hipStream_t st, const DivItem& div, const FinishItem& fin) const {
   cpx<T>* S = reinterpret_cast<cpx<T>*>(spec);
-  strided_pass(S, 9, +1, 1, shape(1), st, nullptr, &fin);
-  strided_pass(S, 9, +1, 2, shape(2), st);
+  strided_pass(S, 9, +1, 1, shape(1), st, SideJobs{nullptr, &div, nullptr});
+  strided_pass(S, 9, +1, 2, shape(2), st, SideJobs{nullptr, nullptr, &fin});
   x_pass_bwd(S, real, 9, (T)1, shape(0), st, 0);
 }
 
@@ -1604,8 +1625,8 @@ template void FftPlan<float>::forward<double>(const double*, float*, int, hipStr
 template void FftPlan<float>::backward<double>(float*, double*, int, double, hipStream_t, int) const;
 template void FftPlan<float>::forward<float>(const float*, float*, int, hipStream_t, int, double*) const;
 template void FftPlan<float>::backward<float>(float*, float*, int, double, hipStream_t, int) const;
-template void FftPlan<double>::backward_fin<double>(double*, double*, hipStream_t, const FinishItem&) const;
-template void FftPlan<float>::backward_fin<float>(float*, float*, hipStream_t, const FinishItem&) const;
+template void FftPlan<double>::backward_fin<double>(double*, double*, hipStream_t, const DivItem&, const FinishItem&) const;
+template void FftPlan<float>::backward_fin<float>(float*, float*, hipStream_t, const DivItem&, const FinishItem&) const;
 
 static GammaArgs gamma_args(const GammaHost& gh, const double* d_xi_tab, const double* d_aim) {
   GammaArgs g;
@@ -1649,8 +1670,8 @@ static BcArgs bc_args(const double S[81], const double R[9], double wgt, int rot
 }
 
 template <typename T>
-int launch_zgamma(const FftPlan<T>& plan, T* spec, const GammaHost& gh, const double* d_xi_tab, const double* sums,
-                  const double S[81], const double R[9], double wgt, double* div_partial, hipStream_t st) {
+void launch_zgamma(const FftPlan<T>& plan, T* spec, const GammaHost& gh, const double* d_xi_tab, const double* sums,
+                   const double S[81], const double R[9], double wgt, double* div_terms, hipStream_t st) {
   if (gh.derivative == 2 || !gh.do_gamma) throw std::runtime_error("fused Gamma convolution: unsupported form");
   const GammaArgs g = gamma_args(gh, d_xi_tab, nullptr);
   const BcArgs bc = bc_args(S, R, wgt, 1);
@@ -1663,7 +1684,7 @@ int launch_zgamma(const FftPlan<T>& plan, T* spec, const GammaHost& gh, const do
     if constexpr (pencil::ZShape<T, N>::fits) {                                                                     \
       nb = (int)((nq + pencil::ZShape<T, N>::W - 1) / pencil::ZShape<T, N>::W);                                     \
       hipLaunchKernelGGL((zgamma_kernel<T, N>), dim3((nb + 7) / 8 * 8), dim3(pencil::ZShape<T, N>::THREADS), 0, st,               \
-                         reinterpret_cast<cpx<T>*>(spec), plan.K, g, sums, bc, tw, div_partial);                    \
+                         reinterpret_cast<cpx<T>*>(spec), plan.K, g, sums, bc, tw, div_terms);                      \
     }                                                                                                               \
     break;
     SCA_ZGAMMA_LENGTHS(SCA_CASE)
@@ -1672,12 +1693,11 @@ int launch_zgamma(const FftPlan<T>& plan, T* spec, const GammaHost& gh, const do
   }
   if (nb == 0) throw std::runtime_error("fused Gamma convolution: unsupported z length");
   SCA_HIP(hipGetLastError());
-  return nb;
 }
-template int launch_zgamma<double>(const FftPlan<double>&, double*, const GammaHost&, const double*, const double*,
+template void launch_zgamma<double>(const FftPlan<double>&, double*, const GammaHost&, const double*, const double*,
+                                    const double*, const double*, double, double*, hipStream_t);
+template void launch_zgamma<float>(const FftPlan<float>&, float*, const GammaHost&, const double*, const double*,
                                    const double*, const double*, double, double*, hipStream_t);
-template int launch_zgamma<float>(const FftPlan<float>&, float*, const GammaHost&, const double*, const double*,
-                                  const double*, const double*, double, double*, hipStream_t);
 
 void launch_coords_uhat(double* spec, int64_t K, const GammaHost& gh, const double* d_xi_tab, double* fsum,
                         hipStream_t st) {

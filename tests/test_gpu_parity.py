@@ -393,6 +393,33 @@ def test_field_reads_beside_each_other_and_a_solve(product, precision):
             r.close()
 
 
+@pytest.mark.parametrize("derivative", [0, 1])
+@pytest.mark.parametrize("cells", [(8, 8, 8), (16, 8, 16), (8, 16, 32), (16, 16, 64), (8, 8, 128), (64, 64, 64)])
+def test_divergence_of_an_evaluation_equals_the_separate_launches(product, cells, derivative):
+    """The divergence decides convergence, and a context alone (its convolution in
+    one kernel with the z transforms) has to stop where a batch of it does (separate
+    launches, the kernels of sc_divergence_rms).  err_div of a solution's last
+    evaluation is bitwise the divergence of its P.  (A power-of-two cell count:
+    the two scale the root by N in different ways, which are then the same.)"""
+    assert np.log2(np.prod(cells)) % 1 == 0
+    mat, ori, size = polycrystal(cells, 5, seed=17, ori_seed=18)
+    r = Rve(product, cells, size, mat, ori, derivative=derivative, **EXAMPLE_NUMERICS)
+    try:
+        r.init()
+        r.forward(False, False, 0.5, 1.0, 10.0, tension_x(t=10.0, N=20))
+        sol = r.calculate_solution()
+        c, size = np.array(cells, dtype=np.int32), np.array(size, dtype=float)
+        scaled, rms = np.zeros(3), np.zeros(1)
+        product.check(product.sc_scaled_geom_size(ptr(c, IP), ptr(size), r.desc.grid_num.divergence_correction,
+                                                  ptr(scaled)), "scaled size")
+        xi1, _ = _xi(product, cells, size, derivative)
+        product.check(product.sc_divergence_rms(ptr(c, IP), ptr(size), ptr(scaled), ptr(xi1), ptr(r.field("P")),
+                                                ptr(rms)), "divergence")
+        assert sol.err_div == rms[0], (float(sol.err_div).hex(), float(rms[0]).hex())
+    finally:
+        r.close()
+
+
 @pytest.mark.parametrize("cells", [(27, 18, 24), (20, 14, 22)])
 def test_fft_plan_modes_give_the_same_bits(product, cells):
     """fft_plan_mode 1 (launch shapes timed per grid, like FFTW_MEASURE) and 0
