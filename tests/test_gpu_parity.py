@@ -219,7 +219,8 @@ def test_mp_update_edges(product, oracle, n, kind):
     output of the points with the oracle's counts within 1e-10 (the two solve
     the same equations to a stopping test that both meet or miss alike); a
     stopping decision at its threshold may move for 1 point in 100, so at most
-    two points here have other counts."""
+    two points here have other counts (none where there is one point), and they
+    agree within the stopping tests' spread.  No point is broken."""
     F, Fp0 = _random_batch(oracle, 1e-3, n=65)
     F, Fp0 = F[:n].copy(), Fp0[:n].copy()
 
@@ -233,12 +234,13 @@ def test_mp_update_edges(product, oracle, n, kind):
 
     a = _mp_batch(product, F, Fp0, 0.5, material=material)
     b = _mp_batch(oracle, F, Fp0, 0.5, material=material)
-    np.testing.assert_array_equal(a["broken"], b["broken"])
-    same = (a["iterations"] == b["iterations"]).all(axis=1) & (b["broken"] == 0)
-    assert (~same & (b["broken"] == 0)).sum() <= 2
-    if same.any():
-        for k in ["P", "Fp", "Lp", "S", "Fe", "xi", "gamma", "dPdF"]:
-            close(a[k][same], b[k][same], REL, k)
+    assert not a["broken"].any() and not b["broken"].any()
+    same = (a["iterations"] == b["iterations"]).all(axis=1)
+    assert (~same).sum() <= (0 if n == 1 else 2)
+    for k in ["P", "Fp", "Lp", "S", "Fe", "xi", "gamma", "dPdF"]:
+        close(a[k][same], b[k][same], REL, k)
+    for k in ("P", "Fp", "xi"):
+        close(a[k], b[k], 5e-5, k)
 
 
 def test_mp_update_substepping(product, oracle):
@@ -269,6 +271,70 @@ def test_mp_update_substepping(product, oracle):
     bound = {"P": 2 * 1.41e-3, "Fp": 2 * 1.40e-4, "xi": 2 * 6.66e-4}
     for k, v in spread.items():
         assert v <= bound[k], (k, v)
+
+
+# The grid solver updates its cells with kernels of its own (csrc/constitutive.hip);
+# sc_mp_update runs the callers' (csrc/points.hip).  The tests above reach the
+# latter, the ones below the former.
+EXPONENTS = {"example": (20.0, 2.25), "powers": (10.0, 2.0), "pow": (17.3, 1.7)}
+
+
+def _context_update(lib, F, ori, kind):
+    """One residual evaluation of a 16^3 context with an orientation for every
+    cell, at the given F, over 0.5 s from the undeformed state."""
+    m, _, _ = lib.defaults()
+    m.n_sl, m.a_sl = EXPONENTS[kind]
+    r = Rve(lib, (16, 16, 16), (1e-5,) * 3, np.arange(4096), ori, material=m, **EXAMPLE_NUMERICS)
+    try:
+        r.init()
+        r.forward(False, False, 0.5, 1.0, 10.0, tension_x(t=10.0, N=20))
+        r.form_residual(F)
+        out = {k: r.field(k).reshape(4096, -1) for k in ("P", "Fp", "Lp", "S", "Fe", "xi", "gamma")}
+        out["iterations"] = r.field("iterations").reshape(4096, 2).astype(int)
+        return out
+    finally:
+        r.close()
+
+
+@pytest.mark.parametrize("kind", list(EXPONENTS))
+def test_solver_update(product, oracle, kind):
+    """The inputs of test_mp_update (1e-3) and test_mp_update_other_exponents
+    through the solver's kernels, with those tests' requirements against the
+    oracle, and against the callers' update of the same points."""
+    F, Fp0 = _random_batch(oracle, 1e-3)
+    ori = uniform_orientations(4096, 11)
+    print(f"solver update: {kind}", flush=True)
+    a, b = _context_update(product, F, ori, kind), _context_update(oracle, F, ori, kind)
+
+    def material(m):
+        m.n_sl, m.a_sl = EXPONENTS[kind]
+
+    c = _mp_batch(product, F, Fp0, 0.5, material=material)
+    assert not c["broken"].any()
+    for other, what in ((b, "oracle"), (c, "callers' update")):
+        same = (a["iterations"] == other["iterations"]).all(axis=1)
+        assert same.mean() >= (1.0 if kind == "example" else 0.99), (what, same.mean())
+        for k in ["P", "Fp", "Lp", "S", "Fe", "xi", "gamma"]:
+            close(a[k][same], other[k][same], REL, f"{k} ({what})")
+        for k in ("P", "Fp", "xi"):
+            close(a[k], other[k], 5e-5, f"{k} ({what})")
+
+
+def test_solver_update_substepping(product, oracle):
+    """The inputs of test_mp_update_substepping through the solver's kernels: at
+    most 300 of 4096 points with other counts than the oracle, the rest within
+    1e-10.  Points with other counts are not compared here: on this path (Fp of
+    the start state as init leaves it) two CPU builds of the oracle differ from
+    each other on 215 points, by up to 1.5e-3 of P and 2.8e-4 of Fp."""
+    F, _ = _random_batch(oracle, 2e-2)
+    ori = uniform_orientations(4096, 11)
+    a, b = _context_update(product, F, ori, "example"), _context_update(oracle, F, ori, "example")
+    same = (a["iterations"] == b["iterations"]).all(axis=1)
+    print(f"solver substepping: {(~same).sum()} points with other counts", flush=True)
+    assert (~same).sum() <= 300, (~same).sum()
+    assert (b["iterations"][:, 1] > 12).any()  # substepping happened
+    for k in ["P", "Fp", "Lp", "xi", "gamma"]:
+        close(a[k][same], b[k][same], REL, k)
 
 
 # ---- outer solver ----------------------------------------------------------------------
@@ -312,16 +378,15 @@ def test_first_increment_homogeneous_forward(product, oracle):
     close(a.field("P"), b.field("P"), REL, "P")
 
 
-def test_state_read_between_forward_and_solve(product):
+@pytest.mark.parametrize("cells", [(16, 12, 8), (10, 6, 7), (80, 80, 80)])
+def test_state_read_between_forward_and_solve(product, cells):
     """f_materialpoint_forward (phase_mechanical.f90:992-1007) copies the
-    state into its start values.  A context above the captured-graph size
-    (80^3 > 64^3 cells) instead exchanges the current and start buffers of
-    Fp, S, xi and gamma and copies them back only for a reader that comes
-    before the next material-point update.  Read right after the forward
+    state into its start values.  A context instead exchanges the current and
+    start buffers of Fp, S, xi and gamma, and a read that comes before the next
+    material-point update takes the start ones.  Read right after the forward
     step, the fields are the previous increment's converged values, as after
     the copy, and the next increment is bitwise the one of a context whose
     fields were not read in between."""
-    cells = (80, 80, 80)
     mat, ori, size = polycrystal(cells, 4, seed=11, ori_seed=12)
     load = tension_x(t=10.0, N=20)
     names = ["Fp", "S", "xi", "gamma"]
@@ -489,6 +554,33 @@ def test_loadcase_16cubed_20grains(product, oracle):
     close(a.field("x_p"), b.field("x_p"), 1e-12, "x_p")
 
 
+@pytest.mark.parametrize("kind", ["powers", "pow"])
+def test_loadcase_other_exponents(product, oracle, kind):
+    """Five increments of tension (to 0.25 % strain, past the yield point) with
+    exponents that are not compiled in: the solver's run-time instantiations of
+    the update and of the tangent.  Same counts; a stopping decision that the
+    powers' rounding moves is worth up to 5e-5 of a point's P (see
+    test_mp_update_other_exponents) and n_sl = 20 times that in its tangent."""
+    cells = (8, 6, 12)
+    mat, ori, size = polycrystal(cells, 5, seed=23, ori_seed=24)
+    print(f"load case: exponents {kind}", flush=True)
+    rs = []
+    for lib in (product, oracle):
+        m, _, _ = lib.defaults()
+        m.n_sl, m.a_sl = EXPONENTS[kind]
+        r = Rve(lib, cells, size, mat, ori, material=m, **EXAMPLE_NUMERICS)
+        r.init()
+        rs.append((r, *r.loop_over_loadcase([tension_x(t=2.5, N=5)])))
+    (a, ia, ea), (b, ib, eb) = rs
+    np.testing.assert_array_equal(ia, ib)
+    np.testing.assert_array_equal(ea, eb)
+    assert b.field("gamma").max() > 1e-4  # plastic
+    for k in ("F", "P", "Fp", "xi"):
+        close(a.field(k), b.field(k), 5e-5, k)
+    close(a.scalars().C_volAvg, b.scalars().C_volAvg, 1e-3, "C_volAvg")
+    close(a.scalars().C_minMaxAvg, b.scalars().C_minMaxAvg, 1e-3, "C_minMaxAvg")
+
+
 def test_loadcase_update_gamma(product, oracle):
     """update_gamma = 1 (MechSolverBasic::calculate_solution,
     mech_solver_basic.cpp:127 -> MechBase::update_gamma, mech_base.cpp:156-211):
@@ -554,13 +646,12 @@ def test_mixed_precision_larger_pencils(product, oracle, cells):
 
 
 @pytest.mark.parametrize("precision", [0, 1])
-def test_residual_graph_replays_match_eager(product, precision):
-    """Small grids evaluate the residual as a captured HIP graph, replayed
-    many times per increment between the solver's own eager launches and
-    host synchronisations, and captured again when its arguments change
-    (time step, compliance, precision phase).  Kernel timing forces the
-    eager launches: both runs must agree bitwise in every increment."""
-    print(f"graph vs eager: precision {precision}", flush=True)
+def test_profiling_changes_no_bits(product, precision):
+    """Kernel timing brackets the launches of an evaluation with events and adds
+    the sums of the iteration counts, which also make the scalars that the
+    evaluation's last kernels send to the host more: counts, <P>, err_div and
+    fields are bitwise those without it in every increment."""
+    print(f"profiled: precision {precision}", flush=True)
     cells = (16, 12, 8)
     mat, ori, size = polycrystal(cells, 9, seed=21, ori_seed=22)
     runs = []
@@ -568,7 +659,7 @@ def test_residual_graph_replays_match_eager(product, precision):
         r = Rve(product, cells, size, mat, ori, precision=precision, **EXAMPLE_NUMERICS)
         r.init()
         r.profile(timed)
-        trace = [(d["iterations"], d["evaluations"], r.scalars().P_av[:])
+        trace = [(d["iterations"], d["evaluations"], r.scalars().P_av[:], r.scalars().err_div)
                  for d in r.increments([tension_x(t=4.0, N=8)])]
         runs.append((trace, r.field("F"), r.field("P"), r.field("xi")))
     (ta, Fa, Pa, xa), (tb, Fb, Pb, xb) = runs
