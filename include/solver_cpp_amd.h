@@ -268,9 +268,12 @@ int sc_rve_reset_stats(sc_rve* rve);
 enum {
   SC_KT_RESPONSE = 0,  /* material-point update (stress integration)       */
   SC_KT_TANGENT = 1,   /* consistent tangent dPdF                           */
-  SC_KT_FFT_FWD = 2,   /* forward 3D FFT of the 9 stress planes             */
-  SC_KT_FFT_BWD = 3,   /* inverse 3D FFT of the 9 residual planes           */
-  SC_KT_GAMMA = 4,     /* fused Gamma convolution + divergence              */
+  SC_KT_FFT_FWD = 2,   /* forward 3D FFT of the 9 stress planes (x and y passes with the P
+                          sums where one kernel holds the z pass and the convolution) */
+  SC_KT_FFT_BWD = 3,   /* inverse 3D FFT of the 9 residual planes (there with the divergence
+                          sum and the response scalars' way to the host) */
+  SC_KT_GAMMA = 4,     /* Gamma convolution + divergence (there with the forward z pass
+                          and the aim, and without the divergence sum) */
   SC_KT_REDUCE = 5,    /* reductions and N-GMRES vector updates             */
   SC_KT_OTHER = 6,
   SC_KT_COUNT = 7
@@ -425,10 +428,10 @@ int sc_mp_update(int64_t n, double dt, const sc_material* m, const sc_phase_nume
  * (i,j) of every point), a slip field 12 planes of n doubles, dPdF 81 planes
  * (plane i+3j+9k+27l), iterations 2 planes of n ints (Newton, state
  * iterations) and broken n ints.  The substep scratch lives in one fixed
- * device array of the library sized for SC_MP_NOALLOC_MAX_POINTS points (about 16 MB, held
- * on each GPU the library runs on until the process ends); larger n is
- * refused with an error.  The call allocates nothing.  Calls that overlap on
- * one GPU share that array and race: serialise them. */
+ * device array of the library sized for SC_MP_NOALLOC_MAX_POINTS points (about
+ * 16 MB, held on each GPU the library runs on until the process ends); larger
+ * n is refused with an error.  The call allocates nothing.  Calls that overlap
+ * on one GPU share that array and race: serialise them. */
 #define SC_MP_NOALLOC_MAX_POINTS 32768
 typedef struct sc_mp_device_planes {
   const double *F, *F0, *Fp0, *Lp0, *S0, *xi0, *gamma0;  /* inputs, as in sc_mp_update */

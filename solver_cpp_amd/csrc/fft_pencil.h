@@ -218,7 +218,8 @@ __device__ __forceinline__ const cpx<T>* stage_tw(cpx<T>* lds_tw, const cpx<T>* 
 // pencils, since neighbouring blocks of a y pass share the cache lines at
 // their ends (rows of N/2 + 1 entries start anywhere in a line): y pass of
 // 9 x 128^3, forward / inverse 68 / 68 -> 62 / 48 us, in single precision
-// 39 / 40 -> 28 / 28; z pass 46 -> 45.
+// 39 / 40 -> 28 / 27; inverse z pass 46 -> 48 with the end of the evaluation
+// (4160 divergence partials) in a block of it.
 template <typename T, int N, int SIGN, typename Side>
 __global__ void __launch_bounds__(MAX_PENCIL_BLOCK) strided_kernel(cpx<T>* data, int ni, int64_t npen, int d1,
                                                                    int64_t s1, int64_t s2, int64_t es,

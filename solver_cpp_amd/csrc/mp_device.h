@@ -311,7 +311,8 @@ __device__ __forceinline__ void st(double* plane, Lane l, double v) {
 // formed here (two scalar adds a plane).  From the plain N the compiler forms
 // the pointers of every access once at the kernel's entry, keeps them in
 // vector lanes (it has no scalar registers for 150 of them) and reads each
-// back at its use: 630 instructions of the 12000 that a wave executes.
+// back at its use: 838 lane moves among the update kernel's 7824 instructions,
+// 304 among 7478 with the stride formed where it is used.
 __device__ __forceinline__ int64_t stride_here(int64_t N) {
   asm volatile("" : "+s"(N));
   return N;

@@ -9,8 +9,9 @@
 // hipGetSymbolAddress and only that address is ever handed to kernels.
 //
 // Every call on a GPU shares that GPU's array and leaves its contents behind.
-// The substep planes of a point are written before they are read.  Two calls that overlap on one GPU race on the array: callers
-// serialise them (one stream, or one call at a time).
+// The substep planes of a point are written before they are read.  Two calls
+// that overlap on one GPU race on the array: callers serialise them (one stream,
+// or one call at a time).
 #include <mutex>
 
 #include "common.h"

@@ -9,7 +9,7 @@
 // spectral stages are in single), and a load case, its checkpoints and its
 // restarts keep their bits.
 //
-// Bound: one lane per point and one wave per SIMD (456 of 512 registers), so a
+// Bound: one lane per point and one wave per SIMD (466 of 512 registers), so a
 // call of up to 65536 points is one wave's chain of dependent operations, and
 // part of that is fetching its instructions: the code is kept short (one copy
 // of the rate evaluation, no second pass).  60 points: 45 -> 32 us a call;
@@ -332,7 +332,7 @@ __device__ __forceinline__ bool newton_step(const double* Fe, const double* A, c
   // multiplies.  J acts on the five numbers w(x) only, and those are known
   // without cancellation: y_i / kappa_i.  The symmetric traceless matrix that
   // has the difference for its five numbers (G taken as the identity) removes
-  // it to within |G - I|.  Without it 871 instead of 162 of the 4096 points of
+  // it to within |G - I|.  Without it 864 instead of 162 of the 4096 points of
   // 2 % strain steps take other iteration counts than with a pivoted 9x9 LU.
   double e[NW];
   newton_w(G, b, e);
@@ -769,7 +769,7 @@ __device__ __forceinline__ void mp_point(ConstArgs* ap, const int64_t c, MpLds& 
   if (!converged && p->ill) atomicOr(p->ill, 1);
 }
 
-// the arguments of a kernel whose only parameter they are, and a table's entry
+// the arguments of a kernel whose only parameter they are
 __device__ __forceinline__ ConstArgs* kernel_args() {
 #if defined(__HIP_DEVICE_COMPILE__)
   return (ConstArgs*)__builtin_amdgcn_kernarg_segment_ptr();
@@ -777,7 +777,6 @@ __device__ __forceinline__ ConstArgs* kernel_args() {
   return nullptr;
 #endif
 }
-__device__ __forceinline__ ConstArgs* table_args(const KernelArgs* p) { return (ConstArgs*)p; }
 
 template <int NE4, int AE4>
 __global__ void __launch_bounds__(64) mp_points_kernel(KernelArgs) {
@@ -799,7 +798,7 @@ __global__ void __launch_bounds__(64) mp_points_kernel(KernelArgs) {
 // the Newton system (newton_step, H in the place of G)
 //   (diag + w(H U_j)) y = w(X),   V = sum_j U_j y_j,   dS = C : (X - H V),
 // and dFp^-1/dF = -invFp0 V.  The 5x5 matrix is inverted once (partial
-// pivoting) for the nine columns: 5730 instead of 8400 instructions, no 9x9
+// pivoting) for the nine columns: 5730 instead of 10426 instructions, no 9x9
 // elimination in one dependent chain (26 -> 13 us for 4097 points).
 // ---------------------------------------------------------------------------
 

@@ -690,8 +690,10 @@ GammaHost Rve::gamma_host(bool do_gamma) const {
 // Launched, not replayed from a captured graph, on grids of every size: a
 // graph needs F copied in and r out of its own buffers, and the forward step
 // could not exchange the state's.  Re-solved increments, captured / launched:
-// 16^3 1818 / 1699 us, 64^3 5.46 / 5.18 ms, 27 x 40 x 22 mixed (fourteen
-// launches an evaluation) 2.69 / 2.59 ms.
+// 16^3 1818 / 1699 us, 64^3 5.46 / 5.18 ms; with fourteen launches an
+// evaluation 27 x 40 x 22 mixed 2.69 / 2.59 ms, 20^3 2.54 / 2.35 ms, 50^3
+// 4.78 / 4.33 ms, 6 x 5 x 4 2.32 / 2.07 ms, 16^3 with derivative 2 (81
+// evaluations) 14.8 / 14.0 ms.
 // clear: the pivoting list and the ill flag are not clear yet.
 void Rve::launch_residual(const double* Fdev, void* rdev, bool clear) {
   state_stale = false;  // the update writes the current set of every cell

@@ -454,9 +454,10 @@ __global__ void __launch_bounds__(256) gamma_div_batch_kernel(const GammaBatchEn
 // and z passes (DivSide, FinishSide): the divergence decides convergence, and a
 // context alone stops where a batch of it does.
 // Bound: HBM (two passes over the spectrum instead of four) and, at 128^3 in
-// single precision, the one block a CU has registers for.  At 128^3: 92 us
-// (3.3 TB/s) after 54 + 52 apart, without the XCD order 112; at 64^3 17 after
-// 10 + 9; at 16^3 8 after 5 + 5 and the two launches between them.
+// single precision, the one block a CU has registers for.  At 128^3: 77 us
+// (4.1 TB/s; single 74) after 54 + 52 apart (with the divergence summed inside
+// the blocks 92, and 112 without the XCD order); at 64^3 18 after 10 + 9; at
+// 16^3 9 after 5 + 5 and the two launches between them.
 __device__ __forceinline__ double rnd_mul(double a, double b) {
 #pragma clang fp contract(off)
   return a * b;
